@@ -67,11 +67,11 @@ int round_up(int v, int m) { return (v + m - 1) / m * m; }
 // 12 N * blocks bytes; past kSymBandCap they are kept one column band at a
 // time).
 constexpr int kSymSlotsTarget = 512;
-// Below N = 512 * kSmallSymBlocks the default symmetric plan takes smaller
-// blocks (256, then 128 bodies below N = 256 * kSmallSymBlocks), keeping
-// about this many: at N = 8192, 16384 and 32768 the autotuner's choices
-// (blocks of 128, 256, 512) all have 64.
-constexpr int kSmallSymBlocks = 64;
+// Below this N the default symmetric plan takes blocks of 128 bodies, one wave
+// each with 2 bodies per lane: at N = 4096 it takes 16.2 us against 18.0 with
+// blocks of 512, whose 36 block pairs leave most CUs idle; at N = 6000 26.1
+// against 22.5.
+constexpr size_t kSmallSymN = 5120;
 
 // Default decomposition: enough blocks for ~48 waves per SIMD (the dispatcher
 // balances them across the 256 CUs), j slices of at least 1024 bodies in
@@ -94,16 +94,14 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
     }
     if (variant == VAR_SYMMETRIC) {
         // blocks of B = 64 * ipl * waves (default 8 bodies per lane and the
-        // fewest waves that keep at most kSymSlotsTarget blocks: B = 512 from
-        // N = 32K up to 256K, 2048 at N = 1M; smaller systems below); the block
-        // slots are always summed with TwoSum
+        // fewest waves that keep at most kSymSlotsTarget blocks: B = 512 up to
+        // N = 256K, 2048 at N = 1M); the block slots are always summed with
+        // TwoSum
         p.ipl = (opt && opt->i_per_lane > 0) ? opt->i_per_lane : 8;
         const bool shape_given = opt && (opt->i_per_lane > 0 || opt->jslice > 0);
-        if (!shape_given && N < (size_t)kSmallSymBlocks * 512) {
-            // small systems: keep about kSmallSymBlocks blocks (the shapes the
-            // autotuner picks there), so the pair tasks fill the chip
-            p.ipl = N < (size_t)kSmallSymBlocks * 256 ? 2 : 4;
-            p.jslice = 64 * p.ipl;
+        if (!shape_given && N < kSmallSymN) {
+            p.ipl = 2;
+            p.jslice = 128;
         } else if (opt && opt->jslice > 0) {
             p.jslice = opt->jslice;
         } else if (p.ipl == 2) {

@@ -41,7 +41,7 @@ __global__ __launch_bounds__(kWave) void k_force_batch(const ForceTask* __restri
         if (t >= ntasks) return;
         const ForceTask task = tasks[t];
         if (task.kind == TASK_PAIR) {
-            sym_pair<kPairA, 1, false, true>(task.pm, task.n, task.eps2, SlotMap::whole(task.part, task.nb, task.npad),
+            sym_pair<kPairA, 1, false, REGS_APART>(task.pm, task.n, task.eps2, SlotMap::whole(task.part, task.nb, task.npad),
                                              task.a, task.b, jacc);
             continue;
         }

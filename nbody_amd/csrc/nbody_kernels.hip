@@ -375,10 +375,9 @@ __global__ __launch_bounds__(kBlock) void k_force_dpp(ForceParams p)
 //
 // The symmetric plan (see nbody_sym.h): workgroup t < nb(nb-1)/2 computes
 // block pair (P, Q), P < Q; the remaining nb*A workgroups are the diagonal
-// pieces, one-sided, last in the grid: their small size lets them fill the
-// end of the launch evenly (one task per diagonal block, each pair once,
-// halves their work but measured 2.5 % slower at N = 98304 for its coarser
-// end; the batched kernel, whose queue mixes many systems, uses it).
+// pieces, one-sided, last in the grid. With 8 bodies per lane and blocks of
+// 512, k_force_sym_deal below divides the same block triangle among
+// workgroups of four waves.
 // One launch covers the column band q0 <= Q < q1 of the block triangle: the
 // pairs (P, Q), P < Q, then A pieces of each band block's diagonal.
 struct SymParams {
@@ -388,6 +387,9 @@ struct SymParams {
     int npairs;    // pairs in the band: Q(Q-1)/2 summed over its columns
     float eps2;
     SlotMap slots; // where the band's partials go
+    int split;       // k_force_sym_deal: tasks per block pair (1, 2 or 4), each with its own i-side slot
+    int diag_tasks;  // and diagonal tasks, first in the grid (one per block, two with split 4)
+    size_t more;     // floats from the slot rows of a pair's task h to those of task h + 1
 };
 
 template <int A, int W, bool NEWTON>
@@ -395,13 +397,6 @@ __global__ __launch_bounds__(64 * W) void k_force_sym(SymParams p)
 {
     constexpr int B = 64 * A * W;
     __shared__ float jacc[3][B];
-    // Registers decide how many waves share a SIMD; LDS only how many
-    // workgroups share a CU, which the dispatcher may spread unevenly over its
-    // four SIMDs. With 8 bodies per lane on one wave the kernel needs 71
-    // VGPRs (7 waves per SIMD; 6.5 by LDS) but runs fastest at exactly 6 per
-    // SIMD (121 TFLOP/s credited at N = 98304 against 115), so it claims v79:
-    // 80 VGPRs, 6 waves on every SIMD.
-    if constexpr (A == 8 && W == 1) asm volatile("" ::: "v79");
     const int t = blockIdx.x;
     if (t < p.npairs) {
         int P, Q;
@@ -413,59 +408,210 @@ __global__ __launch_bounds__(64 * W) void k_force_sym(SymParams p)
     }
 }
 
-// The band's slots of each body summed in slot order with TwoSum. One lane
-// per (body, component) (blockIdx.y = component); slots are fetched eight at
-// a time so the loads overlap, then folded strictly in slot order. With one
-// band the sum is rounded once into the force. With several, the running
-// (sum, error) pair of each body carries from band to band in `state`
-// ([2][3][n]; the first band starts it, a body of a block past the band adds
-// nothing yet) and the last band rounds it into the force; each body's slots
-// are then folded in band order, the same fixed order on every run. With
-// force64 the last band writes the pair's value in FP64 instead (a share of
-// the columns, whose partial force is summed with the other shares').
-__global__ __launch_bounds__(kBlock) void k_reduce_band(SlotMap m, int n, int B, int q0, int q1, bool first,
-                                                        bool last, float* __restrict__ state,
-                                                        float* __restrict__ force, double* __restrict__ force64)
+constexpr int kDealWaves = 4;
+
+// The symmetric plan with 8 bodies per lane and blocks of 512: a workgroup of
+// 4 waves, one per SIMD, each holding the same 512 bodies of block P, deals
+// the 64-body tiles of block Q among them. A tile's reactions go from the
+// lanes of the one wave that meets it straight to their slot, and only the i
+// sides of the four waves meet, in LDS at the end: no barrier until then.
+//
+// Bound by the VALU issue of the pair chain (nbody_sym.h): 52 clocks of a SIMD
+// per 64 pairs with 4 or more waves on it, 59 with 2, 76 with 1 (stamps in the
+// kernel). What is left to lose is the spread of the work, which this split is
+// about: one-wave workgroups of whole block pairs gave the SIMDs of a small
+// system 2 or 3 tasks each; four-wave ones load a CU's SIMDs alike, and with
+// `split` tasks per pair (sym_split) the CUs too. The diagonal tasks come
+// first in the grid: each costs about a tenth more than a pair task (tiles
+// that meet one or two sub-blocks rotate as often as full ones), and the
+// oldest wave of a SIMD issues first, so last they would run on alone
+// (N = 16384: the pairs end at 51 us, such a diagonal at 55).
+// Kernel time, N = 98304 ball: 1.521 ms, 0.807 of the FP32 peak (1.58 ms with
+// one wave per block pair and the diagonal in one-sided pieces at the end);
+// unequal masses 1.70 ms (1.78). Whole evaluations, before and after:
+// N = 49999 480 and 422 us, 32768 212 and 188, 24576 141 and 115, 16384 68.5
+// and 59, 12000 53 and 43.
+template <bool NEWTON>
+__global__ __launch_bounds__(64 * kDealWaves, 6) void k_force_sym_deal(SymParams p)
+{
+    constexpr int W = kDealWaves, B = 512, T = B / 64;
+    __shared__ float part[W][3][B];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int halves = p.split == 4 ? 2 : 1;  // a tile's 64 steps on one wave, or 32 on each of two
+    const int half = halves == 2 ? wave & 1 : 0;
+    const bool diag = (int)blockIdx.x < p.diag_tasks;
+    int P, Q, h;  // task h of the block pair, or h of the diagonal block
+    if (diag) {
+        P = Q = p.q0 + blockIdx.x / halves;
+        h = blockIdx.x % halves;
+    } else {
+        const int t = blockIdx.x - p.diag_tasks;
+        h = t % p.split;
+        upper_pair(p.q0 * (p.q0 - 1) / 2 + t / p.split, P, Q);
+    }
+    const float m0 = p.pm[P * B].w;
+    Lanes<8> me, acc;
+    float mi[8];
+    bool same = true;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int i = P * B + u * 64 + lane;
+        const float4 q = i < p.n ? p.pm[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+        me.x[u] = q.x;
+        me.y[u] = q.y;
+        me.z[u] = q.z;
+        mi[u] = q.w;
+        same &= (i < p.n) & (q.w == m0);
+    }
+    zero<8>(acc);
+    float scale = 1.0f;
+    if (diag) {
+        const bool eq = !NEWTON && __builtin_amdgcn_ballot_w64(!same) == 0;
+        sym_deal_diag<NEWTON>(p.pm, p.n, p.eps2, P, wave, h, halves, eq, me, mi, acc);
+        if (eq) scale = m0;
+    } else {
+        // tiles t0, t0 + W, ... < t1 of block Q
+        const int t0 = h * (T / p.split) + (halves == 2 ? wave >> 1 : wave), t1 = p.split == 1 ? T : t0 + 1;
+        for (int tile = t0; tile < t1; tile += W) {
+            const int j = Q * B + tile * 64 + lane;
+            same &= (j < p.n) & (p.pm[min(j, p.n - 1)].w == m0);
+        }
+        const bool eq = __builtin_amdgcn_ballot_w64(!same) == 0;
+        if (eq) scale = m0;
+        float* jdst = p.slots.j_side(P, Q, B);
+        const size_t plane = p.slots.bplane;
+        const int out = t0 * 64;
+        float r[3];
+        if (eq)
+            sym_deal_tiles<NEWTON, true>(p.pm, p.n, p.eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst, plane,
+                                         m0, r);
+        else
+            sym_deal_tiles<NEWTON, false>(p.pm, p.n, p.eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst, plane,
+                                          1.0f, r);
+        if (halves == 2) {
+            // the first half's reactions are half a turn from home; the second wave adds both in order
+            if (half == 0) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) part[wave][c][lane ^ 32] = r[c];
+            }
+            __syncthreads();
+            if (half == 1 && Q * B + out < p.n) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) jdst[c * plane + out + lane] = part[wave - 1][c][lane] + r[c];
+            }
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        part[wave][0][u * 64 + lane] = acc.x[u] * scale;
+        part[wave][1][u * 64 + lane] = acc.y[u] * scale;
+        part[wave][2][u * 64 + lane] = acc.z[u] * scale;
+    }
+    __syncthreads();
+    float* __restrict__ idst = (diag ? p.slots.j_side(P, P, B) : p.slots.i_side(P, Q, B)) + h * p.more;
+    const size_t iplane = diag ? p.slots.bplane : p.slots.i_plane(P);
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int k = 0; k < B; k += 64 * W) {
+            const int o = k + threadIdx.x;
+            float sum = part[0][c][o];
+#pragma unroll
+            for (int w = 1; w < W; ++w) sum += part[w][c][o];
+            idst[c * iplane + o] = sum;
+        }
+}
+
+constexpr int kReduceGroups = 4;
+
+// The band's slots of each body summed with TwoSum. A workgroup of 12 waves
+// takes 64 bodies: wave (g, c) adds the g-th quarter of component c's slot
+// rows in slot order, eight loads in flight (one contiguous 256-byte run
+// each), and group 0 then folds the four (sum, error) pairs in order. Bound
+// by HBM on a large system (N = 98304, 226 MB of slots: 33 us, 6.8 TB/s) and
+// by the chain of loads on a small one, hence the quarters: N = 16384 with
+// two tasks per block pair takes 4.8 us, 6.5 us with one wave over all rows.
+// With one band the sum is rounded once into the force. With several, the
+// running (sum, error) pair of each body carries from band to band in
+// `state` ([2][3][n]; the first band starts it, a body of a block past the
+// band adds nothing yet) and the last band rounds it into the force; each
+// body's slots are then folded in band order, the same fixed order on every
+// run. With force64 the last band writes the pair's value in FP64 instead (a
+// share of the columns, whose partial force is summed with the other
+// shares').
+__global__ __launch_bounds__(64 * 3 * kReduceGroups) void k_reduce_band(SlotMap m, int n, int B, int q0, int q1,
+                                                                        bool first, bool last,
+                                                                        float* __restrict__ state,
+                                                                        float* __restrict__ force,
+                                                                        double* __restrict__ force64, int split)
 {
     constexpr int G = 8;
-    const int b = blockIdx.x * kBlock + threadIdx.x;
-    if (b >= n) return;
-    const int c = blockIdx.y;
-    const int blk = b / B;
+    __shared__ float sums[kReduceGroups][3][64], errs[kReduceGroups][3][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int c = wave % 3, group = wave / 3;
+    const int b0 = blockIdx.x * 64, blk = b0 / B, b = b0 + lane;  // blocks hold whole groups of 64 bodies
     if (!first && !last && blk >= q1) return;
     const float* src = nullptr;
-    int slots = 0;
+    int rows = 0, base = 0;  // slot rows, and how many of them are the first run
     size_t row = 0;
     if (blk < q0) {
-        src = m.a + c * m.aplane + b;
-        slots = q1 - q0;
+        src = m.a + c * m.aplane + b0;
+        rows = base = q1 - q0;
         row = m.arow;
     } else if (blk < q1) {
-        src = m.b + c * m.bplane + (b - (size_t)q0 * B);
-        slots = q1;
+        src = m.b + c * m.bplane + (b0 - (size_t)q0 * B);
+        rows = base = q1;
         row = m.brow;
     }
+    // Split block pairs (one band over q1 blocks): task h > 0 keeps its i
+    // sides in rows h q1 + blk + 1 .. (h + 1) q1 - 1, and with four tasks the
+    // diagonal's second half is in row q1 + blk.
+    const int extra = q1 - blk - 1, second = split == 4 ? extra + 1 : extra;
+    if (split > 1) rows += second + (split - 2) * extra;
+    auto row_of = [&](int k) {
+        if (k < base) return k;
+        k -= base;
+        if (k < second) return 2 * q1 - second + k;
+        k -= second;
+        return k < extra ? 3 * q1 - extra + k : 4 * q1 - 2 * extra + k;
+    };
     float s = 0.f, e = 0.f;
-    if (!first) {
-        s = state[(size_t)c * n + b];
-        e = state[(size_t)(3 + c) * n + b];
-    }
-    int k = 0;
-    for (; k + G <= slots; k += G) {
-        float v[G];
+    if (b < n) {
+        if (!first && group == 0) {
+            s = state[(size_t)c * n + b];
+            e = state[(size_t)(3 + c) * n + b];
+        }
+        int k = rows * group / kReduceGroups;
+        const int end = rows * (group + 1) / kReduceGroups;
+        for (; k + G <= end; k += G) {
+            float v[G];
 #pragma unroll
-        for (int g = 0; g < G; ++g) v[g] = src[(size_t)(k + g) * row];
+            for (int g = 0; g < G; ++g) v[g] = src[row_of(k + g) * row + lane];
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
+            for (int g = 0; g < G; ++g) {
+                float err;
+                s = two_sum(s, v[g], err);
+                e += err;
+            }
+        }
+        for (; k < end; ++k) {
             float err;
-            s = two_sum(s, v[g], err);
+            s = two_sum(s, src[row_of(k) * row + lane], err);
             e += err;
         }
     }
-    for (; k < slots; ++k) {
+    sums[group][c][lane] = s;
+    errs[group][c][lane] = e;
+    __syncthreads();
+    if (group != 0 || b >= n) return;
+#pragma unroll
+    for (int g = 1; g < kReduceGroups; ++g) {
         float err;
-        s = two_sum(s, src[(size_t)k * row], err);
-        e += err;
+        s = two_sum(s, sums[g][c][lane], err);
+        e += err + errs[g][c][lane];
     }
     if (last && force64) {
         force64[4 * (size_t)b + c] = (double)s + (double)e;
@@ -791,6 +937,12 @@ const void* sym_kernel()
     return reinterpret_cast<const void*>(&k_force_sym<A, W, NEWTON>);
 }
 
+const void* deal_kernel(bool newton)
+{
+    return newton ? reinterpret_cast<const void*>(&k_force_sym_deal<true>)
+                  : reinterpret_cast<const void*>(&k_force_sym_deal<false>);
+}
+
 template <int A, int W>
 hipError_t go_sym(const ForcePlan& plan, const SymParams& sp, int band_blocks, hipStream_t s)
 {
@@ -802,6 +954,16 @@ hipError_t go_sym(const ForcePlan& plan, const SymParams& sp, int band_blocks, h
     return hipGetLastError();
 }
 
+hipError_t go_sym_deal(const ForcePlan& plan, const SymParams& sp, hipStream_t s)
+{
+    const int tasks = sp.npairs * sp.split + sp.diag_tasks, threads = 64 * kDealWaves;
+    const void* k = deal_kernel(plan.newton);
+    const size_t dyn = plan.occ > 0 ? lds_for_occupancy(k, threads, plan.occ) : 0;
+    if (plan.newton) k_force_sym_deal<true><<<tasks, threads, dyn, s>>>(sp);
+    else k_force_sym_deal<false><<<tasks, threads, dyn, s>>>(sp);
+    return hipGetLastError();
+}
+
 hipError_t go_sym_shape(const ForcePlan& plan, const SymParams& sp, int band_blocks, hipStream_t s)
 {
     const int w = plan.jslice / (64 * plan.ipl);
@@ -810,7 +972,7 @@ hipError_t go_sym_shape(const ForcePlan& plan, const SymParams& sp, int band_blo
         return w == 1   ? go_sym<4, 1>(plan, sp, band_blocks, s)
                : w == 2 ? go_sym<4, 2>(plan, sp, band_blocks, s)
                         : go_sym<4, 4>(plan, sp, band_blocks, s);
-    return w == 1   ? go_sym<8, 1>(plan, sp, band_blocks, s)
+    return w == 1   ? go_sym_deal(plan, sp, s)
            : w == 2 ? go_sym<8, 2>(plan, sp, band_blocks, s)
                     : go_sym<8, 4>(plan, sp, band_blocks, s);
 }
@@ -818,9 +980,47 @@ hipError_t go_sym_shape(const ForcePlan& plan, const SymParams& sp, int band_blo
 // Floats of slot regions band [q0, q1) keeps: region A then region B.
 size_t band_floats(int q0, int q1, int B) { return (size_t)3 * (q1 - q0) * B * ((size_t)q0 + q1); }
 
-// Where band [q0, q1) keeps its slots, from `base`: region A, then region B.
+// Diagonal tasks per block: one, or two where the pairs are in four.
+int deal_diag_tasks(int split) { return split == 4 ? 2 : 1; }
+
+// Tasks per block pair of a plan's k_force_sym_deal launch, 1, 2 or 4; only in
+// a single band over every column. More tasks put more waves on a SIMD and
+// end the launch more evenly: the fullest CU gets ceil(tasks / 256) of them,
+// each 1 / split of a pair, and a pair takes 22 us of a CU whose SIMDs hold 4
+// waves or more (1.46, 1.13 and 1.08 times that with 1, 2 and 3). But each
+// further task keeps its i sides in more slot rows, which the slot sum reads
+// back (12 bytes per body and row at about 4 TB/s). Measured, whole
+// evaluations with 1, 2, 4 tasks: N = 8192 40, 27, 24 us; 12000 51, 47, 43;
+// 16384, where 2 gives every CU exactly four tasks, 70, 59, 61; 20000 94, 91,
+// 86; 32768 199, 188, 195; 49999 424, 427, 442.
+int sym_split(const ForcePlan& plan, size_t nbands)
+{
+    const bool whole = plan.col0 == 0 && (plan.col1 <= 0 || plan.col1 == plan.nslices);
+    if (plan.acc64 || plan.ipl != 8 || plan.jslice != 512 || !whole || nbands != 1) return 1;
+    const size_t cap = plan.band_cap ? plan.band_cap : kSymBandCap;
+    const double nb = plan.nslices;
+    constexpr double few_waves[] = {1.0, 1.46, 1.13, 1.08};
+    int best = 1;
+    double least = 0.0;
+    for (int split : {1, 2, 4}) {
+        if (split > 1 && split * band_floats(0, plan.nslices, 512) * sizeof(float) > cap) break;
+        const double tasks = 0.5 * nb * (nb - 1.0) * split + nb * deal_diag_tasks(split);
+        const double rows = nb + 0.5 * (nb - 1.0) * (split - 1);
+        const double fullest = std::ceil(tasks / 256.0);
+        const double us = fullest * 22.0 / split * (fullest < 4.0 ? few_waves[(int)fullest] : 1.0) +
+                          rows * nb * 512.0 * 12.0 / 4.0e6;
+        if (split == 1 || us < least) {
+            least = us;
+            best = split;
+        }
+    }
+    return best;
+}
+
+// Where band [q0, q1) keeps its slots, from `base`: region A, then region B
+// (with split block pairs one band, `split` times the rows).
 template <class T>
-SlotMapT<T> band_slots(T* base, int q0, int q1, int B)
+SlotMapT<T> band_slots(T* base, int q0, int q1, int B, int split = 1)
 {
     const int w = q1 - q0;
     SlotMapT<T> m;
@@ -829,7 +1029,7 @@ SlotMapT<T> band_slots(T* base, int q0, int q1, int B)
     m.aplane = (size_t)w * q0 * B;
     m.b = base + 3 * m.aplane;
     m.brow = w * B;
-    m.bplane = (size_t)q1 * w * B;
+    m.bplane = (size_t)split * q1 * w * B;
     m.q0 = q0;
     return m;
 }
@@ -858,8 +1058,8 @@ int symmetric_natural_occupancy(const ForcePlan& plan)
     if (plan.ipl == 4)
         return w == 1 ? natural_occupancy<4, 1>(plan.newton) : w == 2 ? natural_occupancy<4, 2>(plan.newton)
                                                                       : natural_occupancy<4, 4>(plan.newton);
-    return w == 1 ? natural_occupancy<8, 1>(plan.newton) : w == 2 ? natural_occupancy<8, 2>(plan.newton)
-                                                                  : natural_occupancy<8, 4>(plan.newton);
+    if (w == 1) return blocks_per_cu(deal_kernel(plan.newton), 64 * kDealWaves, 0) * kDealWaves / 4;
+    return w == 2 ? natural_occupancy<8, 2>(plan.newton) : natural_occupancy<8, 4>(plan.newton);
 }
 
 void symmetric_share_columns(int nb, int k, int G, int* c0, int* c1)
@@ -903,6 +1103,7 @@ size_t plan_scratch_bytes(const ForcePlan& plan, int ni)
                                            elem, plan.col0, plan.col1 > 0 ? plan.col1 : plan.nslices);
         size_t most = 0;
         for (const auto& b : bands) most = std::max(most, band_floats(b.first, b.second, plan.jslice));
+        most *= sym_split(plan, bands.size());
         // the running sums carried between bands: (sum, error) float pairs or one double per component
         const size_t carry = bands.size() > 1 ? (size_t)6 * ni * sizeof(float) : 0;
         return most * elem + carry;
@@ -945,7 +1146,8 @@ hipError_t launch_force(const ForcePlan& plan, const ForceParams& p, hipStream_t
         for (const auto& b : bands) most = std::max(most, band_floats(b.first, b.second, B));
         // a share with no columns still writes its (zero) partial forces
         if (bands.empty()) bands.emplace_back(c0, c0);
-        const dim3 gr((p.n + kBlock - 1) / kBlock, 3);
+        const dim3 gr((p.n + kBlock - 1) / kBlock, 3);       // k_reduce_band64
+        const int groups = (p.n + 63) / 64;                  // k_reduce_band
         e = hipSuccess;
         for (size_t k = 0; k < bands.size(); ++k) {
             const int q0 = bands[k].first, q1 = bands[k].second, w = q1 - q0;
@@ -983,13 +1185,16 @@ hipError_t launch_force(const ForcePlan& plan, const ForceParams& p, hipStream_t
                 sp.npairs = npairs;
                 sp.eps2 = p.eps2;
                 float* base = reinterpret_cast<float*>(p.hi);
-                sp.slots = band_slots(base, q0, q1, B);
+                sp.split = sym_split(plan, bands.size());
+                sp.slots = band_slots(base, q0, q1, B, sp.split);
+                sp.diag_tasks = w * deal_diag_tasks(sp.split);
+                sp.more = (size_t)nb * sp.slots.brow;
                 if (npairs + w > 0) e = go_sym_shape(plan, sp, w, stream);
                 if (e == hipSuccess && after && last) e = hipEventRecord(after, stream);
                 if (e != hipSuccess) return e;
                 float* state = bands.size() > 1 ? base + most : nullptr;
-                k_reduce_band<<<gr, kBlock, 0, stream>>>(sp.slots, p.n, B, q0, q1, first, last, state, p.force,
-                                                         p.force64);
+                k_reduce_band<<<groups, 64 * 3 * kReduceGroups, 0, stream>>>(sp.slots, p.n, B, q0, q1, first, last,
+                                                                             state, p.force, p.force64, sp.split);
             }
             e = hipGetLastError();
             if (e != hipSuccess) return e;

@@ -15,10 +15,10 @@
 // waves own a tile and the per-tile reaction sums enter LDS in a fixed order,
 // with one barrier per phase: no atomics anywhere.
 //
-// The diagonal of block P (its bodies against each other) comes after every
-// pair: in the single-system kernel as A one-sided pieces of 64*W bodies
-// each (sym_diag_piece), in the batched kernel as one task that takes each
-// pair of the block once (sym_diag_block, blocks of 512 on one wave).
+// The diagonal of block P (its bodies against each other) is A one-sided
+// pieces of 64*W bodies each (sym_diag_piece), or, in blocks of 512, takes
+// each pair of the block once: on one wave in the batched kernel
+// (sym_diag_block), on four in k_force_sym_deal (sym_deal_diag).
 //
 // Every body then has exactly one partial per block slot: slot Q for the i
 // side of (P, Q), slot P for its j side, slot P for the diagonal. The partials
@@ -35,6 +35,8 @@
 #pragma once
 
 #include "nbody_device.h"
+
+#include <type_traits>
 
 namespace nbody {
 
@@ -85,6 +87,7 @@ __device__ __forceinline__ void upper_pair(int t, int& P, int& Q)
     int q = (int)((sqrtf(8.0f * (float)t + 1.0f) + 1.0f) * 0.5f);
     while (q > 1 && q * (q - 1) / 2 > t) --q;
     while ((q + 1) * q / 2 <= t) ++q;
+    q = __builtin_amdgcn_readfirstlane(q);  // (the square root ran in vector registers)
     Q = q;
     P = t - q * (q - 1) / 2;
 }
@@ -174,26 +177,28 @@ __device__ __forceinline__ void upper_pair(int t, int& P, int& Q)
     "v_add_f32 %[Rz], %[Rz], %[rz]\n"
 
 // The chain's five temporaries (d, then s, then t = s^3) are either left to
-// the compiler or, with PIN, held in v21, v25, v29, v33 and v34. On gfx950
+// the compiler (REGS_FREE) or held in v21, v25, v29, v33 and v34. On gfx950
 // the issue rate of one instruction stream depends on which registers hold
 // them relative to the rest: the loop bodies run verbatim, ALU only, issue
-// 1.18 to 1.29 VALU instructions per clock per CU. The single-system kernel's
-// own allocation measures at the top of that range. In the batched kernel
-// the compiler picks a slow one, and pinning raises that kernel's rate by
-// about 7 %.
-// The batched kernel's steps (PIN) also sum each step's 8 reaction terms
+// 1.18 to 1.29 VALU instructions per clock per CU, and those five at the top
+// of that range. In the batched kernel the compiler picks a slow set, and
+// pinning raises its rate by about 7 %; in k_force_sym_deal, whose equal-mass
+// steps are REGS_PINNED, by 11 % (N = 98304: 1.74 and 1.57 ms). The general
+// step's own allocation there is as fast as the pinned one.
+// The batched kernel's steps (REGS_APART) also sum each step's 8 reaction terms
 // apart and add that partial to the running reaction (3 more VALU per 8
 // pairs, 1.2 % of its rate): the running j-side sums then take 64 roundings
 // per tile instead of 512, which keeps every system of the 512-system
 // ensemble within 1e-5 of the FP64 sum on its evolved states (1.8e-5
 // without). The single-system kernel keeps one running sum: it holds the
 // bound on its configured state without the extra adds.
-template <bool PIN>
+enum : int { REGS_FREE = 0, REGS_PINNED = 1, REGS_APART = 2 };
+template <int REGS>
 __device__ __forceinline__ void sym_step8(float& xj, float& yj, float& zj, float& mj, float& rx, float& ry, float& rz,
                                           Lanes<8>& acc, const Lanes<8>& me, const float (&mi)[8], float eps2)
 {
     float dx, dy, dz, s, t;
-    if constexpr (PIN) {
+    if constexpr (REGS == REGS_APART) {
         float qx, qy, qz;
         asm volatile(NBODY_SYM_PAIR_FIRST(0) NBODY_SYM_PAIR(1) NBODY_SYM_PAIR(2) NBODY_SYM_PAIR(3)
                      NBODY_SYM_PAIR(4) NBODY_SYM_PAIR(5) NBODY_SYM_PAIR(6) NBODY_SYM_PAIR(7)
@@ -311,12 +316,12 @@ __device__ __forceinline__ void sym_step8(float& xj, float& yj, float& zj, float
     "v_fmac_f32 %[ay" #u "], %[dy], %[t]\n"                                                            \
     "v_fmac_f32 %[az" #u "], %[dz], %[t]\n"
 
-template <bool PIN>
+template <int REGS>
 __device__ __forceinline__ void sym_step8_eq(float& xj, float& yj, float& zj, float& rx, float& ry, float& rz,
                                              Lanes<8>& acc, const Lanes<8>& me, float eps2)
 {
     float dx, dy, dz, s, t;
-    if constexpr (PIN) {
+    if constexpr (REGS == REGS_APART) {
         float qx, qy, qz;
         asm volatile(NBODY_SYM_PAIR_EQ_FIRST(0) NBODY_SYM_PAIR_EQ(1) NBODY_SYM_PAIR_EQ(2) NBODY_SYM_PAIR_EQ(3)
                      NBODY_SYM_PAIR_EQ(4) NBODY_SYM_PAIR_EQ(5) NBODY_SYM_PAIR_EQ(6) NBODY_SYM_PAIR_EQ(7)
@@ -325,6 +330,26 @@ __device__ __forceinline__ void sym_step8_eq(float& xj, float& yj, float& zj, fl
                      NBODY_ROR1(Rx) NBODY_ROR1(Ry) NBODY_ROR1(Rz)
                      : [xj] "+v"(xj), [yj] "+v"(yj), [zj] "+v"(zj), [Rx] "+v"(rx), [Ry] "+v"(ry), [Rz] "+v"(rz),
                        [rx] "=&v"(qx), [ry] "=&v"(qy), [rz] "=&v"(qz),
+                       [ax0] "+v"(acc.x[0]), [ax1] "+v"(acc.x[1]), [ax2] "+v"(acc.x[2]),
+                       [ax3] "+v"(acc.x[3]), [ax4] "+v"(acc.x[4]), [ax5] "+v"(acc.x[5]), [ax6] "+v"(acc.x[6]),
+                       [ax7] "+v"(acc.x[7]), [ay0] "+v"(acc.y[0]), [ay1] "+v"(acc.y[1]), [ay2] "+v"(acc.y[2]),
+                       [ay3] "+v"(acc.y[3]), [ay4] "+v"(acc.y[4]), [ay5] "+v"(acc.y[5]), [ay6] "+v"(acc.y[6]),
+                       [ay7] "+v"(acc.y[7]), [az0] "+v"(acc.z[0]), [az1] "+v"(acc.z[1]), [az2] "+v"(acc.z[2]),
+                       [az3] "+v"(acc.z[3]), [az4] "+v"(acc.z[4]), [az5] "+v"(acc.z[5]), [az6] "+v"(acc.z[6]),
+                       [az7] "+v"(acc.z[7]), [dx] "=&{v21}"(dx), [dy] "=&{v25}"(dy), [dz] "=&{v29}"(dz),
+                       [s] "=&{v33}"(s), [t] "=&{v34}"(t)
+                     : [x0] "v"(me.x[0]), [x1] "v"(me.x[1]), [x2] "v"(me.x[2]), [x3] "v"(me.x[3]),
+                       [x4] "v"(me.x[4]), [x5] "v"(me.x[5]), [x6] "v"(me.x[6]), [x7] "v"(me.x[7]),
+                       [y0] "v"(me.y[0]), [y1] "v"(me.y[1]), [y2] "v"(me.y[2]), [y3] "v"(me.y[3]),
+                       [y4] "v"(me.y[4]), [y5] "v"(me.y[5]), [y6] "v"(me.y[6]), [y7] "v"(me.y[7]),
+                       [z0] "v"(me.z[0]), [z1] "v"(me.z[1]), [z2] "v"(me.z[2]), [z3] "v"(me.z[3]),
+                       [z4] "v"(me.z[4]), [z5] "v"(me.z[5]), [z6] "v"(me.z[6]), [z7] "v"(me.z[7]), [eps] "s"(eps2));
+    } else if constexpr (REGS == REGS_PINNED) {
+        asm volatile(NBODY_SYM_PAIR_EQ(0) NBODY_SYM_PAIR_EQ(1) NBODY_SYM_PAIR_EQ(2) NBODY_SYM_PAIR_EQ(3)
+                     NBODY_SYM_PAIR_EQ(4) NBODY_SYM_PAIR_EQ(5) NBODY_SYM_PAIR_EQ(6) NBODY_SYM_PAIR_EQ(7)
+                     NBODY_ROR1(xj) NBODY_ROR1(yj) NBODY_ROR1(zj)
+                     NBODY_ROR1(rx) NBODY_ROR1(ry) NBODY_ROR1(rz)
+                     : [xj] "+v"(xj), [yj] "+v"(yj), [zj] "+v"(zj), [rx] "+v"(rx), [ry] "+v"(ry), [rz] "+v"(rz),
                        [ax0] "+v"(acc.x[0]), [ax1] "+v"(acc.x[1]), [ax2] "+v"(acc.x[2]),
                        [ax3] "+v"(acc.x[3]), [ax4] "+v"(acc.x[4]), [ax5] "+v"(acc.x[5]), [ax6] "+v"(acc.x[6]),
                        [ax7] "+v"(acc.x[7]), [ay0] "+v"(acc.y[0]), [ay1] "+v"(acc.y[1]), [ay2] "+v"(acc.y[2]),
@@ -565,10 +590,52 @@ __device__ __forceinline__ void sym_diag_step8(float& xj, float& yj, float& zj, 
 #undef NBODY_SYM_PAIR
 #undef NBODY_ROR1
 
+// One rotation step with A i bodies per lane: the assembly chain for 8 and 2,
+// else (and with a Newton step) the generic loop, which it equals bit for bit.
+template <int A, bool NEWTON, bool EQ, int REGS>
+__device__ __forceinline__ void sym_step(float& xj, float& yj, float& zj, float& mj, float& rx, float& ry, float& rz,
+                                         Lanes<A>& acc, const Lanes<A>& me, const float (&mi)[A], float eps2)
+{
+    if constexpr (A == 8 && !NEWTON) {
+        if constexpr (EQ) sym_step8_eq<REGS>(xj, yj, zj, rx, ry, rz, acc, me, eps2);
+        else sym_step8<REGS>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+    } else if constexpr (A == 2 && !NEWTON) {
+        if constexpr (EQ) sym_step2_eq(xj, yj, zj, rx, ry, rz, acc, me, eps2);
+        else sym_step2(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+    } else {
+#pragma unroll
+        for (int u = 0; u < A; ++u) {
+            const float dx = xj - me.x[u];
+            const float dy = yj - me.y[u];
+            const float dz = zj - me.z[u];
+            float d2 = __builtin_fmaf(dx, dx, eps2);
+            d2 = __builtin_fmaf(dy, dy, d2);
+            d2 = __builtin_fmaf(dz, dz, d2);
+            const float inv = rsqrt_f32<NEWTON>(d2);
+            const float inv3 = (inv * inv) * inv;
+            const float si = EQ ? inv3 : mj * inv3;
+            const float sj = EQ ? -inv3 : -mi[u] * inv3;
+            acc.x[u] = __builtin_fmaf(dx, si, acc.x[u]);
+            acc.y[u] = __builtin_fmaf(dy, si, acc.y[u]);
+            acc.z[u] = __builtin_fmaf(dz, si, acc.z[u]);
+            rx = __builtin_fmaf(dx, sj, rx);
+            ry = __builtin_fmaf(dy, sj, ry);
+            rz = __builtin_fmaf(dz, sj, rz);
+        }
+        xj = wave_ror1(xj);
+        yj = wave_ror1(yj);
+        zj = wave_ror1(zj);
+        if constexpr (!EQ) mj = wave_ror1(mj);
+        rx = wave_ror1(rx);
+        ry = wave_ror1(ry);
+        rz = wave_ror1(rz);
+    }
+}
+
 // The phases of block pair (P, Q): every wave streams the T tiles of block Q
 // past its A i bodies per lane, adding the i side into acc and each tile's
 // reaction into jacc. With EQ the pair weights leave out the (common) mass.
-template <int A, int W, bool NEWTON, bool EQ, bool PIN>
+template <int A, int W, bool NEWTON, bool EQ, int REGS>
 __device__ __forceinline__ void sym_phases(const float4* __restrict__ pm, int n, float eps2, int Q,
                                            const Lanes<A>& me, const float (&mi)[A], Lanes<A>& acc,
                                            float (*jacc)[64 * A * W])
@@ -589,44 +656,7 @@ __device__ __forceinline__ void sym_phases(const float4* __restrict__ pm, int n,
             const float4 b = lane < n - jbase ? pm[jbase + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
             float xj = b.x, yj = b.y, zj = b.z, mj = b.w;
             float rx = 0.f, ry = 0.f, rz = 0.f;
-            for (int k = 0; k < 64; ++k) {
-                if constexpr (A == 8 && !NEWTON) {
-                    if constexpr (EQ) sym_step8_eq<PIN>(xj, yj, zj, rx, ry, rz, acc, me, eps2);
-                    else sym_step8<PIN>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
-                    continue;
-                }
-                if constexpr (A == 2 && !NEWTON) {
-                    if constexpr (EQ) sym_step2_eq(xj, yj, zj, rx, ry, rz, acc, me, eps2);
-                    else sym_step2(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
-                    continue;
-                }
-#pragma unroll
-                for (int u = 0; u < A; ++u) {
-                    const float dx = xj - me.x[u];
-                    const float dy = yj - me.y[u];
-                    const float dz = zj - me.z[u];
-                    float d2 = __builtin_fmaf(dx, dx, eps2);
-                    d2 = __builtin_fmaf(dy, dy, d2);
-                    d2 = __builtin_fmaf(dz, dz, d2);
-                    const float inv = rsqrt_f32<NEWTON>(d2);
-                    const float inv3 = (inv * inv) * inv;
-                    const float si = EQ ? inv3 : mj * inv3;
-                    const float sj = EQ ? -inv3 : -mi[u] * inv3;
-                    acc.x[u] = __builtin_fmaf(dx, si, acc.x[u]);
-                    acc.y[u] = __builtin_fmaf(dy, si, acc.y[u]);
-                    acc.z[u] = __builtin_fmaf(dz, si, acc.z[u]);
-                    rx = __builtin_fmaf(dx, sj, rx);
-                    ry = __builtin_fmaf(dy, sj, ry);
-                    rz = __builtin_fmaf(dz, sj, rz);
-                }
-                xj = wave_ror1(xj);
-                yj = wave_ror1(yj);
-                zj = wave_ror1(zj);
-                if constexpr (!EQ) mj = wave_ror1(mj);
-                rx = wave_ror1(rx);
-                ry = wave_ror1(ry);
-                rz = wave_ror1(rz);
-            }
+            for (int k = 0; k < 64; ++k) sym_step<A, NEWTON, EQ, REGS>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
             const int slot = tile * 64 + lane;
             jacc[0][slot] += rx;
             jacc[1][slot] += ry;
@@ -651,7 +681,7 @@ __device__ __forceinline__ bool workgroup_all(bool ok)
 // weights leave the mass out and the partials are multiplied by it once, at
 // the store; with m = 1 (or any power of two) the result is bit-identical to
 // the general weights.
-template <int A, int W, bool NEWTON, bool PIN = false>
+template <int A, int W, bool NEWTON, int REGS = REGS_FREE>
 __device__ __forceinline__ void sym_pair(const float4* __restrict__ pm, int n, float eps2, const SlotMap& slots, int P,
                                          int Q, float (*jacc)[64 * A * W])
 {
@@ -681,8 +711,8 @@ __device__ __forceinline__ void sym_pair(const float4* __restrict__ pm, int n, f
     for (int k = threadIdx.x; k < B; k += 64 * W) jacc[0][k] = jacc[1][k] = jacc[2][k] = 0.f;
     __syncthreads();
     const bool eq = workgroup_all<W>(same);
-    if (eq) sym_phases<A, W, NEWTON, true, PIN>(pm, n, eps2, Q, me, mi, acc, jacc);
-    else sym_phases<A, W, NEWTON, false, PIN>(pm, n, eps2, Q, me, mi, acc, jacc);
+    if (eq) sym_phases<A, W, NEWTON, true, REGS>(pm, n, eps2, Q, me, mi, acc, jacc);
+    else sym_phases<A, W, NEWTON, false, REGS>(pm, n, eps2, Q, me, mi, acc, jacc);
     const float scale = eq ? m0 : 1.0f;
     float* __restrict__ jdst = slots.j_side(P, Q, B);
     for (int k = threadIdx.x; k < B; k += 64 * W) {
@@ -709,25 +739,43 @@ __device__ __forceinline__ void sym_pair(const float4* __restrict__ pm, int n, f
 // so this covers every pair of the 64 exactly once. When the tile's
 // reactions come home after 64 steps they sit in the lanes that hold the
 // same bodies' i sums, and are added there: no LDS, no cross-lane traffic.
+// `which` 0 or 1 takes steps 0..31 or 32..63 alone, -1 all of them. The second
+// half starts half a turn on; the first one's reactions end half a turn from
+// home and are brought there across the wave.
+template <int T, bool EQ>
+__device__ __forceinline__ void sym_diag_tile(const float4* __restrict__ pm, int n, float eps2, int P, int which,
+                                              const Lanes<8>& me, const float (&mi)[8], Lanes<8>& acc)
+{
+    const int jbase = P * 512 + T * 64;  // wave-uniform
+    if (jbase >= n) return;              // the rest of the block is padding
+    const int lane = threadIdx.x & 63, from = which == 1 ? lane ^ 32 : lane;
+    const float4 b = from < n - jbase ? pm[jbase + from] : make_float4(0.f, 0.f, 0.f, 0.f);
+    float xj = b.x, yj = b.y, zj = b.z, mj = b.w;
+    float rx = 0.f, ry = 0.f, rz = 0.f;
+    constexpr unsigned long long upper = 0xffffffff00000000ull;  // lanes 32..63
+    if (which != 1) {
+        // step 0: the tile meets itself lane by lane (self pairs, skipped)
+        sym_diag_step8<T, 0, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
+        for (int k = 1; k < 32; ++k) sym_diag_step8<T, 1, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
+    }
+    if (which != 0) {
+        sym_diag_step8<T, 2, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
+        for (int k = 33; k < 64; ++k) sym_diag_step8<T, 0, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
+    } else {
+        rx = __shfl_xor(rx, 32);
+        ry = __shfl_xor(ry, 32);
+        rz = __shfl_xor(rz, 32);
+    }
+    acc.x[T] += rx;
+    acc.y[T] += ry;
+    acc.z[T] += rz;
+}
+
 template <int T, bool EQ>
 __device__ __forceinline__ void sym_diag_phases(const float4* __restrict__ pm, int n, float eps2, int P,
                                                 const Lanes<8>& me, const float (&mi)[8], Lanes<8>& acc)
 {
-    const int jbase = P * 512 + T * 64;  // wave-uniform
-    if (jbase >= n) return;              // the rest of the block is padding
-    const int lane = threadIdx.x & 63;
-    const float4 b = lane < n - jbase ? pm[jbase + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
-    float xj = b.x, yj = b.y, zj = b.z, mj = b.w;
-    float rx = 0.f, ry = 0.f, rz = 0.f;
-    constexpr unsigned long long upper = 0xffffffff00000000ull;  // lanes 32..63
-    // step 0: the tile meets itself lane by lane (self pairs, skipped)
-    sym_diag_step8<T, 0, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
-    for (int k = 1; k < 32; ++k) sym_diag_step8<T, 1, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
-    sym_diag_step8<T, 2, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
-    for (int k = 33; k < 64; ++k) sym_diag_step8<T, 0, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
-    acc.x[T] += rx;
-    acc.y[T] += ry;
-    acc.z[T] += rz;
+    sym_diag_tile<T, EQ>(pm, n, eps2, P, -1, me, mi, acc);
     if constexpr (T + 1 < 8) sym_diag_phases<T + 1, EQ>(pm, n, eps2, P, me, mi, acc);
 }
 
@@ -765,6 +813,91 @@ __device__ __forceinline__ void sym_diag_block(const float4* __restrict__ pm, in
         part[o] = acc.x[u] * scale;
         part[plane + o] = acc.y[u] * scale;
         part[2 * plane + o] = acc.z[u] * scale;
+    }
+}
+
+// Tiles t0, t0 + step, ... < t1 of the block that starts at body j0 past this
+// wave's 512 i bodies, the i side into acc. With halves = 1 each tile takes
+// its 64 steps and its reactions times `scale` go to their place in jdst (this
+// wave alone meets the tile with these i bodies). With halves = 2 (one tile)
+// this wave takes steps 0..31 (half 0) or 32..63 (half 1), where it starts
+// half a turn on, and leaves the scaled reactions in r: half 0's in the lane
+// half a turn from the body's, half 1's in the body's own lane.
+template <bool NEWTON, bool EQ>
+__device__ __forceinline__ void sym_deal_tiles(const float4* __restrict__ pm, int n, float eps2, int j0, int t0,
+                                               int t1, int step, int half, int halves, const Lanes<8>& me,
+                                               const float (&mi)[8], Lanes<8>& acc, float* jdst, size_t plane,
+                                               float scale, float (&r)[3])
+{
+    const int lane = threadIdx.x & 63;
+    float rx = 0.f, ry = 0.f, rz = 0.f;
+    for (int tile = t0; tile < t1; tile += step) {
+        const int jbase = j0 + tile * 64;  // wave-uniform
+        if (jbase >= n) break;             // the rest of the block is padding
+        const int from = lane ^ (half * 32);
+        const float4 b = from < n - jbase ? pm[jbase + from] : make_float4(0.f, 0.f, 0.f, 0.f);
+        float xj = b.x, yj = b.y, zj = b.z, mj = b.w;
+        rx = ry = rz = 0.f;
+        const int steps = halves == 2 ? 32 : 64;
+        for (int k = 0; k < steps; ++k)
+            sym_step<8, NEWTON, EQ, EQ ? REGS_PINNED : REGS_FREE>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+        rx *= scale;
+        ry *= scale;
+        rz *= scale;
+        if (halves == 1) {
+            float* dst = jdst + tile * 64;
+            dst[lane] = rx;
+            dst[plane + lane] = ry;
+            dst[2 * plane + lane] = rz;
+        }
+    }
+    r[0] = rx;
+    r[1] = ry;
+    r[2] = rz;
+}
+
+// This wave's share of block P's diagonal (blocks of 512, 4 waves): tiles w
+// and 7 - w against the sub-blocks before them and their own, 7 tile blocks
+// and two halves on every wave, all 64 steps or those of one half (halves = 2).
+// With a Newton step (whose pair chains are not in assembly): sub-blocks w and
+// w + 4 one-sided, against the block or one half of it.
+template <bool NEWTON>
+__device__ __forceinline__ void sym_deal_diag(const float4* __restrict__ pm, int n, float eps2, int P, int wave,
+                                              int half, int halves, bool eq, const Lanes<8>& me, const float (&mi)[8],
+                                              Lanes<8>& acc)
+{
+    if constexpr (NEWTON) {
+        const int j0 = P * 512 + half * 256, len = min(n - j0, halves == 2 ? 256 : 512);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            if ((u & 3) != wave || len <= 0) continue;
+            Lanes<1> one, sum;
+            one.x[0] = me.x[u];
+            one.y[0] = me.y[u];
+            one.z[0] = me.z[u];
+            zero<1>(sum);
+            sweep_sgpr<1, true>(pm + j0, len, eps2, one, sum);
+            acc.x[u] = sum.x[0];
+            acc.y[u] = sum.y[0];
+            acc.z[u] = sum.z[0];
+        }
+    } else {
+        const int which = halves == 2 ? half : -1;
+        auto tiles = [&](auto lo, auto hi) {
+            if (eq) {
+                sym_diag_tile<lo, true>(pm, n, eps2, P, which, me, mi, acc);
+                sym_diag_tile<hi, true>(pm, n, eps2, P, which, me, mi, acc);
+            } else {
+                sym_diag_tile<lo, false>(pm, n, eps2, P, which, me, mi, acc);
+                sym_diag_tile<hi, false>(pm, n, eps2, P, which, me, mi, acc);
+            }
+        };
+        switch (wave) {
+        case 0: tiles(std::integral_constant<int, 0>{}, std::integral_constant<int, 7>{}); break;
+        case 1: tiles(std::integral_constant<int, 1>{}, std::integral_constant<int, 6>{}); break;
+        case 2: tiles(std::integral_constant<int, 2>{}, std::integral_constant<int, 5>{}); break;
+        default: tiles(std::integral_constant<int, 3>{}, std::integral_constant<int, 4>{});
+        }
     }
 }
 

@@ -1,0 +1,44 @@
+"""The symmetric plan with 8 bodies per lane and blocks of 512, whose block
+pairs are 1, 2 or 4 tasks each: every split at the sizes where a block, a
+half or a tile is ragged, empty or alone, on unequal masses, one mass, and
+one mass with one heavier body, against the FP64 oracle.
+
+Tolerance: the path's own (max 1e-5, RMS 1e-6 per body): FP32 terms, sums of
+at most 512 terms per lane, TwoSum over the slots.
+"""
+import numpy as np
+import pytest
+
+from conftest import EPS2
+from gpu_util import dev, run_force
+from oracle_lib import force_errors
+
+from nbody_amd import _native, ics
+
+pytestmark = pytest.mark.gpu
+
+TOL_MAX, TOL_RMS = 1e-5, 1e-6
+SHAPE = dict(variant=_native.SYMMETRIC, i_per_lane=8, jslice=512)
+
+
+@pytest.mark.parametrize("n", [2, 64, 511, 512, 513, 577, 1024, 1500, 3 * 512 + 320, 5003])
+@pytest.mark.parametrize("split", [1, 2, 4])
+@pytest.mark.parametrize("newton", [0, 1])
+def test_every_split(oracle, n, split, newton):
+    """A slot budget of `split` times one task's slots (12 bytes per body and
+    block) allows at most that many tasks per pair."""
+    nb = -(-n // 512)
+    budget = split * 12 * 512 * nb * nb
+    pm, _ = ics.random_unit_bodies(n, seed=31)
+    one = pm.copy()
+    one[:, 3] = 0.37
+    heavier = one.copy()
+    heavier[n // 2, 3] = 0.6
+    for what, x in (("unequal", pm), ("one mass", one), ("one heavier", heavier)):
+        d = dev(x)
+        f = run_force(d, EPS2, slot_bytes=budget, newton=newton, **SHAPE)
+        mx, rms = force_errors(f, oracle.fp64_forces(x, EPS2))
+        assert mx <= TOL_MAX and rms <= TOL_RMS, (what, n, split, newton, mx, rms)
+        assert np.all(f[:, 3] == -7.0)
+        again = run_force(d, EPS2, slot_bytes=budget, newton=newton, **SHAPE)
+        assert np.array_equal(f.view(np.uint32), again.view(np.uint32)), (what, n, split, newton)
