@@ -47,7 +47,7 @@ enum {
     NBODY_HIP_DPP = 2,       /* j tile passed around the wave64 by DPP (src/nbody_GPU_Shuffle.cu:44-107) */
     NBODY_HIP_SGPR = 3,      /* scalar-memory broadcast (src/nbody_GPU_AOS_const.cu:45-121) */
     NBODY_HIP_SYMMETRIC = 4, /* each pair once, no global atomics (src/nbody_GPU_AOS_tiled.cu:44-220) */
-    NBODY_HIP_AUTO = -1      /* the autotuned plan, else SYMMETRIC for whole systems of N >= 1024, else LDS */
+    NBODY_HIP_AUTO = -1      /* the autotuned plan, else SYMMETRIC for whole systems of N > 10240, else LDS */
 };
 
 /* Options of the general entry; zero / -1 fields mean "choose".
@@ -88,7 +88,7 @@ float ComputeGravitation_HIP_SGPR(float *force, float *posMass, float softeningS
  * with the reaction scaled by m_i (the reference scales it by m_j). */
 float ComputeGravitation_HIP_Symmetric(float *force, float *posMass, float softeningSquared, size_t N);
 /* The library's choice for N: the plan nbody_hip_autotune found for this N
- * if it ran, else the symmetric kernel (whole systems, N >= 1024) or LDS. */
+ * if it ran, else the symmetric kernel (whole systems, N > 10240) or LDS. */
 float ComputeGravitation_HIP(float *force, float *posMass, float softeningSquared, size_t N);
 
 /* Host-pointer twin with the ALGORITHM_AOS contract (src/nbody.cu:343-349): force and posMass are
@@ -180,7 +180,10 @@ int nbody_hip_energy_fp64(double *out, const float *posMass, const float *velInv
 /* ---- plans and tuning ---------------------------------------------------- */
 
 /* The plan the library would use: fills variant, i_per_lane, jslice,
- * compensated, newton for an n-body i range of an N-body system. */
+ * compensated, newton for an n-body i range of an N-body system. LDS with
+ * i_per_lane and jslice 0 is the one-launch plan of small evaluations (n N up
+ * to 10240^2, plain sums, no shape given): it keeps no partial sums, and the
+ * same zeros select it again. */
 int nbody_hip_plan(size_t N, size_t n, const nbody_hip_options *opt, nbody_hip_options *plan);
 /* Time candidate plans of `variant` (NBODY_HIP_AUTO: the LDS, SGPR and
  * symmetric families) on the given device data, force kernel plus slice

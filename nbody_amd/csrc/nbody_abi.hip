@@ -73,6 +73,22 @@ constexpr int kSymSlotsTarget = 512;
 // against 22.5.
 constexpr size_t kSmallSymN = 5120;
 
+// Interactions up to which the LDS variant runs as one launch over the whole
+// j range (nbody_tile.h), and whole systems do so instead of the symmetric
+// plan. Whole systems, that kernel and the symmetric plan: N = 4096 8.1 and
+// 16.2 us, 8192 22 and 24, 10000 33 and 35, 12288 45 and 43.
+constexpr double kTileMaxWork = 10240.0 * 10240.0;
+
+// Whether an n-body i range of N bodies runs so: with plain sums, no Newton
+// step and nothing of the shape fixed.
+bool tile_plan(size_t N, size_t n, const nbody_hip_options* opt)
+{
+    const int comp_opt = opt ? opt->compensated : -1;
+    const bool comp = comp_opt < 0 ? N > 65536 : comp_opt > 0;
+    const bool shape_given = opt && (opt->i_per_lane > 0 || opt->jslice > 0 || opt->waves_per_simd > 0);
+    return n > 0 && !comp && !shape_given && !(opt && opt->newton > 0) && (double)n * (double)N <= kTileMaxWork;
+}
+
 // Default decomposition: enough blocks for ~48 waves per SIMD (the dispatcher
 // balances them across the 256 CUs), j slices of at least 1024 bodies in
 // multiples of 256.
@@ -123,6 +139,12 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
         p.comp = false;
         return p;
     }
+    if (variant == VAR_LDS && tile_plan(N, n, opt)) {
+        tile_shape(N, n, &p.li, &p.ipl);
+        p.jslice = (int)N;
+        p.nslices = 1;
+        return p;
+    }
     p.ipl = (opt && opt->i_per_lane > 0) ? opt->i_per_lane : 1;
     if (variant == VAR_DPP && !(opt && opt->i_per_lane > 0)) {
         // the rotation's 4 moves per step are shared by the lane's i bodies:
@@ -147,15 +169,16 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
 }
 
 // The untuned choice for NBODY_HIP_AUTO: the symmetric kernel for whole
-// systems of at least two of its blocks (half the pairs, 14-16 VALU + 1 rsq
-// per pair); otherwise the LDS broadcast, whose VALU operands all sit in VGPRs
-// (gfx950 issues those faster than ops reading an SGPR).
+// systems past kTileMaxWork (half the pairs, 14-16 VALU + 1 rsq per pair);
+// otherwise the LDS broadcast, whose VALU operands all sit in VGPRs (gfx950
+// issues those faster than ops reading an SGPR), in one launch where small.
 // Largest block count of a symmetric plan (the pair index must fit an int).
 constexpr int kMaxSymBlocks = 16384;
 
-int auto_variant(size_t N, size_t n)
+int auto_variant(size_t N, size_t n, const nbody_hip_options* opt)
 {
     if (n != N || N < 1024) return VAR_LDS;
+    if (tile_plan(N, n, opt) && !(opt && opt->slot_bytes > 0)) return VAR_LDS;
     const ForcePlan p = default_plan(VAR_SYMMETRIC, N, N, 1, nullptr);
     return p.nslices <= kMaxSymBlocks ? VAR_SYMMETRIC : VAR_LDS;
 }
@@ -197,6 +220,7 @@ int validate_plan(const ForcePlan& p, size_t N)
         }
         return OK;
     }
+    if (p.li > 0) return OK;  // a shape of tile_shape's
     if (p.ipl != 1 && p.ipl != 2 && p.ipl != 4 && !(p.ipl == 8 && p.variant == VAR_DPP)) {
         set_error("i_per_lane must be 1, 2 or 4 (8 also for the DPP variant; got %d)", p.ipl);
         return E_ARG;
@@ -207,7 +231,7 @@ int validate_plan(const ForcePlan& p, size_t N)
 int make_plan(DeviceState& d, size_t N, size_t n, const nbody_hip_options* opt, ForcePlan* plan)
 {
     const int requested = opt ? opt->variant : NBODY_HIP_AUTO;
-    const int variant = requested == NBODY_HIP_AUTO ? auto_variant(N, n) : requested;
+    const int variant = requested == NBODY_HIP_AUTO ? auto_variant(N, n, opt) : requested;
     if (variant < 0 || variant >= VAR_COUNT) {
         set_error("unknown variant %d", requested);
         return E_ARG;
@@ -222,6 +246,19 @@ int make_plan(DeviceState& d, size_t N, size_t n, const nbody_hip_options* opt, 
     if (int r = validate_plan(p, N)) return r;
     *plan = p;
     return OK;
+}
+
+void describe_plan(const ForcePlan& p, nbody_hip_options* out)
+{
+    // the one-launch kernel has no slices and its shape is no option: zeros
+    // ("choose"), with which the same sizes get the same plan again
+    out->variant = p.variant;
+    out->i_per_lane = p.li > 0 ? 0 : p.ipl;
+    out->jslice = p.li > 0 ? 0 : p.jslice;
+    out->compensated = p.acc64 ? 2 : p.comp ? 1 : 0;
+    out->newton = p.newton ? 1 : 0;
+    out->waves_per_simd = p.occ;
+    out->slot_bytes = p.band_cap;
 }
 
 int check_args(const void* force, const void* pm, size_t N, size_t base, size_t n)
@@ -676,13 +713,7 @@ int nbody_hip_plan(size_t N, size_t n, const nbody_hip_options* opt, nbody_hip_o
     if (int r = device_state(&d)) return r;
     ForcePlan p;
     if (int r = make_plan(*d, N, n, opt, &p)) return r;
-    out->variant = p.variant;
-    out->i_per_lane = p.ipl;
-    out->jslice = p.jslice;
-    out->compensated = p.acc64 ? 2 : p.comp ? 1 : 0;
-    out->newton = p.newton ? 1 : 0;
-    out->waves_per_simd = p.occ;
-    out->slot_bytes = p.band_cap;
+    describe_plan(p, out);
     return OK;
 }
 
@@ -729,6 +760,7 @@ float nbody_hip_autotune(float* force, const float* posMass, float softeningSqua
                 }
             }
         } else {
+            if (ForcePlan c = default_plan(fam, N, N, d->cus, &o); c.li > 0) cands.push_back(c);
             for (int ipl : {1, 2, 4, 8}) {
                 if (ipl == 8 && fam != VAR_DPP) continue;
                 o.i_per_lane = ipl;

@@ -153,6 +153,17 @@ __device__ __forceinline__ void zero(Lanes<I>& a)
     for (int u = 0; u < I; ++u) a.x[u] = a.y[u] = a.z[u] = 0.f;
 }
 
+template <int I>
+__device__ __forceinline__ void scale(Lanes<I>& a, float m)
+{
+#pragma unroll
+    for (int u = 0; u < I; ++u) {
+        a.x[u] *= m;
+        a.y[u] *= m;
+        a.z[u] *= m;
+    }
+}
+
 // hi += part with TwoSum, residue into lo.
 template <int I>
 __device__ __forceinline__ void fold(Lanes<I>& hi, Lanes<I>& lo, const Lanes<I>& part)

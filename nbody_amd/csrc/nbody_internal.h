@@ -126,6 +126,8 @@ int device_state(DeviceState** out);
 int round_up(int v, int m);
 ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip_options* opt);
 int make_plan(DeviceState& d, size_t N, size_t n, const nbody_hip_options* opt, ForcePlan* plan);
+// The plan as options (nbody_hip_plan, nbody_hip_system_plan).
+void describe_plan(const ForcePlan& p, nbody_hip_options* out);
 int check_args(const void* force, const void* pm, size_t N, size_t base, size_t n);
 // Queue one force evaluation on `stream`. Slice/slot scratch comes from
 // `own` (the device's shared buffer when null; a caller that captures the

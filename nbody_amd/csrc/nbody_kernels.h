@@ -27,6 +27,7 @@ struct ForcePlan {
     int ipl = 1;        // i bodies per lane: 1, 2, 4 (symmetric: 2, 4 or 8)
     int jslice = 0;     // j bodies per slice (symmetric: bodies per block)
     int nslices = 1;    // ceil(n / jslice)
+    int li = 0;         // LDS: > 0 runs the one-launch kernel (nbody_tile.h), li lanes times ipl i bodies a workgroup
     bool comp = false;  // TwoSum-compensated accumulation
     bool acc64 = false; // every term added in FP64, partial sums kept in FP64 (LDS and symmetric)
     bool newton = false;
@@ -64,6 +65,9 @@ struct ForceParams {
                                  // written instead of force
     float* force = nullptr;      // 4 floats per i body; x, y, z written, w left alone
 };
+
+// The shape of the one-launch kernel that ends first for ni of n bodies.
+void tile_shape(size_t n, size_t ni, int* li, int* ipl);
 
 // Whether (i per lane, block size) is a compiled symmetric shape.
 bool symmetric_shape_ok(int ipl, int block);

@@ -17,6 +17,7 @@
 #include "nbody_device.h"
 #include "nbody_kernels.h"
 #include "nbody_sym.h"
+#include "nbody_tile.h"
 
 #include <algorithm>
 #include <cmath>
@@ -87,17 +88,6 @@ __device__ __forceinline__ bool uniform_mass(const float4* __restrict__ src, int
     bool ok = true;
     for (int k = threadIdx.x & 63; k < len; k += 64) ok &= src[k].w == m0;
     return __builtin_amdgcn_ballot_w64(!ok) == 0;
-}
-
-template <int I>
-__device__ __forceinline__ void scale(Lanes<I>& a, float m)
-{
-#pragma unroll
-    for (int u = 0; u < I; ++u) {
-        a.x[u] *= m;
-        a.y[u] *= m;
-        a.z[u] *= m;
-    }
 }
 
 // A slice's sums into hi through sweep(c, len, acc), which adds the terms of
@@ -905,6 +895,22 @@ hipError_t go_family(const ForcePlan& plan, dim3 g, hipStream_t s, const ForcePa
     return hipGetLastError();
 }
 
+hipError_t go_tile(const ForcePlan& plan, dim3 g, hipStream_t s, const ForceParams& p)
+{
+    switch (plan.li * 100 + plan.ipl) {
+    case 401: k_force_tile<4, 1><<<g, kTileThreads, 0, s>>>(p); break;
+    case 402: k_force_tile<4, 2><<<g, kTileThreads, 0, s>>>(p); break;
+    case 403: k_force_tile<4, 3><<<g, kTileThreads, 0, s>>>(p); break;
+    case 802: k_force_tile<8, 2><<<g, kTileThreads, 0, s>>>(p); break;
+    case 803: k_force_tile<8, 3><<<g, kTileThreads, 0, s>>>(p); break;
+    case 804: k_force_tile<8, 4><<<g, kTileThreads, 0, s>>>(p); break;
+    case 805: k_force_tile<8, 5><<<g, kTileThreads, 0, s>>>(p); break;
+    case 806: k_force_tile<8, 6><<<g, kTileThreads, 0, s>>>(p); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 // Resident workgroups per CU of `kernel` with `dyn` bytes of dynamic LDS.
 int blocks_per_cu(const void* kernel, int threads, size_t dyn)
 {
@@ -1042,6 +1048,39 @@ int natural_occupancy(bool newton)
 
 }  // namespace
 
+namespace {
+
+// The compiled shapes of k_force_tile and the clocks of a CU one interaction
+// takes in them when the workgroups fill it (measured at N = 8192 to 16384).
+struct TileShape {
+    int li, ipl;
+    double clocks;
+};
+constexpr TileShape kTileShapes[] = {{4, 1, .263}, {4, 2, .200}, {4, 3, .183}, {8, 2, .175},
+                                     {8, 3, .172}, {8, 4, .180}, {8, 5, .178}, {8, 6, .175}};
+
+}  // namespace
+
+void tile_shape(size_t n, size_t ni, int* li, int* ipl)
+{
+    constexpr size_t cus = 256;
+    double least = 0.0;
+    for (const TileShape& s : kTileShapes) {
+        const size_t ti = (size_t)s.li * s.ipl, groups = (ni + ti - 1) / ti, per_cu = s.ipl <= 3 ? 2 : 1;
+        const double work = (double)ti * (double)n * s.clocks;  // of one workgroup, on a full CU
+        const double fixed = 4000.0 + 900.0 * s.ipl;            // launch, first loads, last sum
+        const size_t full = groups / (per_cu * cus), rest = groups % (per_cu * cus);
+        double t = (double)full * ((double)per_cu * work + fixed);
+        // a last round of one workgroup per CU has half the waves where two fit
+        if (rest) t += fixed + (rest > cus ? 2.0 * work : per_cu == 2 ? 1.15 * work : work);
+        if (least == 0.0 || t < least) {
+            least = t;
+            *li = s.li;
+            *ipl = s.ipl;
+        }
+    }
+}
+
 bool symmetric_shape_ok(int ipl, int block)
 {
     const int w = block / (64 * ipl);
@@ -1129,6 +1168,12 @@ hipError_t launch_force(const ForcePlan& plan, const ForceParams& p, hipStream_t
         if (plan.newton) k_force_aos<true><<<g, kBlock, 0, stream>>>(q);
         else k_force_aos<false><<<g, kBlock, 0, stream>>>(q);
         e = hipGetLastError();
+        if (e == hipSuccess && after) e = hipEventRecord(after, stream);
+        return e;
+    }
+    if (plan.li > 0) {
+        const dim3 g((p.ni + plan.li * plan.ipl - 1) / (plan.li * plan.ipl));
+        e = go_tile(plan, g, stream, p);
         if (e == hipSuccess && after) e = hipEventRecord(after, stream);
         return e;
     }
