@@ -35,8 +35,9 @@ nbody_hip_system *nbody_hip_system_create(const float *posMass, const float *vel
                                           const nbody_hip_options *opt);
 /* Runs `steps` steps and waits for them; *ms (may be NULL) receives their
  * elapsed time measured with events on the system's stream. use_graph = 1
- * replays one captured graph per step (force kernel, slice/slot reduction,
- * integrator; captured on first use). */
+ * replays a captured graph of 16 steps (force kernel, slice/slot reduction,
+ * integrator; captured on first use) as often as it fits and launches the
+ * remaining steps one by one. */
 int nbody_hip_system_run(nbody_hip_system *s, int steps, int use_graph, float *ms);
 /* Copies the current state (and the last force) to the host; NULL skips one. */
 int nbody_hip_system_read(const nbody_hip_system *s, float *posMass, float *velInvMass, float *force);

@@ -280,7 +280,7 @@ int check_args(const void* force, const void* pm, size_t N, size_t base, size_t 
 
 // Queue one force evaluation on `stream` (caller holds g_mutex).
 int run_force(DeviceState& d, const ForcePlan& plan, float* force, const float* pm, float eps2, size_t N, size_t base,
-              size_t n, hipStream_t stream, Buffer* own, bool timed, double* force64)
+              size_t n, hipStream_t stream, Buffer* own, bool timed, double* force64, const StepParams* step)
 {
     Buffer& buf = own ? *own : d.partial;
     if (plan.variant == VAR_SYMMETRIC && (base != 0 || n != N)) {
@@ -297,6 +297,7 @@ int run_force(DeviceState& d, const ForcePlan& plan, float* force, const float* 
     p.nslices = plan.nslices;
     p.force = force;
     p.force64 = force64;
+    if (step) p.step = *step;
     const size_t bytes = plan_scratch_bytes(plan, (int)n);
     const bool shared = bytes && !own;
     if (shared) {

@@ -119,8 +119,7 @@ __global__ __launch_bounds__(kWave) void k_force_batch64(const ForceTask* __rest
 // each slot row read as one contiguous run), then the first kBodyTaskBodies
 // threads integrate. The slot sum is k_reduce_band's (slot order, TwoSum,
 // rounded once) for FP32 slots and k_reduce_band64's (slot order, FP64,
-// rounded once) for FP64 slots; the update is k_integrate's, all in
-// nbody_kernels.hip.
+// rounded once) for FP64 slots, both in nbody_kernels.hip.
 template <class T>
 __global__ __launch_bounds__(3 * kBodyTaskBodies) void k_reduce_integrate_batch(const BodyTask* __restrict__ tasks,
                                                                                 float dt, float damping,
@@ -177,19 +176,7 @@ __global__ __launch_bounds__(3 * kBodyTaskBodies) void k_reduce_integrate_batch(
     g.y = sum[1][lane];
     g.z = sum[2][lane];
     task.force[i] = g;
-    float4 p = task.pm[i];
-    float4 v = task.vm[i];
-    v.x = __builtin_fmaf(v.w, g.x * dt, v.x);
-    v.y = __builtin_fmaf(v.w, g.y * dt, v.y);
-    v.z = __builtin_fmaf(v.w, g.z * dt, v.z);
-    v.x *= damping;
-    v.y *= damping;
-    v.z *= damping;
-    p.x = __builtin_fmaf(v.x, dt, p.x);
-    p.y = __builtin_fmaf(v.y, dt, p.y);
-    p.z = __builtin_fmaf(v.z, dt, p.z);
-    task.pm[i] = p;
-    task.vm[i] = v;
+    step_body(StepParams{task.pm, task.pm, task.vm, dt, damping}, i, g.x, g.y, g.z);
 }
 
 // Work of a ROW_COMP task in VALU instructions per lane (12 + rsq per

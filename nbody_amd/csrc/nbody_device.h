@@ -11,6 +11,8 @@
 // optional Newton step (NEWTON) is off by default.
 #pragma once
 
+#include "nbody_kernels.h"
+
 #include <hip/hip_runtime.h>
 
 namespace nbody {
@@ -138,6 +140,26 @@ __device__ __forceinline__ void interact(float xj, float yj, float zj, float mj,
     else if constexpr (EQ) body_body_chain_eq_v(xj, yj, zj, mj, xi, yi, zi, eps2, ax, ay, az);
     else if constexpr (SGPR_J) body_body_chain_s(xj, yj, zj, mj, xi, yi, zi, eps2, ax, ay, az);
     else body_body_chain_v(xj, yj, zj, mj, xi, yi, zi, eps2, ax, ay, az);
+}
+
+// src/nbody.cu:158-182 integrateOne, in the operation order the reference's
+// -ffast-math CPU build executes it: v = fma(invMass, f*dt, v); v *= damping;
+// x = fma(v, dt, x). Mass (posMass.w) and invMass (velInvMass.w) are kept.
+__device__ __forceinline__ void step_body(const StepParams& st, int i, float fx, float fy, float fz)
+{
+    float4 p = st.pm_in[i];
+    float4 v = st.vm[i];
+    v.x = __builtin_fmaf(v.w, fx * st.dt, v.x);
+    v.y = __builtin_fmaf(v.w, fy * st.dt, v.y);
+    v.z = __builtin_fmaf(v.w, fz * st.dt, v.z);
+    v.x *= st.damping;
+    v.y *= st.damping;
+    v.z *= st.damping;
+    p.x = __builtin_fmaf(v.x, st.dt, p.x);
+    p.y = __builtin_fmaf(v.y, st.dt, p.y);
+    p.z = __builtin_fmaf(v.z, st.dt, p.z);
+    st.pm_out[i] = p;
+    st.vm[i] = v;
 }
 
 // Per-lane state of I i bodies (or their accumulators).

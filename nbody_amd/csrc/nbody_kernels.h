@@ -50,6 +50,15 @@ std::vector<std::pair<int, int>> symmetric_bands(int nb, int B, size_t cap, int 
 // block pairs and one diagonal block).
 void symmetric_share_columns(int nb, int k, int G, int* c0, int* c1);
 
+// One body's update once its force is known (integrateGravitation): reads
+// pm_in and vm, writes pm_out (which may be pm_in) and vm.
+struct StepParams {
+    const float4* pm_in = nullptr;
+    float4* pm_out = nullptr;
+    float4* vm = nullptr;
+    float dt = 0.f, damping = 1.f;
+};
+
 struct ForceParams {
     const float4* pm = nullptr;  // posMass (x, y, z, m) of the whole system: j source and i source
     int n = 0;                   // bodies in the system
@@ -64,7 +73,14 @@ struct ForceParams {
     double* force64 = nullptr;   // symmetric column share: FP64 partial forces, 4 doubles per body (w untouched),
                                  // written instead of force
     float* force = nullptr;      // 4 floats per i body; x, y, z written, w left alone
+    StepParams step;             // with step.vm set, a plan that fuses_step also integrates in its last launch
 };
+
+// Whether a whole-system plan's last launch can integrate the bodies too, and
+// whether it then needs pm_out to be another buffer than pm (its workgroups
+// still read the positions that others have already stepped).
+bool fuses_step(const ForcePlan& plan);
+bool step_needs_buffer(const ForcePlan& plan);
 
 // The shape of the one-launch kernel that ends first for ni of n bodies.
 void tile_shape(size_t n, size_t ni, int* li, int* ipl);

@@ -530,12 +530,15 @@ constexpr int kReduceGroups = 4;
 // body's slots are then folded in band order, the same fixed order on every
 // run. With force64 the last band writes the pair's value in FP64 instead (a
 // share of the columns, whose partial force is summed with the other
-// shares').
+// shares'). STEP also integrates the bodies (the last band): a step's third
+// launch took 4 us.
+template <bool STEP>
 __global__ __launch_bounds__(64 * 3 * kReduceGroups) void k_reduce_band(SlotMap m, int n, int B, int q0, int q1,
                                                                         bool first, bool last,
                                                                         float* __restrict__ state,
                                                                         float* __restrict__ force,
-                                                                        double* __restrict__ force64, int split)
+                                                                        double* __restrict__ force64, int split,
+                                                                        StepParams st)
 {
     constexpr int G = 8;
     __shared__ float sums[kReduceGroups][3][64], errs[kReduceGroups][3][64];
@@ -596,20 +599,26 @@ __global__ __launch_bounds__(64 * 3 * kReduceGroups) void k_reduce_band(SlotMap 
     sums[group][c][lane] = s;
     errs[group][c][lane] = e;
     __syncthreads();
-    if (group != 0 || b >= n) return;
+    if (group == 0 && b < n) {
 #pragma unroll
-    for (int g = 1; g < kReduceGroups; ++g) {
-        float err;
-        s = two_sum(s, sums[g][c][lane], err);
-        e += err + errs[g][c][lane];
+        for (int g = 1; g < kReduceGroups; ++g) {
+            float err;
+            s = two_sum(s, sums[g][c][lane], err);
+            e += err + errs[g][c][lane];
+        }
+        if (last && force64) {
+            force64[4 * (size_t)b + c] = (double)s + (double)e;
+        } else if (last) {
+            force[4 * (size_t)b + c] = s + e;
+        } else {
+            state[(size_t)c * n + b] = s;
+            state[(size_t)(3 + c) * n + b] = e;
+        }
     }
-    if (last && force64) {
-        force64[4 * (size_t)b + c] = (double)s + (double)e;
-    } else if (last) {
-        force[4 * (size_t)b + c] = s + e;
-    } else {
-        state[(size_t)c * n + b] = s;
-        state[(size_t)(3 + c) * n + b] = e;
+    if constexpr (STEP) {
+        if (group == 0) sums[0][c][lane] = s + e;
+        __syncthreads();
+        if (wave == 0 && b < n) step_body(st, b, sums[0][0][lane], sums[0][1][lane], sums[0][2][lane]);
     }
 }
 
@@ -731,28 +740,13 @@ __global__ __launch_bounds__(kBlock) void k_reduce(const float4* __restrict__ hi
     f[2] = a.z + c.z;
 }
 
-// src/nbody.cu:158-182 integrateOne, in the operation order the reference's
-// -ffast-math CPU build executes it: v = fma(invMass, f*dt, v); v *= damping;
-// x = fma(v, dt, x). Mass (posMass.w) and invMass (velInvMass.w) are kept.
-__global__ __launch_bounds__(kBlock) void k_integrate(float4* __restrict__ pm, float4* __restrict__ vim,
-                                                      const float4* __restrict__ f, float dt, float damping, int n)
+// integrateGravitation as a launch of its own.
+__global__ __launch_bounds__(kBlock) void k_integrate(StepParams st, const float4* __restrict__ f, int n)
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    float4 p = pm[i];
-    float4 v = vim[i];
     const float4 g = f[i];
-    v.x = __builtin_fmaf(v.w, g.x * dt, v.x);
-    v.y = __builtin_fmaf(v.w, g.y * dt, v.y);
-    v.z = __builtin_fmaf(v.w, g.z * dt, v.z);
-    v.x *= damping;
-    v.y *= damping;
-    v.z *= damping;
-    p.x = __builtin_fmaf(v.x, dt, p.x);
-    p.y = __builtin_fmaf(v.y, dt, p.y);
-    p.z = __builtin_fmaf(v.z, dt, p.z);
-    pm[i] = p;
-    vim[i] = v;
+    step_body(st, i, g.x, g.y, g.z);
 }
 
 // FP64 direct sum, one i body per lane over one j slice (the j body again
@@ -895,17 +889,24 @@ hipError_t go_family(const ForcePlan& plan, dim3 g, hipStream_t s, const ForcePa
     return hipGetLastError();
 }
 
+template <int LI, int I>
+void go_tile_shape(dim3 g, hipStream_t s, const ForceParams& p)
+{
+    if (p.step.vm) k_force_tile<LI, I, true><<<g, kTileThreads, 0, s>>>(p);
+    else k_force_tile<LI, I, false><<<g, kTileThreads, 0, s>>>(p);
+}
+
 hipError_t go_tile(const ForcePlan& plan, dim3 g, hipStream_t s, const ForceParams& p)
 {
     switch (plan.li * 100 + plan.ipl) {
-    case 401: k_force_tile<4, 1><<<g, kTileThreads, 0, s>>>(p); break;
-    case 402: k_force_tile<4, 2><<<g, kTileThreads, 0, s>>>(p); break;
-    case 403: k_force_tile<4, 3><<<g, kTileThreads, 0, s>>>(p); break;
-    case 802: k_force_tile<8, 2><<<g, kTileThreads, 0, s>>>(p); break;
-    case 803: k_force_tile<8, 3><<<g, kTileThreads, 0, s>>>(p); break;
-    case 804: k_force_tile<8, 4><<<g, kTileThreads, 0, s>>>(p); break;
-    case 805: k_force_tile<8, 5><<<g, kTileThreads, 0, s>>>(p); break;
-    case 806: k_force_tile<8, 6><<<g, kTileThreads, 0, s>>>(p); break;
+    case 401: go_tile_shape<4, 1>(g, s, p); break;
+    case 402: go_tile_shape<4, 2>(g, s, p); break;
+    case 403: go_tile_shape<4, 3>(g, s, p); break;
+    case 802: go_tile_shape<8, 2>(g, s, p); break;
+    case 803: go_tile_shape<8, 3>(g, s, p); break;
+    case 804: go_tile_shape<8, 4>(g, s, p); break;
+    case 805: go_tile_shape<8, 5>(g, s, p); break;
+    case 806: go_tile_shape<8, 6>(g, s, p); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1081,6 +1082,10 @@ void tile_shape(size_t n, size_t ni, int* li, int* ipl)
     }
 }
 
+bool fuses_step(const ForcePlan& plan) { return plan.li > 0 || (plan.variant == VAR_SYMMETRIC && !plan.acc64); }
+
+bool step_needs_buffer(const ForcePlan& plan) { return plan.li > 0; }
+
 bool symmetric_shape_ok(int ipl, int block)
 {
     const int w = block / (64 * ipl);
@@ -1238,8 +1243,9 @@ hipError_t launch_force(const ForcePlan& plan, const ForceParams& p, hipStream_t
                 if (e == hipSuccess && after && last) e = hipEventRecord(after, stream);
                 if (e != hipSuccess) return e;
                 float* state = bands.size() > 1 ? base + most : nullptr;
-                k_reduce_band<<<groups, 64 * 3 * kReduceGroups, 0, stream>>>(sp.slots, p.n, B, q0, q1, first, last,
-                                                                             state, p.force, p.force64, sp.split);
+                auto reduce = p.step.vm && last ? k_reduce_band<true> : k_reduce_band<false>;
+                reduce<<<groups, 64 * 3 * kReduceGroups, 0, stream>>>(sp.slots, p.n, B, q0, q1, first, last, state,
+                                                                      p.force, p.force64, sp.split, p.step);
             }
             e = hipGetLastError();
             if (e != hipSuccess) return e;
@@ -1283,7 +1289,8 @@ hipError_t launch_integrate(float4* posMass, float4* velInvMass, const float4* f
                             hipStream_t stream)
 {
     if (n <= 0) return hipSuccess;
-    k_integrate<<<(n + kBlock - 1) / kBlock, kBlock, 0, stream>>>(posMass, velInvMass, force, dt, damping, n);
+    const StepParams st{posMass, posMass, velInvMass, dt, damping};
+    k_integrate<<<(n + kBlock - 1) / kBlock, kBlock, 0, stream>>>(st, force, n);
     return hipGetLastError();
 }
 

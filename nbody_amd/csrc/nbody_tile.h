@@ -82,8 +82,9 @@ __device__ __forceinline__ void tile_sweep(const vec4* t4, int stride, int steps
 }
 
 // Up to 3 bodies per lane the kernel fits 64 VGPRs, two workgroups (8 waves
-// per SIMD) on a CU.
-template <int LI, int I>
+// per SIMD) on a CU. STEP also integrates the workgroup's bodies, into another
+// position buffer: a step of a small system is then one launch.
+template <int LI, int I, bool STEP>
 __global__ __launch_bounds__(kTileThreads, I <= 3 ? 8 : 4) void k_force_tile(ForceParams p)
 {
     constexpr int S = 64 / LI;             // groups per wave
@@ -174,12 +175,21 @@ __global__ __launch_bounds__(kTileThreads, I <= 3 ? 8 : 4) void k_force_tile(For
     }
     __syncthreads();
     const int m = first + t % TI;
+    float total = 0.f;
     if (t < 3 * TI && m < p.ni) {
         // in FP64: the 16 roundings of this one sum would outweigh those of all the sums before it
         double sum = 0.0;
 #pragma unroll
         for (int w = 0; w < kTileWaves; ++w) sum += red[w * 3 * TI + t];
-        p.force[4 * (size_t)m + t / TI] = (float)sum;
+        total = (float)sum;
+        p.force[4 * (size_t)m + t / TI] = total;
+    }
+    if constexpr (STEP) {
+        float* of = red + kTileWaves * 3 * TI;  // [3][TI], behind the waves' sums
+        static_assert((kTileWaves + 1) * 3 * TI * sizeof(float) <= sizeof(vec4) * 2 * kTileChunk, "fits the tiles");
+        if (t < 3 * TI) of[t] = total;
+        __syncthreads();
+        if (t < TI && m < p.ni) step_body(p.step, m, of[t], of[TI + t], of[2 * TI + t]);
     }
 }
 
