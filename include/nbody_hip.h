@@ -181,9 +181,9 @@ int nbody_hip_energy_fp64(double *out, const float *posMass, const float *velInv
 
 /* The plan the library would use: fills variant, i_per_lane, jslice,
  * compensated, newton for an n-body i range of an N-body system. LDS with
- * i_per_lane and jslice 0 is the one-launch plan of small evaluations (n N up
- * to 10240^2, plain sums, no shape given): it keeps no partial sums, and the
- * same zeros select it again. */
+ * i_per_lane and jslice 0 is the one-launch plan of small evaluations (plain
+ * sums, no shape given): it keeps no partial sums, and the same zeros select
+ * it again. */
 int nbody_hip_plan(size_t N, size_t n, const nbody_hip_options *opt, nbody_hip_options *plan);
 /* Time candidate plans of `variant` (NBODY_HIP_AUTO: the LDS, SGPR and
  * symmetric families) on the given device data, force kernel plus slice

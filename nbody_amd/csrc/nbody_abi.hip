@@ -73,20 +73,38 @@ constexpr int kSymSlotsTarget = 512;
 // against 22.5.
 constexpr size_t kSmallSymN = 5120;
 
-// Interactions up to which the LDS variant runs as one launch over the whole
-// j range (nbody_tile.h), and whole systems do so instead of the symmetric
-// plan. Whole systems, that kernel and the symmetric plan: N = 4096 8.1 and
-// 16.2 us, 8192 22 and 24, 10000 33 and 35, 12288 45 and 43.
-constexpr double kTileMaxWork = 10240.0 * 10240.0;
+// Bodies up to which NBODY_HIP_AUTO evaluates a whole system in one launch
+// over the whole j range (nbody_tile.h) instead of by the symmetric plan. The
+// two: N = 4096 8.1 and 16.2 us, 8192 22 and 24, 10000 33 and 35, 12288 45
+// and 43.
+constexpr size_t kTileMaxN = 10240;
 
-// Whether an n-body i range of N bodies runs so: with plain sums, no Newton
-// step and nothing of the shape fixed.
-bool tile_plan(size_t N, size_t n, const nbody_hip_options* opt)
+// Whether the options leave an i range free to run so: plain sums, no Newton
+// step, nothing of the shape fixed.
+bool tile_allowed(size_t N, size_t n, const nbody_hip_options* opt)
 {
     const int comp_opt = opt ? opt->compensated : -1;
     const bool comp = comp_opt < 0 ? N > 65536 : comp_opt > 0;
     const bool shape_given = opt && (opt->i_per_lane > 0 || opt->jslice > 0 || opt->waves_per_simd > 0);
-    return n > 0 && !comp && !shape_given && !(opt && opt->newton > 0) && (double)n * (double)N <= kTileMaxWork;
+    return n > 0 && !comp && !shape_given && !(opt && opt->newton > 0);
+}
+
+// The LDS variant's own shape. Two i bodies per lane halve the LDS reads, but
+// also the workgroups, so only past kLdsWideWork interactions; slices as
+// short as give each CU about 20 workgroups (the launch ends unevenly with
+// fewer), 256 bodies at least, and longer than 1024 only where even those give
+// it 80 (the slice sum reads 16 or 32 bytes per body and slice). Microseconds
+// for one GPU's eighth of N = 98304 with slices of 256, 512, 1024, 2048, two
+// bodies per lane: 308, 299, 305, 350, and with one: 332, 324, 326, 344; its
+// quarter of 150751: 1536, 1492, 1472, 1528; half of 33588 153, 164, 188, 240.
+constexpr double kLdsWideWork = 5.0e8;
+
+void lds_shape(size_t N, size_t n, int cus, int* ipl, int* jslice)
+{
+    *ipl = (double)n * (double)N >= kLdsWideWork ? 2 : 1;
+    const double per_cu = std::ceil((double)n / (256.0 * *ipl)) * (double)N / std::max(cus, 1);
+    const double len = per_cu / 20.0 <= 1024.0 ? per_cu / 20.0 : std::max(1024.0, per_cu / 80.0);
+    *jslice = std::max(1, (int)(len / 256.0 + 0.5)) * 256;
 }
 
 // Default decomposition: enough blocks for ~48 waves per SIMD (the dispatcher
@@ -139,10 +157,20 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
         p.comp = false;
         return p;
     }
-    if (variant == VAR_LDS && tile_plan(N, n, opt)) {
-        tile_shape(N, n, &p.li, &p.ipl);
-        p.jslice = (int)N;
-        p.nslices = 1;
+    if (variant == VAR_LDS && !p.acc64 && !(opt && (opt->i_per_lane > 0 || opt->jslice > 0))) {
+        lds_shape(N, n, cus, &p.ipl, &p.jslice);
+        int li, ipl;
+        // the sliced plan's time: a wave's chain through its slice at the least, and about 16 us of
+        // launches and slice sum (one GPU's share, half of N: N = 16384 52 and, in one launch, 41 us,
+        // 20000 71 and 63, 33588 153 and 188)
+        const double sliced = std::max(0.26e-6 * (double)n * (double)N, 0.044 * p.jslice * p.ipl) + 16.0;
+        if (tile_allowed(N, n, opt) && tile_shape(N, n, &li, &ipl) < sliced) {
+            p.li = li;
+            p.ipl = ipl;
+            p.jslice = (int)N;
+        }
+        p.jslice = std::max(1, std::min(p.jslice, (int)N));
+        p.nslices = (int)((N + p.jslice - 1) / p.jslice);
         return p;
     }
     p.ipl = (opt && opt->i_per_lane > 0) ? opt->i_per_lane : 1;
@@ -169,7 +197,7 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
 }
 
 // The untuned choice for NBODY_HIP_AUTO: the symmetric kernel for whole
-// systems past kTileMaxWork (half the pairs, 14-16 VALU + 1 rsq per pair);
+// systems past kTileMaxN (half the pairs, 14-16 VALU + 1 rsq per pair);
 // otherwise the LDS broadcast, whose VALU operands all sit in VGPRs (gfx950
 // issues those faster than ops reading an SGPR), in one launch where small.
 // Largest block count of a symmetric plan (the pair index must fit an int).
@@ -178,7 +206,7 @@ constexpr int kMaxSymBlocks = 16384;
 int auto_variant(size_t N, size_t n, const nbody_hip_options* opt)
 {
     if (n != N || N < 1024) return VAR_LDS;
-    if (tile_plan(N, n, opt) && !(opt && opt->slot_bytes > 0)) return VAR_LDS;
+    if (N <= kTileMaxN && tile_allowed(N, n, opt) && !(opt && opt->slot_bytes > 0)) return VAR_LDS;
     const ForcePlan p = default_plan(VAR_SYMMETRIC, N, N, 1, nullptr);
     return p.nslices <= kMaxSymBlocks ? VAR_SYMMETRIC : VAR_LDS;
 }

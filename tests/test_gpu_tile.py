@@ -1,5 +1,5 @@
 """The one-launch plan of small evaluations (whole systems up to 10240 bodies,
-i ranges of n N up to 10240^2): sizes at the edges of its workgroups, of a
+small i ranges): sizes at the edges of its workgroups, of a
 step of its lane groups and of its 2048-body chunks, one for each of its
 shapes, against the FP64 oracle; i ranges; masses that change in the middle
 of a chunk and after a whole chunk of one mass.
@@ -55,12 +55,13 @@ def test_sizes_and_masses(oracle, n, masses):
         assert mx <= TOL_MAX and rms <= TOL_RMS, (n, masses, mx, rms)
 
 
-@pytest.mark.parametrize("n,base,count", [(5000, 0, 1), (5000, 4999, 1), (5000, 123, 1777), (30000, 7, 3000),
-                                          (65536, 60000, 100), (16384, 4096, 6400)])
+@pytest.mark.parametrize("n,base,count", [(5000, 0, 1), (5000, 4999, 1), (5000, 123, 1777), (16384, 4096, 6400),
+                                          (30000, 7, 3000), (65536, 60000, 100), (65536, 1, 20000)])
 def test_i_ranges(oracle, n, base, count):
-    """Ranges against the oracle, and with a mass scaled by a power of two
-    exactly (one mass and unequal masses)."""
-    assert plan(n, count).jslice == 0
+    """Ranges, in one launch or (the last two) in slices, against the oracle,
+    and with a mass scaled by a power of two exactly (one mass and unequal
+    masses)."""
+    assert (plan(n, count).jslice == 0) == (n < 60000)
     for one in (False, True):
         pm, _ = ics.random_unit_bodies(n, seed=42)
         if one:
@@ -83,7 +84,7 @@ def test_other_options_keep_their_plans():
     assert plan(10241, 10241).variant == _native.SYMMETRIC
     assert plan(4096, 4096, variant=_native.LDS, i_per_lane=1).jslice > 0
     assert plan(4096, 4096, variant=_native.LDS, compensated=1).jslice > 0
-    assert plan(98304, 12288).jslice > 0
+    assert plan(98304, 12288).jslice > 0 and plan(60000, 15000).jslice > 0
 
 
 def test_empty_range_writes_nothing():
@@ -91,3 +92,19 @@ def test_empty_range_writes_nothing():
     d, f = dev(pm), force_buffer(1)
     rc = _native.lib().nbody_hip_force(ptr(f), ptr(d), EPS2, 100, 50, 0, None, None)
     assert rc == 0 and np.all(np.isnan(host(f)[:, :3]))
+
+
+@pytest.mark.parametrize("slices", [1, 2, 3, 4, 5, 7, 16, 17, 33])
+@pytest.mark.parametrize("comp", [0, 1])
+def test_slice_sum(oracle, slices, comp):
+    """The sum over j slices, a quarter of them per wave, at slice counts below,
+    at and past the waves and the loads in flight, on a body count that is no
+    multiple of 64."""
+    n = 256 * slices
+    pm, _ = ics.random_unit_bodies(n, seed=44)
+    f = run_force(dev(pm), EPS2, base=1, count=min(n - 1, 777), variant=_native.LDS, i_per_lane=1, jslice=256,
+                  compensated=comp)
+    f64 = oracle.fp64_forces(pm, EPS2, np.arange(1, 1 + f.shape[0]))
+    mx, rms = force_errors(f, f64)
+    assert mx <= TOL_MAX and rms <= TOL_RMS, (slices, comp, mx, rms)
+    assert np.all(f[:, 3] == -7.0)
