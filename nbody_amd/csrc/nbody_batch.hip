@@ -1,9 +1,10 @@
 // Batched force and integrate kernels for many independent systems: a
-// persistent grid of one-wave workgroups pulls ForceTasks (block pairs,
+// persistent grid of four-wave workgroups pulls ForceTasks (block pairs,
 // diagonal blocks, compensated rows) from a device work queue, then one
 // launch adds every body's slots and integrates it. Task lists are built on
 // the host, most expensive first. With FP64 accumulation the same scheme
-// runs the FP64 symmetric plan's pieces (k_force_batch64).
+// runs the FP64 symmetric plan's pieces in one-wave workgroups
+// (k_force_batch64).
 #include "nbody_acc64.h"
 #include "nbody_device.h"
 #include "nbody_kernels.h"
@@ -18,63 +19,73 @@ namespace {
 
 constexpr int kWave = 64;
 constexpr int kChunk = 128;                  // j bodies between TwoSum folds of a ROW_COMP task
-constexpr int kPairA = kBatchBlock / kWave;  // bodies per lane of a PAIR task
-constexpr int kBodyTaskBodies = 256;         // bodies per BodyTask (one thread each, per component)
+constexpr int kBodyTaskBodies = 256;         // bodies per BodyTask
+constexpr int kBodyTaskParts = kBodyTaskBodies / kWave;  // workgroups per BodyTask
 constexpr int kPairA64 = kBatchBlock64 / kWave;  // bodies per lane of a PAIR64 task
 
-static_assert(kBatchBlock % kWave == 0 && kPairA == 8, "PAIR tasks are compiled for 8 bodies per lane");
+static_assert(kBatchBlock == 512, "PAIR and DIAG tasks are sym_deal_task's");
 static_assert(kBatchBlock64 % kWave == 0 && kPairA64 == 4, "PAIR64 tasks are compiled for 4 bodies per lane");
 
-__global__ __launch_bounds__(kWave) void k_force_batch(const ForceTask* __restrict__ tasks, int ntasks,
-                                                       unsigned* __restrict__ counter)
+// A ROW_COMP task: 64 bodies per wave against task.len bodies, TwoSum-folded chunks.
+__device__ __forceinline__ void row_comp(const ForceTask& task)
 {
-    __shared__ float jacc[3][kBatchBlock];
-    // Workgroup b's first task is task b; later tickets come from the
-    // counter, offset by the grid. All workgroups start together, and their
-    // first tickets from one atomic counter would queue up behind each other
-    // (the launch measured 3 % slower that way).
-    for (bool first = true;; first = false) {
-        int t = (int)blockIdx.x;
-        if (!first && threadIdx.x == 0) t = (int)atomicAdd(counter, 1u) + (int)gridDim.x;
-        // one wave per workgroup: lane 0's ticket is the wave's task, kept scalar
-        t = __builtin_amdgcn_readfirstlane(t);
-        if (t >= ntasks) return;
+    const int i = task.a + (int)threadIdx.x;
+    const float4 q = task.pm[min(i, task.n - 1)];
+    Lanes<1> me, hi, lo;
+    me.x[0] = q.x;
+    me.y[0] = q.y;
+    me.z[0] = q.z;
+    zero<1>(hi);
+    zero<1>(lo);
+    const float4* src = task.pm + task.b;
+    for (int c = 0; c < task.len; c += kChunk) {
+        Lanes<1> part1;
+        zero<1>(part1);
+        sweep_const<1, false>(src + c, min(kChunk, task.len - c), task.eps2, me, part1);
+        fold<1>(hi, lo, part1);
+    }
+    hi.x[0] += lo.x[0];
+    hi.y[0] += lo.y[0];
+    hi.z[0] += lo.z[0];
+    if (i < task.n) {
+        const size_t plane = (size_t)task.nb * task.npad;
+        const size_t o = (size_t)task.slot * task.npad + i;
+        task.part[o] = hi.x[0];
+        task.part[plane + o] = hi.y[0];
+        task.part[2 * plane + o] = hi.z[0];
+    }
+}
+
+// Block pairs and diagonal blocks as k_force_sym_deal's (one task per pair),
+// with the steps' reactions summed apart: every block general or on one mass
+// runs at the top rate of the pair chain, with the smaller rounding error.
+// Workgroup b's first task is task b, later ones come from the counter,
+// offset by the grid; the number of a workgroup's next task is fetched while
+// it runs one. Bound by the pair chain's VALU issue. Four waves to a task
+// instead of one: a small batch's step is as long as its longest task. 8
+// systems of 64..500 bodies took 77 us a step and take 27, 32 of 256..4000
+// 233 and 53, 512 of 256..16384 (with the slot sums apart, below) 2590 and
+// 2452; one wave per task 2428 on the last, one workgroup per task 2475, the
+// number fetched after the task 2470.
+__global__ __launch_bounds__(kWave * kDealWaves, 6) void k_force_batch(const ForceTask* __restrict__ tasks, int ntasks,
+                                                                       unsigned* __restrict__ counter)
+{
+    __shared__ float part[kDealWaves][3][kBatchBlock];
+    __shared__ int ticket;
+    for (int t = blockIdx.x; t < ntasks;) {
+        // the next task's number is on its way while this one runs
+        int next = 0;
+        if (threadIdx.x == 0) next = (int)atomicAdd(counter, 1u) + (int)gridDim.x;
         const ForceTask task = tasks[t];
-        if (task.kind == TASK_PAIR) {
-            sym_pair<kPairA, 1, false, REGS_APART>(task.pm, task.n, task.eps2, SlotMap::whole(task.part, task.nb, task.npad),
-                                             task.a, task.b, jacc);
-            continue;
-        }
-        if (task.kind == TASK_DIAG) {
-            sym_diag_block(task.pm, task.n, task.npad, task.eps2, task.part, task.a);
-            continue;
-        }
-        // TASK_ROW_COMP: 64 bodies against task.len bodies, TwoSum-folded chunks
-        const int i = task.a + (int)threadIdx.x;
-        const float4 q = task.pm[min(i, task.n - 1)];
-        Lanes<1> me, hi, lo;
-        me.x[0] = q.x;
-        me.y[0] = q.y;
-        me.z[0] = q.z;
-        zero<1>(hi);
-        zero<1>(lo);
-        const float4* src = task.pm + task.b;
-        for (int c = 0; c < task.len; c += kChunk) {
-            Lanes<1> part;
-            zero<1>(part);
-            sweep_const<1, false>(src + c, min(kChunk, task.len - c), task.eps2, me, part);
-            fold<1>(hi, lo, part);
-        }
-        hi.x[0] += lo.x[0];
-        hi.y[0] += lo.y[0];
-        hi.z[0] += lo.z[0];
-        if (i < task.n) {
-            const size_t plane = (size_t)task.nb * task.npad;
-            const size_t o = (size_t)task.slot * task.npad + i;
-            task.part[o] = hi.x[0];
-            task.part[plane + o] = hi.y[0];
-            task.part[2 * plane + o] = hi.z[0];
-        }
+        if (task.kind == TASK_ROW_COMP) row_comp(task);
+        else
+            sym_deal_task<false, REGS_APART, REGS_APART>(task.pm, task.n, task.eps2,
+                                                         SlotMap::whole(task.part, task.nb, task.npad), task.a, task.b,
+                                                         0, 1, 0, part);
+        if (threadIdx.x == 0) ticket = next;
+        __syncthreads();  // (`part` is free after it as well)
+        t = __builtin_amdgcn_readfirstlane(ticket);
+        __syncthreads();
     }
 }
 
@@ -114,26 +125,35 @@ __global__ __launch_bounds__(kWave) void k_force_batch64(const ForceTask* __rest
     }
 }
 
-// 3 x kBodyTaskBodies threads per task: the threads of component c add that
-// component of the task's bodies over their slots (eight slots in flight,
-// each slot row read as one contiguous run), then the first kBodyTaskBodies
-// threads integrate. The slot sum is k_reduce_band's (slot order, TwoSum,
-// rounded once) for FP32 slots and k_reduce_band64's (slot order, FP64,
-// rounded once) for FP64 slots, both in nbody_kernels.hip.
+// Three waves per 64 bodies of a task: wave c adds component c over the
+// bodies' slots (eight slots in flight, each slot row read as one contiguous
+// run), then wave 0 integrates. The slot sum is k_reduce_band's (slot order,
+// TwoSum, rounded once) for FP32 slots and k_reduce_band64's (slot order,
+// FP64, rounded once) for FP64 slots, both in nbody_kernels.hip.
+// Bound by HBM. The workgroups are small on purpose: with one wave per SIMD
+// of at most 32 VGPRs, they fit beside the other group's force launch, whose
+// six waves leave 32 of a SIMD's 512 registers free, so the sum of one group
+// runs under the other's force, at a higher wave priority (512 systems of
+// 256..16384 bodies: 2590 us a step with 12-wave workgroups, 2428 so, both
+// over one-wave force tasks).
 template <class T>
-__global__ __launch_bounds__(3 * kBodyTaskBodies) void k_reduce_integrate_batch(const BodyTask* __restrict__ tasks,
-                                                                                float dt, float damping,
-                                                                                unsigned* __restrict__ counter)
+__global__ __launch_bounds__(3 * kWave) void k_reduce_integrate_batch(const BodyTask* __restrict__ tasks, float dt,
+                                                                      float damping, unsigned* __restrict__ counter)
 {
     constexpr int G = 8;
-    __shared__ float sum[3][kBodyTaskBodies];
+    __shared__ float sum[3][kWave];
+    __builtin_amdgcn_s_setprio(3);
     if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0u;
-    const BodyTask task = tasks[blockIdx.x];
-    const int lane = threadIdx.x % kBodyTaskBodies;
-    const int c = threadIdx.x / kBodyTaskBodies;  // wave-uniform component
+    const BodyTask task = tasks[blockIdx.x / kBodyTaskParts];
+    const int i0 = (int)(blockIdx.x % kBodyTaskParts) * kWave;
+    if (i0 >= task.ni) return;  // the rest of a ragged task
+    const int lane = threadIdx.x & (kWave - 1);
+    const int c = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const bool body = i0 + lane < task.ni;
+    const int i = task.i0 + i0 + lane;
     if constexpr (std::is_same<T, double>::value) {
-        if (lane < task.ni) {
-            const double* src = task.part64 + (size_t)c * task.nb * task.npad + task.i0 + lane;
+        if (body) {
+            const double* src = task.part64 + (size_t)c * task.nb * task.npad + i;
             double s = 0.0;
             int k = 0;
             for (; k + G <= task.nb; k += G) {
@@ -146,8 +166,8 @@ __global__ __launch_bounds__(3 * kBodyTaskBodies) void k_reduce_integrate_batch(
             for (; k < task.nb; ++k) s += src[(size_t)k * task.npad];
             sum[c][lane] = (float)s;
         }
-    } else if (lane < task.ni) {
-        const float* src = task.part + (size_t)c * task.nb * task.npad + task.i0 + lane;
+    } else if (body) {
+        const float* src = task.part + (size_t)c * task.nb * task.npad + i;
         float s = 0.f, e = 0.f;
         int k = 0;
         for (; k + G <= task.nb; k += G) {
@@ -169,8 +189,7 @@ __global__ __launch_bounds__(3 * kBodyTaskBodies) void k_reduce_integrate_batch(
         sum[c][lane] = s + e;
     }
     __syncthreads();
-    if (c != 0 || lane >= task.ni) return;
-    const int i = task.i0 + lane;
+    if (c != 0 || !body) return;
     float4 g = task.force[i];
     g.x = sum[0][lane];
     g.y = sum[1][lane];
@@ -187,7 +206,7 @@ double row_cost(const ForceTask& t) { return (double)t.len * (t.kind == TASK_ROW
 bool is_row(const ForceTask& t) { return t.kind == TASK_ROW_COMP || t.kind == TASK_ROW64; }
 
 // Cost of a block task in halves of a 64 x 64 tile block: a pair meets the
-// tiles of block Q that hold bodies (one-wave pairs skip the padding tiles)
+// tiles of block Q that hold bodies (padding tiles are skipped)
 // with all 8 tiles of block P, 16 per Q tile, 128 for a full pair; a
 // diagonal block of T tiles takes each pair once, T^2, 64 when full. A
 // PAIR64 task meets block P's 4 tiles, 8 per Q tile; a DIAG64 piece (one
@@ -261,7 +280,7 @@ void append_force_tasks(std::vector<ForceTask>& out, const float4* pm, void* par
         t.b = 0;
         t.len = (int)n;
         t.slot = 0;
-        for (size_t i = 0; i < n; i += kWave) {
+        for (size_t i = 0; i < n; i += acc64 ? kWave : kWave * kDealWaves) {
             t.a = (int)i;
             out.push_back(t);
         }
@@ -275,9 +294,8 @@ void append_force_tasks(std::vector<ForceTask>& out, const float4* pm, void* par
             out.push_back(t);
         }
     t.kind = acc64 ? TASK_DIAG64 : TASK_DIAG;
-    t.b = 0;
     for (int p = 0; p < nb; ++p) {
-        t.a = p;
+        t.a = t.b = p;
         t.len = (int)std::min<size_t>(B, n - (size_t)p * B);
         t.slot = p;
         if (!acc64) {
@@ -289,7 +307,6 @@ void append_force_tasks(std::vector<ForceTask>& out, const float4* pm, void* par
             t.b = k;
             out.push_back(t);
         }
-        t.b = 0;
     }
 }
 
@@ -375,7 +392,7 @@ int batch_force_blocks_per_cu(bool acc64)
         int blocks = 0;
         const hipError_t e =
             acc64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_force_batch64, kWave, 0)
-                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_force_batch, kWave, 0);
+                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_force_batch, kWave * kDealWaves, 0);
         if (e != hipSuccess || blocks < 1) blocks = 16;
         c = blocks;
     }
@@ -388,7 +405,7 @@ hipError_t launch_force_batch(const ForceTask* tasks, int ntasks, unsigned* coun
     if (ntasks <= 0) return hipSuccess;
     blocks = blocks < ntasks ? blocks : ntasks;
     if (acc64) k_force_batch64<<<blocks, kWave, 0, stream>>>(tasks, ntasks, counter);
-    else k_force_batch<<<blocks, kWave, 0, stream>>>(tasks, ntasks, counter);
+    else k_force_batch<<<blocks, kWave * kDealWaves, 0, stream>>>(tasks, ntasks, counter);
     return hipGetLastError();
 }
 
@@ -396,10 +413,8 @@ hipError_t launch_reduce_integrate_batch(const BodyTask* tasks, int ntasks, floa
                                          unsigned* counter, hipStream_t stream, bool acc64)
 {
     if (ntasks <= 0) return hipSuccess;
-    if (acc64)
-        k_reduce_integrate_batch<double><<<ntasks, 3 * kBodyTaskBodies, 0, stream>>>(tasks, dt, damping, counter);
-    else
-        k_reduce_integrate_batch<float><<<ntasks, 3 * kBodyTaskBodies, 0, stream>>>(tasks, dt, damping, counter);
+    auto reduce = acc64 ? k_reduce_integrate_batch<double> : k_reduce_integrate_batch<float>;
+    reduce<<<ntasks * kBodyTaskParts, 3 * kWave, 0, stream>>>(tasks, dt, damping, counter);
     return hipGetLastError();
 }
 

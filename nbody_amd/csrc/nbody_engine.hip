@@ -147,9 +147,8 @@ struct nbody_hip_ensemble {
     char* part = nullptr;          // every system's slot planes, back to back
     bool acc64 = false;            // FP64 accumulation (compensated = 2)
     // The systems in kGroups groups of about equal work, each with its own
-    // task lists and work-queue counter; a batched step forks, runs each
-    // group's force and slot-sum launches on its own stream, and joins, so
-    // one group's launches fill another's drain (two groups measured best:
+    // task lists and work-queue counter, and its launches on its own stream,
+    // so one group's launches fill another's drain (two groups measured best:
     // four were no faster than one, eight slower).
     static constexpr int kGroups = 2;
     int ngroups = 1;
@@ -192,17 +191,20 @@ struct nbody_hip_ensemble {
         return OK;
     }
 
-    int queue_batched()
+    // `steps` batched steps of every system. The groups are independent, so
+    // each queues its own steps on its own stream and they meet only at the
+    // end: a group's slot sum runs under another's force launch.
+    int queue_batched(int steps)
     {
-        if (ngroups == 1) return queue_group(0, stream);
-        HIP_TRY(hipEventRecord(fork, stream));
+        if (ngroups > 1) HIP_TRY(hipEventRecord(fork, stream));
         for (int g = 1; g < ngroups; ++g) HIP_TRY(hipStreamWaitEvent(side[g], fork, 0));
-        if (int r = queue_group(0, stream)) return r;
+        for (int k = 0; k < steps; ++k)
+            for (int g = 0; g < ngroups; ++g)
+                if (int r = queue_group(g, g == 0 ? stream : side[g])) return r;
         for (int g = 1; g < ngroups; ++g) {
-            if (int r = queue_group(g, side[g])) return r;
             HIP_TRY(hipEventRecord(join[g], side[g]));
+            HIP_TRY(hipStreamWaitEvent(stream, join[g], 0));
         }
-        for (int g = 1; g < ngroups; ++g) HIP_TRY(hipStreamWaitEvent(stream, join[g], 0));
         return OK;
     }
 
@@ -467,8 +469,7 @@ int nbody_hip_ensemble_run(nbody_hip_ensemble* e, int steps, int mode, float* ms
     if (int r = device_state(&d)) return r;
     if (mode == NBODY_HIP_BATCHED_GRAPH && !e->exec && steps >= kGraphSteps) {
         HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-        int r = OK;
-        for (int k = 0; k < kGraphSteps && r == OK; ++k) r = e->queue_batched();
+        const int r = e->queue_batched(kGraphSteps);
         hipGraph_t g = nullptr;
         const hipError_t err = hipStreamEndCapture(e->stream, &g);
         if (r) {
@@ -481,13 +482,16 @@ int nbody_hip_ensemble_run(nbody_hip_ensemble* e, int steps, int mode, float* ms
     }
     HIP_TRY(hipEventRecord(e->timing.a, e->stream));
     for (int k = 0; k < steps;) {
-        if (mode == NBODY_HIP_BATCHED_GRAPH && e->exec && steps - k >= kGraphSteps) {
+        if (mode == NBODY_HIP_PER_SYSTEM) {
+            if (int r = e->queue_per_system(*d)) return r;
+            ++k;
+        } else if (mode == NBODY_HIP_BATCHED_GRAPH && e->exec && steps - k >= kGraphSteps) {
             HIP_TRY(hipGraphLaunch(e->exec, e->stream));
             k += kGraphSteps;
-            continue;
+        } else {
+            if (int r = e->queue_batched(steps - k)) return r;
+            k = steps;
         }
-        if (int r = mode == NBODY_HIP_PER_SYSTEM ? e->queue_per_system(*d) : e->queue_batched()) return r;
-        ++k;
     }
     return timed_wait(e->stream, e->timing, ms);
 }

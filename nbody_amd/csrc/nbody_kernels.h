@@ -123,14 +123,14 @@ namespace nbody {
 
 // ---- batches of independent systems (ensembles, served requests) ----------
 //
-// One persistent launch computes the forces of many systems: one-wave
-// workgroups take ForceTasks from a device work queue (an atomic counter).
+// One persistent launch computes the forces of many systems: four-wave
+// workgroups (one-wave ones with FP64 accumulation) take ForceTasks from a device work queue (an atomic counter).
 // A system of n <= kBatchPairMaxN bodies is cut into blocks of kBatchBlock
 // and runs as the symmetric plan does (nbody_sym.h): one PAIR task per block
 // pair P < Q and one DIAG task per diagonal block, each writing its own slot
 // of the system's partial planes part[3][nb][npad]. A
 // larger system (its slot planes would grow as n^2/kBatchBlock) runs as
-// ROW_COMP tasks: 64 bodies against all n with TwoSum-folded chunks, into a
+// ROW_COMP tasks: 256 bodies against all n with TwoSum-folded chunks, into a
 // single slot. A second launch adds each body's slots in slot order (TwoSum)
 // and integrates it. A body's result therefore depends only on its own
 // system, never on what else is in the batch or on scheduling.
@@ -144,7 +144,7 @@ namespace nbody {
 // system of 1024 .. kBatchPairMaxN64 bodies then gets exactly the forces of
 // the single-system FP64 symmetric plan (4 bodies per lane, blocks of 256).
 
-constexpr int kBatchBlock = 512;                     // 8 bodies per lane, one wave
+constexpr int kBatchBlock = 512;                     // 8 bodies per lane, four waves share block Q
 constexpr size_t kBatchPairMaxN = size_t(1) << 18;   // largest system run as block pairs
 constexpr int kBatchBlock64 = 256;                   // FP64 accumulation: 4 bodies per lane, one wave
 constexpr size_t kBatchPairMaxN64 = size_t(1) << 17; // FP64 accumulation: largest system run as block pairs
@@ -167,8 +167,8 @@ struct ForceTask {
     int npad;          // length of one slot row
     float eps2;
     int kind;          // BatchTaskKind
-    int a;             // PAIR, DIAG: block P; ROW_COMP, ROW64: first i body (64 of them)
-    int b;             // PAIR: block Q; DIAG64: piece (0..3); ROW_COMP, ROW64: first j body
+    int a;             // PAIR, DIAG: block P; ROW_COMP, ROW64: first i body (256, or 64, of them)
+    int b;             // PAIR: block Q; DIAG: block P; DIAG64: piece (0..3); ROW_COMP, ROW64: first j body
     int len;           // DIAG, DIAG64: bodies in the block; ROW_COMP, ROW64: number of j bodies
     int slot;          // slot written (DIAG, DIAG64: P; ROW_COMP, ROW64: 0)
     int reserved;
@@ -214,7 +214,7 @@ struct ForceTaskBands {
 };
 void build_force_task_bands(ForceTaskBands& out, const float4* pm, void* part, size_t n, float eps2, bool acc64);
 void concat_force_task_bands(std::vector<ForceTask>& out, const std::vector<const ForceTaskBands*>& systems);
-// Resident one-wave force workgroups per CU (the persistent grid is this
+// Resident force workgroups per CU (the persistent grid is this
 // times the CU count) of the FP32 or the FP64-accumulation force kernel.
 int batch_force_blocks_per_cu(bool acc64);
 

@@ -398,8 +398,6 @@ __global__ __launch_bounds__(64 * W) void k_force_sym(SymParams p)
     }
 }
 
-constexpr int kDealWaves = 4;
-
 // The symmetric plan with 8 bodies per lane and blocks of 512: a workgroup of
 // 4 waves, one per SIMD, each holding the same 512 bodies of block P, deals
 // the 64-body tiles of block Q among them. A tile's reactions go from the
@@ -424,15 +422,10 @@ constexpr int kDealWaves = 4;
 template <bool NEWTON>
 __global__ __launch_bounds__(64 * kDealWaves, 6) void k_force_sym_deal(SymParams p)
 {
-    constexpr int W = kDealWaves, B = 512, T = B / 64;
-    __shared__ float part[W][3][B];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int halves = p.split == 4 ? 2 : 1;  // a tile's 64 steps on one wave, or 32 on each of two
-    const int half = halves == 2 ? wave & 1 : 0;
-    const bool diag = (int)blockIdx.x < p.diag_tasks;
+    __shared__ float part[kDealWaves][3][512];
+    const int halves = p.split == 4 ? 2 : 1;
     int P, Q, h;  // task h of the block pair, or h of the diagonal block
-    if (diag) {
+    if ((int)blockIdx.x < p.diag_tasks) {
         P = Q = p.q0 + blockIdx.x / halves;
         h = blockIdx.x % halves;
     } else {
@@ -440,78 +433,7 @@ __global__ __launch_bounds__(64 * kDealWaves, 6) void k_force_sym_deal(SymParams
         h = t % p.split;
         upper_pair(p.q0 * (p.q0 - 1) / 2 + t / p.split, P, Q);
     }
-    const float m0 = p.pm[P * B].w;
-    Lanes<8> me, acc;
-    float mi[8];
-    bool same = true;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        const int i = P * B + u * 64 + lane;
-        const float4 q = i < p.n ? p.pm[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-        me.x[u] = q.x;
-        me.y[u] = q.y;
-        me.z[u] = q.z;
-        mi[u] = q.w;
-        same &= (i < p.n) & (q.w == m0);
-    }
-    zero<8>(acc);
-    float scale = 1.0f;
-    if (diag) {
-        const bool eq = !NEWTON && __builtin_amdgcn_ballot_w64(!same) == 0;
-        sym_deal_diag<NEWTON>(p.pm, p.n, p.eps2, P, wave, h, halves, eq, me, mi, acc);
-        if (eq) scale = m0;
-    } else {
-        // tiles t0, t0 + W, ... < t1 of block Q
-        const int t0 = h * (T / p.split) + (halves == 2 ? wave >> 1 : wave), t1 = p.split == 1 ? T : t0 + 1;
-        for (int tile = t0; tile < t1; tile += W) {
-            const int j = Q * B + tile * 64 + lane;
-            same &= (j < p.n) & (p.pm[min(j, p.n - 1)].w == m0);
-        }
-        const bool eq = __builtin_amdgcn_ballot_w64(!same) == 0;
-        if (eq) scale = m0;
-        float* jdst = p.slots.j_side(P, Q, B);
-        const size_t plane = p.slots.bplane;
-        const int out = t0 * 64;
-        float r[3];
-        if (eq)
-            sym_deal_tiles<NEWTON, true>(p.pm, p.n, p.eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst, plane,
-                                         m0, r);
-        else
-            sym_deal_tiles<NEWTON, false>(p.pm, p.n, p.eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst, plane,
-                                          1.0f, r);
-        if (halves == 2) {
-            // the first half's reactions are half a turn from home; the second wave adds both in order
-            if (half == 0) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) part[wave][c][lane ^ 32] = r[c];
-            }
-            __syncthreads();
-            if (half == 1 && Q * B + out < p.n) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) jdst[c * plane + out + lane] = part[wave - 1][c][lane] + r[c];
-            }
-            __syncthreads();
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        part[wave][0][u * 64 + lane] = acc.x[u] * scale;
-        part[wave][1][u * 64 + lane] = acc.y[u] * scale;
-        part[wave][2][u * 64 + lane] = acc.z[u] * scale;
-    }
-    __syncthreads();
-    float* __restrict__ idst = (diag ? p.slots.j_side(P, P, B) : p.slots.i_side(P, Q, B)) + h * p.more;
-    const size_t iplane = diag ? p.slots.bplane : p.slots.i_plane(P);
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int k = 0; k < B; k += 64 * W) {
-            const int o = k + threadIdx.x;
-            float sum = part[0][c][o];
-#pragma unroll
-            for (int w = 1; w < W; ++w) sum += part[w][c][o];
-            idst[c * iplane + o] = sum;
-        }
+    sym_deal_task<NEWTON, REGS_PINNED, REGS_FREE>(p.pm, p.n, p.eps2, p.slots, P, Q, h, p.split, p.more, part);
 }
 
 constexpr int kReduceGroups = 4;

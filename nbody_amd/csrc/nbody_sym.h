@@ -16,9 +16,8 @@
 // with one barrier per phase: no atomics anywhere.
 //
 // The diagonal of block P (its bodies against each other) is A one-sided
-// pieces of 64*W bodies each (sym_diag_piece), or, in blocks of 512, takes
-// each pair of the block once: on one wave in the batched kernel
-// (sym_diag_block), on four in k_force_sym_deal (sym_deal_diag).
+// pieces of 64*W bodies each (sym_diag_piece), or, in blocks of 512 on four
+// waves, takes each pair of the block once (sym_deal_diag).
 //
 // Every body then has exactly one partial per block slot: slot Q for the i
 // side of (P, Q), slot P for its j side, slot P for the diagonal. The partials
@@ -731,10 +730,11 @@ __device__ __forceinline__ void sym_pair(const float4* __restrict__ pm, int n, f
     }
 }
 
-// Block P against itself, each pair once, on one wave with 8 bodies per lane
-// (blocks of 512). Tile t of the block rotates past the lanes as in a block
-// pair and meets the i sub-blocks u < t in full, both directions. Against its
-// own sub-block (u = t) it takes steps 1..32 only, step 32 on lanes 32..63:
+// Tile t of block P against the block, on one wave with 8 bodies per lane
+// (blocks of 512); the block's 8 tiles together take each of its pairs once.
+// The tile rotates past the lanes as in a block pair and meets the i
+// sub-blocks u < t in full, both directions. Against its own sub-block
+// (u = t) it takes steps 1..32 only, step 32 on lanes 32..63:
 // a pair of lanes at rotation distance d is met at step d and at step 64 - d,
 // so this covers every pair of the 64 exactly once. When the tile's
 // reactions come home after 64 steps they sit in the lanes that hold the
@@ -771,50 +771,7 @@ __device__ __forceinline__ void sym_diag_tile(const float4* __restrict__ pm, int
     acc.z[T] += rz;
 }
 
-template <int T, bool EQ>
-__device__ __forceinline__ void sym_diag_phases(const float4* __restrict__ pm, int n, float eps2, int P,
-                                                const Lanes<8>& me, const float (&mi)[8], Lanes<8>& acc)
-{
-    sym_diag_tile<T, EQ>(pm, n, eps2, P, -1, me, mi, acc);
-    if constexpr (T + 1 < 8) sym_diag_phases<T + 1, EQ>(pm, n, eps2, P, me, mi, acc);
-}
-
-// Block P's diagonal as one task (see sym_diag_phases), into slot P. Bodies
-// past n are zero-mass padding and store into padding no reduction reads.
-// (v_rsq_f32 without a Newton step, as the batched kernel uses it.)
-__device__ __forceinline__ void sym_diag_block(const float4* __restrict__ pm, int n, int npad, float eps2,
-                                               float* __restrict__ part, int P)
-{
-    constexpr int B = 512;
-    const int lane = threadIdx.x & 63;
-    const size_t plane = (size_t)(npad / B) * npad;
-    const float m0 = pm[P * B].w;
-    Lanes<8> me, acc;
-    float mi[8];
-    bool same = true;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        const int i = P * B + u * 64 + lane;
-        const float4 q = i < n ? pm[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-        me.x[u] = q.x;
-        me.y[u] = q.y;
-        me.z[u] = q.z;
-        mi[u] = q.w;
-        same &= (i < n) & (q.w == m0);
-    }
-    zero<8>(acc);
-    const bool eq = __builtin_amdgcn_ballot_w64(!same) == 0;
-    if (eq) sym_diag_phases<0, true>(pm, n, eps2, P, me, mi, acc);
-    else sym_diag_phases<0, false>(pm, n, eps2, P, me, mi, acc);
-    const float scale = eq ? m0 : 1.0f;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        const size_t o = (size_t)P * npad + (size_t)P * B + u * 64 + lane;
-        part[o] = acc.x[u] * scale;
-        part[plane + o] = acc.y[u] * scale;
-        part[2 * plane + o] = acc.z[u] * scale;
-    }
-}
+constexpr int kDealWaves = 4;
 
 // Tiles t0, t0 + step, ... < t1 of the block that starts at body j0 past this
 // wave's 512 i bodies, the i side into acc. With halves = 1 each tile takes
@@ -823,7 +780,7 @@ __device__ __forceinline__ void sym_diag_block(const float4* __restrict__ pm, in
 // this wave takes steps 0..31 (half 0) or 32..63 (half 1), where it starts
 // half a turn on, and leaves the scaled reactions in r: half 0's in the lane
 // half a turn from the body's, half 1's in the body's own lane.
-template <bool NEWTON, bool EQ>
+template <bool NEWTON, bool EQ, int REGS>
 __device__ __forceinline__ void sym_deal_tiles(const float4* __restrict__ pm, int n, float eps2, int j0, int t0,
                                                int t1, int step, int half, int halves, const Lanes<8>& me,
                                                const float (&mi)[8], Lanes<8>& acc, float* jdst, size_t plane,
@@ -840,7 +797,7 @@ __device__ __forceinline__ void sym_deal_tiles(const float4* __restrict__ pm, in
         rx = ry = rz = 0.f;
         const int steps = halves == 2 ? 32 : 64;
         for (int k = 0; k < steps; ++k)
-            sym_step<8, NEWTON, EQ, EQ ? REGS_PINNED : REGS_FREE>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+            sym_step<8, NEWTON, EQ, REGS>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
         rx *= scale;
         ry *= scale;
         rz *= scale;
@@ -899,6 +856,96 @@ __device__ __forceinline__ void sym_deal_diag(const float4* __restrict__ pm, int
         default: tiles(std::integral_constant<int, 3>{}, std::integral_constant<int, 4>{});
         }
     }
+}
+
+// Task h of block pair (P, Q), P < Q, blocks of 512, on a workgroup of 4
+// waves that each hold block P's bodies (k_force_sym_deal, k_force_batch):
+// part h of `split` = 1, 2 or 4 of block Q's tiles, dealt to the waves. P == Q:
+// the diagonal block, or with split 4 half h of it. Task h's i sides go `more`
+// elements past task h - 1's. `part` is the workgroup's LDS. EQ_REGS, GEN_REGS:
+// the steps' registers on one mass and otherwise.
+template <bool NEWTON, int EQ_REGS, int GEN_REGS>
+__device__ __forceinline__ void sym_deal_task(const float4* __restrict__ pm, int n, float eps2, const SlotMap& slots,
+                                              int P, int Q, int h, int split, size_t more, float (*part)[3][512])
+{
+    constexpr int W = kDealWaves, B = 512, T = B / 64;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int halves = split == 4 ? 2 : 1;  // a tile's 64 steps on one wave, or 32 on each of two
+    const bool diag = P == Q;
+    const float m0 = pm[P * B].w;
+    Lanes<8> me, acc;
+    float mi[8];
+    bool same = true;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int i = P * B + u * 64 + lane;
+        const float4 q = i < n ? pm[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+        me.x[u] = q.x;
+        me.y[u] = q.y;
+        me.z[u] = q.z;
+        mi[u] = q.w;
+        same &= (i < n) & (q.w == m0);
+    }
+    zero<8>(acc);
+    float scale = 1.0f;
+    if (diag) {
+        const bool eq = !NEWTON && __builtin_amdgcn_ballot_w64(!same) == 0;
+        sym_deal_diag<NEWTON>(pm, n, eps2, P, wave, h, halves, eq, me, mi, acc);
+        if (eq) scale = m0;
+    } else {
+        // tiles t0, t0 + W, ... < t1 of block Q
+        const int half = halves == 2 ? wave & 1 : 0;
+        const int t0 = h * (T / split) + (halves == 2 ? wave >> 1 : wave), t1 = split == 1 ? T : t0 + 1;
+        for (int tile = t0; tile < t1; tile += W) {
+            const int j = Q * B + tile * 64 + lane;
+            same &= (j < n) & (pm[min(j, n - 1)].w == m0);
+        }
+        const bool eq = __builtin_amdgcn_ballot_w64(!same) == 0;
+        if (eq) scale = m0;
+        float* jdst = slots.j_side(P, Q, B);
+        const size_t plane = slots.bplane;
+        const int out = t0 * 64;
+        float r[3];
+        if (eq)
+            sym_deal_tiles<NEWTON, true, EQ_REGS>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst,
+                                                  plane, m0, r);
+        else
+            sym_deal_tiles<NEWTON, false, GEN_REGS>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst,
+                                                    plane, 1.0f, r);
+        if (halves == 2) {
+            // the first half's reactions are half a turn from home; the second wave adds both in order
+            if (half == 0) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) part[wave][c][lane ^ 32] = r[c];
+            }
+            __syncthreads();
+            if (half == 1 && Q * B + out < n) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) jdst[c * plane + out + lane] = part[wave - 1][c][lane] + r[c];
+            }
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        part[wave][0][u * 64 + lane] = acc.x[u] * scale;
+        part[wave][1][u * 64 + lane] = acc.y[u] * scale;
+        part[wave][2][u * 64 + lane] = acc.z[u] * scale;
+    }
+    __syncthreads();
+    float* __restrict__ idst = (diag ? slots.j_side(P, P, B) : slots.i_side(P, Q, B)) + h * more;
+    const size_t iplane = diag ? slots.bplane : slots.i_plane(P);
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int k = 0; k < B; k += 64 * W) {
+            const int o = k + threadIdx.x;
+            float sum = part[0][c][o];
+#pragma unroll
+            for (int w = 1; w < W; ++w) sum += part[w][c][o];
+            idst[c * iplane + o] = sum;
+        }
 }
 
 // Piece k (of A) of block P's diagonal: its 64*W threads take bodies

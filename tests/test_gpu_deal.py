@@ -14,6 +14,7 @@ from gpu_util import dev, run_force
 from oracle_lib import force_errors
 
 from nbody_amd import _native, ics
+from nbody_amd.engine import Ensemble
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +43,33 @@ def test_every_split(oracle, n, split, newton):
         assert np.all(f[:, 3] == -7.0)
         again = run_force(d, EPS2, slot_bytes=budget, newton=newton, **SHAPE)
         assert np.array_equal(f.view(np.uint32), again.view(np.uint32)), (what, n, split, newton)
+
+
+def test_batched_blocks(oracle):
+    """The batched form (one task per pair, taken from a queue): a last block
+    of 1..8 tiles, ragged or full, beside none, one or two full blocks, with
+    every kind of masses in one batch, and some of the systems alone."""
+    sizes = sorted({b * 512 + 64 * t - r for b in (0, 1, 2) for t in range(1, 9) for r in (0, 1, 63)})
+    systems = []
+    for k, n in enumerate(sizes):
+        pm, vm = ics.random_unit_bodies(n, seed=400 + k)
+        if k % 3:
+            pm[:, 3] = 0.37
+        if k % 3 == 2:
+            pm[n // 2, 3] = 0.6
+        systems.append((pm, vm))
+
+    def forces(which):
+        with Ensemble(which, EPS2, dt=0.002) as e:
+            e.run(1)
+            return e.split(e.read()[2])
+
+    got = forces(systems)
+    for (pm, _), f in zip(systems, got):
+        if len(pm) == 1:
+            assert np.all(f[:, :3] == 0.0)
+            continue
+        mx, rms = force_errors(f, oracle.fp64_forces(pm, EPS2))
+        assert mx <= TOL_MAX and rms <= TOL_RMS, (len(pm), mx, rms)
+    for k in (0, 7, len(systems) - 1):
+        assert np.array_equal(forces([systems[k]])[0].view(np.uint32), got[k].view(np.uint32)), sizes[k]
