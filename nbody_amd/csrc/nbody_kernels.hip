@@ -19,6 +19,8 @@
 #include "nbody_sym.h"
 #include "nbody_tile.h"
 
+#include <hip/hip_ext.h>
+
 #include <algorithm>
 #include <cmath>
 #include <map>
@@ -839,23 +841,24 @@ hipError_t go_family(const ForcePlan& plan, dim3 g, hipStream_t s, const ForcePa
 }
 
 template <int LI, int I>
-void go_tile_shape(dim3 g, hipStream_t s, const ForceParams& p)
+void go_tile_shape(dim3 g, hipStream_t s, const ForceParams& p, hipEvent_t done)
 {
-    if (p.step.vm) k_force_tile<LI, I, true><<<g, kTileThreads, 0, s>>>(p);
-    else k_force_tile<LI, I, false><<<g, kTileThreads, 0, s>>>(p);
+    const auto kernel = p.step.vm ? k_force_tile<LI, I, true> : k_force_tile<LI, I, false>;
+    if (done) hipExtLaunchKernelGGL(kernel, g, dim3(kTileThreads), 0, s, nullptr, done, 0, p);
+    else kernel<<<g, kTileThreads, 0, s>>>(p);
 }
 
-hipError_t go_tile(const ForcePlan& plan, dim3 g, hipStream_t s, const ForceParams& p)
+hipError_t go_tile(const ForcePlan& plan, dim3 g, hipStream_t s, const ForceParams& p, hipEvent_t done)
 {
     switch (plan.li * 100 + plan.ipl) {
-    case 401: go_tile_shape<4, 1>(g, s, p); break;
-    case 402: go_tile_shape<4, 2>(g, s, p); break;
-    case 403: go_tile_shape<4, 3>(g, s, p); break;
-    case 802: go_tile_shape<8, 2>(g, s, p); break;
-    case 803: go_tile_shape<8, 3>(g, s, p); break;
-    case 804: go_tile_shape<8, 4>(g, s, p); break;
-    case 805: go_tile_shape<8, 5>(g, s, p); break;
-    case 806: go_tile_shape<8, 6>(g, s, p); break;
+    case 401: go_tile_shape<4, 1>(g, s, p, done); break;
+    case 402: go_tile_shape<4, 2>(g, s, p, done); break;
+    case 403: go_tile_shape<4, 3>(g, s, p, done); break;
+    case 802: go_tile_shape<8, 2>(g, s, p, done); break;
+    case 803: go_tile_shape<8, 3>(g, s, p, done); break;
+    case 804: go_tile_shape<8, 4>(g, s, p, done); break;
+    case 805: go_tile_shape<8, 5>(g, s, p, done); break;
+    case 806: go_tile_shape<8, 6>(g, s, p, done); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1108,7 +1111,7 @@ size_t plan_scratch_bytes(const ForcePlan& plan, int ni)
 }
 
 hipError_t launch_force(const ForcePlan& plan, const ForceParams& p, hipStream_t stream, hipEvent_t before,
-                        hipEvent_t after)
+                        hipEvent_t after, hipEvent_t done)
 {
     if (p.ni <= 0 || p.n <= 0) return hipSuccess;
     if (before) {
@@ -1128,7 +1131,7 @@ hipError_t launch_force(const ForcePlan& plan, const ForceParams& p, hipStream_t
     }
     if (plan.li > 0) {
         const dim3 g((p.ni + plan.li * plan.ipl - 1) / (plan.li * plan.ipl));
-        e = go_tile(plan, g, stream, p);
+        e = go_tile(plan, g, stream, p, done);
         if (e == hipSuccess && after) e = hipEventRecord(after, stream);
         return e;
     }

@@ -12,12 +12,13 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 from conftest import EPS2
 from gpu_util import dev, force_buffer, host, ptr, run_force
 from oracle_lib import force_errors
 
-from nbody_amd import _native, ics
+from nbody_amd import _native, algorithms, ics
 
 pytestmark = pytest.mark.gpu
 
@@ -108,3 +109,19 @@ def test_slice_sum(oracle, slices, comp):
     mx, rms = force_errors(f, f64)
     assert mx <= TOL_MAX and rms <= TOL_RMS, (slices, comp, mx, rms)
     assert np.all(f[:, 3] == -7.0)
+
+
+@pytest.mark.parametrize("n", [1, 300, 10240, 10241])
+def test_table_entry_returns_when_the_forces_are_there(n):
+    """The table's synchronous entry, whose end event is the one launch itself
+    (N <= 10240) or a marker behind two: bit for bit the queued entry's forces,
+    read straight from host memory, with no further wait."""
+    pm, _ = ics.random_unit_bodies(n, seed=42)
+    d = dev(pm)
+    want = run_force(d, EPS2)
+    f = torch.empty(n, 4, pin_memory=True)
+    for _ in range(3):
+        f.fill_(-7.0)
+        ms = algorithms.find("HIP")(f.data_ptr(), d.data_ptr(), EPS2, n)
+        assert np.array_equal(f.numpy().view(np.uint32), want.view(np.uint32))
+        assert 0.0 < ms < 1e3
