@@ -406,21 +406,23 @@ __global__ __launch_bounds__(64 * W) void k_force_sym(SymParams p)
 // lanes of the one wave that meets it straight to their slot, and only the i
 // sides of the four waves meet, in LDS at the end: no barrier until then.
 //
-// Bound by the VALU issue of the pair chain (nbody_sym.h): 52 clocks of a SIMD
-// per 64 pairs with 4 or more waves on it, 59 with 2, 76 with 1 (stamps in the
-// kernel). What is left to lose is the spread of the work, which this split is
+// Bound by the VALU issue of the pair chain (nbody_sym.h): 43 to 44 clocks of
+// a SIMD per 64 pairs with 4 or more waves on it, 53 with 2. What is left to
+// lose is the spread of the work, which this split is
 // about: one-wave workgroups of whole block pairs gave the SIMDs of a small
 // system 2 or 3 tasks each; four-wave ones load a CU's SIMDs alike, and with
 // `split` tasks per pair (sym_split) the CUs too. The diagonal tasks come
 // first in the grid: each costs about a tenth more than a pair task (tiles
 // that meet one or two sub-blocks rotate as often as full ones), and the
-// oldest wave of a SIMD issues first, so last they would run on alone
-// (N = 16384: the pairs end at 51 us, such a diagonal at 55).
-// Kernel time, N = 98304 ball: 1.521 ms, 0.807 of the FP32 peak (1.58 ms with
-// one wave per block pair and the diagonal in one-sided pieces at the end);
-// unequal masses 1.70 ms (1.78). Whole evaluations, before and after:
-// N = 49999 480 and 422 us, 32768 212 and 188, 24576 141 and 115, 16384 68.5
-// and 59, 12000 53 and 43.
+// oldest wave of a SIMD issues first among equals, so last they would run on
+// alone (N = 16384, before the wave priorities: the pairs end at 51 us, such
+// a diagonal at 55).
+// Whole evaluations of one mass with one wave per block pair and the diagonal
+// in one-sided pieces at the end, with this split, and with the pair chain's
+// wave priorities too: N = 98304 1619, 1560 and 1358 us (0.905 of the FP32
+// peak), 49999 479, 429 and 379, 32768 212 and 188, 24576 141 and 115, 16384
+// 71.7, 62.2 and 54.7, 12000 53 and 43; unequal masses at 98304 1815, 1770
+// and 1541.
 template <bool NEWTON>
 __global__ __launch_bounds__(64 * kDealWaves, 6) void k_force_sym_deal(SymParams p)
 {

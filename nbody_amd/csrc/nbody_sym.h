@@ -106,19 +106,35 @@ __device__ __forceinline__ void upper_pair(int t, int& P, int& Q)
 // bit-identical to it. The i masses come in unnegated; the reaction weight
 // -m_i s^3 takes its sign from the source modifier, so no negated copies of
 // the masses need registers.
+//
+// Wave priorities (NBODY_PRIO) rise along each pair: lowest for the
+// differences, higher from the middle of d2 on, and not the same around the
+// v_rsq_f32 as in the sums. A SIMD issues up to two FP32 instructions of
+// different waves in four clocks, but not beside a v_rsq_f32. Left alone its
+// waves drift so that few of them can pair up. With the priorities the waves
+// that are past the middle of a pair run first and the others gather at its
+// start, where they pair. Clocks of a SIMD per 64 pairs, without and with, 6
+// waves: one mass 53.0 and 43.5, unequal masses 59.9 and 48.8; 4 waves 54.4
+// and 43.8, 61.0 and 52; 2 waves 58.7 and 53, 63.5 and 56. Of some 350
+// placements measured, one rise right before the v_rsq_f32 gives 43.8 and
+// 50.2, a fall there 52 and 58. The results are the same bits.
+#define NBODY_PRIO(p) "s_setprio " #p "\n"
 #define NBODY_SYM_PAIR(u)                                                                              \
+    NBODY_PRIO(0)                                                                                      \
     "v_sub_f32 %[dx], %[xj], %[x" #u "]\n"                                                             \
     "v_sub_f32 %[dy], %[yj], %[y" #u "]\n"                                                             \
     "v_sub_f32 %[dz], %[zj], %[z" #u "]\n"                                                             \
     "v_fma_f32 %[s], %[dx], %[dx], %[eps]\n"                                                           \
     "v_fmac_f32 %[s], %[dy], %[dy]\n"                                                                  \
+    NBODY_PRIO(2)                                                                                      \
     "v_fmac_f32 %[s], %[dz], %[dz]\n"                                                                  \
     "v_rsq_f32 %[s], %[s]\n"                                                                           \
     "s_nop 0\n"                                                                                        \
     "v_mul_f32 %[t], %[s], %[s]\n"                                                                     \
     "v_mul_f32 %[t], %[t], %[s]\n"                                                                     \
+    NBODY_PRIO(1)                                                                                      \
     "v_mul_f32 %[s], %[mj], %[t]\n"                                                                    \
-    "v_mul_f32 %[t], -%[n" #u "], %[t]\n"                                                               \
+    "v_mul_f32 %[t], -%[n" #u "], %[t]\n"                                                              \
     "v_fmac_f32 %[rx], %[dx], %[t]\n"                                                                  \
     "v_fmac_f32 %[ry], %[dy], %[t]\n"                                                                  \
     "v_fmac_f32 %[rz], %[dz], %[t]\n"                                                                  \
@@ -133,16 +149,19 @@ __device__ __forceinline__ void upper_pair(int t, int& P, int& Q)
 // instead of adding to the running reaction; NBODY_SYM_BLOCK_ADD then adds
 // the partial of the step's 8 pairs to the running reaction (Rx, Ry, Rz).
 #define NBODY_SYM_PAIR_EQ_FIRST(u)                                                                     \
+    NBODY_PRIO(0)                                                                                      \
     "v_sub_f32 %[dx], %[xj], %[x" #u "]\n"                                                             \
     "v_sub_f32 %[dy], %[yj], %[y" #u "]\n"                                                             \
     "v_sub_f32 %[dz], %[zj], %[z" #u "]\n"                                                             \
     "v_fma_f32 %[s], %[dx], %[dx], %[eps]\n"                                                           \
+    NBODY_PRIO(1)                                                                                      \
     "v_fmac_f32 %[s], %[dy], %[dy]\n"                                                                  \
     "v_fmac_f32 %[s], %[dz], %[dz]\n"                                                                  \
     "v_rsq_f32 %[s], %[s]\n"                                                                           \
     "s_nop 0\n"                                                                                        \
     "v_mul_f32 %[t], %[s], %[s]\n"                                                                     \
     "v_mul_f32 %[t], %[t], %[s]\n"                                                                     \
+    NBODY_PRIO(2)                                                                                      \
     "v_mul_f32 %[rx], -%[dx], %[t]\n"                                                                  \
     "v_mul_f32 %[ry], -%[dy], %[t]\n"                                                                  \
     "v_mul_f32 %[rz], -%[dz], %[t]\n"                                                                  \
@@ -151,18 +170,21 @@ __device__ __forceinline__ void upper_pair(int t, int& P, int& Q)
     "v_fmac_f32 %[az" #u "], %[dz], %[t]\n"
 
 #define NBODY_SYM_PAIR_FIRST(u)                                                                        \
+    NBODY_PRIO(0)                                                                                      \
     "v_sub_f32 %[dx], %[xj], %[x" #u "]\n"                                                             \
     "v_sub_f32 %[dy], %[yj], %[y" #u "]\n"                                                             \
     "v_sub_f32 %[dz], %[zj], %[z" #u "]\n"                                                             \
     "v_fma_f32 %[s], %[dx], %[dx], %[eps]\n"                                                           \
     "v_fmac_f32 %[s], %[dy], %[dy]\n"                                                                  \
+    NBODY_PRIO(2)                                                                                      \
     "v_fmac_f32 %[s], %[dz], %[dz]\n"                                                                  \
     "v_rsq_f32 %[s], %[s]\n"                                                                           \
     "s_nop 0\n"                                                                                        \
     "v_mul_f32 %[t], %[s], %[s]\n"                                                                     \
     "v_mul_f32 %[t], %[t], %[s]\n"                                                                     \
+    NBODY_PRIO(1)                                                                                      \
     "v_mul_f32 %[s], %[mj], %[t]\n"                                                                    \
-    "v_mul_f32 %[t], -%[n" #u "], %[t]\n"                                                               \
+    "v_mul_f32 %[t], -%[n" #u "], %[t]\n"                                                              \
     "v_mul_f32 %[rx], %[dx], %[t]\n"                                                                   \
     "v_mul_f32 %[ry], %[dy], %[t]\n"                                                                   \
     "v_mul_f32 %[rz], %[dz], %[t]\n"                                                                   \
@@ -254,16 +276,19 @@ __device__ __forceinline__ void sym_step8(float& xj, float& yj, float& zj, float
 // stores them. The reaction FMA negates d through the source modifier.
 // Bit-identical to the generic loop with EQ.
 #define NBODY_SYM_PAIR_EQ(u)                                                                           \
+    NBODY_PRIO(0)                                                                                      \
     "v_sub_f32 %[dx], %[xj], %[x" #u "]\n"                                                             \
     "v_sub_f32 %[dy], %[yj], %[y" #u "]\n"                                                             \
     "v_sub_f32 %[dz], %[zj], %[z" #u "]\n"                                                             \
     "v_fma_f32 %[s], %[dx], %[dx], %[eps]\n"                                                           \
+    NBODY_PRIO(1)                                                                                      \
     "v_fmac_f32 %[s], %[dy], %[dy]\n"                                                                  \
     "v_fmac_f32 %[s], %[dz], %[dz]\n"                                                                  \
     "v_rsq_f32 %[s], %[s]\n"                                                                           \
     "s_nop 0\n"                                                                                        \
     "v_mul_f32 %[t], %[s], %[s]\n"                                                                     \
     "v_mul_f32 %[t], %[t], %[s]\n"                                                                     \
+    NBODY_PRIO(2)                                                                                      \
     "v_fma_f32 %[rx], -%[dx], %[t], %[rx]\n"                                                           \
     "v_fma_f32 %[ry], -%[dy], %[t], %[ry]\n"                                                           \
     "v_fma_f32 %[rz], -%[dz], %[t], %[rz]\n"                                                           \
@@ -276,19 +301,22 @@ __device__ __forceinline__ void sym_step8(float& xj, float& yj, float& zj, float
 // Used for the one step of a diagonal tile against itself that would
 // otherwise take each pair twice.
 #define NBODY_SYM_PAIR_M(u)                                                                            \
+    NBODY_PRIO(0)                                                                                      \
     "v_sub_f32 %[dx], %[xj], %[x" #u "]\n"                                                             \
     "v_sub_f32 %[dy], %[yj], %[y" #u "]\n"                                                             \
     "v_sub_f32 %[dz], %[zj], %[z" #u "]\n"                                                             \
     "v_fma_f32 %[s], %[dx], %[dx], %[eps]\n"                                                           \
     "v_fmac_f32 %[s], %[dy], %[dy]\n"                                                                  \
+    NBODY_PRIO(2)                                                                                      \
     "v_fmac_f32 %[s], %[dz], %[dz]\n"                                                                  \
     "v_rsq_f32 %[s], %[s]\n"                                                                           \
     "s_nop 0\n"                                                                                        \
     "v_mul_f32 %[t], %[s], %[s]\n"                                                                     \
     "v_mul_f32 %[t], %[t], %[s]\n"                                                                     \
+    NBODY_PRIO(1)                                                                                      \
     "v_cndmask_b32 %[t], 0, %[t], %[mask]\n"                                                           \
     "v_mul_f32 %[s], %[mj], %[t]\n"                                                                    \
-    "v_mul_f32 %[t], -%[n" #u "], %[t]\n"                                                               \
+    "v_mul_f32 %[t], -%[n" #u "], %[t]\n"                                                              \
     "v_fmac_f32 %[rx], %[dx], %[t]\n"                                                                  \
     "v_fmac_f32 %[ry], %[dy], %[t]\n"                                                                  \
     "v_fmac_f32 %[rz], %[dz], %[t]\n"                                                                  \
@@ -297,16 +325,19 @@ __device__ __forceinline__ void sym_step8(float& xj, float& yj, float& zj, float
     "v_fmac_f32 %[az" #u "], %[dz], %[s]\n"
 
 #define NBODY_SYM_PAIR_EQ_M(u)                                                                         \
+    NBODY_PRIO(0)                                                                                      \
     "v_sub_f32 %[dx], %[xj], %[x" #u "]\n"                                                             \
     "v_sub_f32 %[dy], %[yj], %[y" #u "]\n"                                                             \
     "v_sub_f32 %[dz], %[zj], %[z" #u "]\n"                                                             \
     "v_fma_f32 %[s], %[dx], %[dx], %[eps]\n"                                                           \
+    NBODY_PRIO(1)                                                                                      \
     "v_fmac_f32 %[s], %[dy], %[dy]\n"                                                                  \
     "v_fmac_f32 %[s], %[dz], %[dz]\n"                                                                  \
     "v_rsq_f32 %[s], %[s]\n"                                                                           \
     "s_nop 0\n"                                                                                        \
     "v_mul_f32 %[t], %[s], %[s]\n"                                                                     \
     "v_mul_f32 %[t], %[t], %[s]\n"                                                                     \
+    NBODY_PRIO(2)                                                                                      \
     "v_cndmask_b32 %[t], 0, %[t], %[mask]\n"                                                           \
     "v_fma_f32 %[rx], -%[dx], %[t], %[rx]\n"                                                           \
     "v_fma_f32 %[ry], -%[dy], %[t], %[ry]\n"                                                           \
@@ -579,6 +610,7 @@ __device__ __forceinline__ void sym_diag_step8(float& xj, float& yj, float& zj, 
 #undef NBODY_LT7
 #undef NBODY_ROR_GEN
 #undef NBODY_ROR_EQ
+#undef NBODY_PRIO
 #undef NBODY_SYM_PAIR_M
 #undef NBODY_SYM_PAIR_EQ_M
 #undef NBODY_SYM_PAIR_EQ_FIRST
