@@ -64,19 +64,26 @@ __device__ __forceinline__ void body_body(float xj, float yj, float zj, float mj
 // at a measurably higher rate than the compiler's interleaving of independent
 // interactions. Same operations and rounding as body_body<false> (bit-
 // identical); one s_nop after v_rsq_f32 is the wait state gfx950 requires
-// before a VALU reads a transcendental result. JC is the register class of
-// the j body: "v" (from LDS or a DPP tile) or "s" (from scalar loads).
+// before a VALU reads a transcendental result. The wave's priority is low for
+// the differences and d2 and high from v_rsq_f32 on, so that the waves of a
+// SIMD meet in the first half, where two issue at once (nbody_sym.h): N =
+// 98304, one-sided, one mass 2407 and 2300 us, unequal masses 2597 and 2415;
+// from scalar loads 2748 and 2520. Nine other placements are within 2 % of
+// this one. JC is the register class of the j body: "v" (from LDS or a DPP
+// tile) or "s" (from scalar loads).
 #define NBODY_BODY_CHAIN(NAME, JC)                                                                     \
     __device__ __forceinline__ void NAME(float xj, float yj, float zj, float mj, float xi, float yi,   \
                                          float zi, float eps2, float& ax, float& ay, float& az)        \
     {                                                                                                  \
         float dx, dy, dz, s, t;                                                                        \
-        asm volatile("v_sub_f32 %[dx], %[xj], %[xi]\n"                                                 \
+        asm volatile("s_setprio 0\n"                                                                   \
+                     "v_sub_f32 %[dx], %[xj], %[xi]\n"                                                 \
                      "v_sub_f32 %[dy], %[yj], %[yi]\n"                                                 \
                      "v_sub_f32 %[dz], %[zj], %[zi]\n"                                                 \
                      "v_fma_f32 %[s], %[dx], %[dx], %[eps]\n"                                          \
                      "v_fmac_f32 %[s], %[dy], %[dy]\n"                                                 \
                      "v_fmac_f32 %[s], %[dz], %[dz]\n"                                                 \
+                     "s_setprio 1\n"                                                                   \
                      "v_rsq_f32 %[s], %[s]\n"                                                          \
                      "s_nop 0\n"                                                                       \
                      "v_mul_f32 %[t], %[mj], %[s]\n"                                                   \
@@ -106,12 +113,14 @@ NBODY_BODY_CHAIN(body_body_chain_s, "s")
                                          float zi, float eps2, float& ax, float& ay, float& az)        \
     {                                                                                                  \
         float dx, dy, dz, s, t;                                                                        \
-        asm volatile("v_sub_f32 %[dx], %[xj], %[xi]\n"                                                 \
+        asm volatile("s_setprio 0\n"                                                                   \
+                     "v_sub_f32 %[dx], %[xj], %[xi]\n"                                                 \
                      "v_sub_f32 %[dy], %[yj], %[yi]\n"                                                 \
                      "v_sub_f32 %[dz], %[zj], %[zi]\n"                                                 \
                      "v_fma_f32 %[s], %[dx], %[dx], %[eps]\n"                                          \
                      "v_fmac_f32 %[s], %[dy], %[dy]\n"                                                 \
                      "v_fmac_f32 %[s], %[dz], %[dz]\n"                                                 \
+                     "s_setprio 1\n"                                                                   \
                      "v_rsq_f32 %[s], %[s]\n"                                                          \
                      "s_nop 0\n"                                                                       \
                      "v_mul_f32 %[t], %[s], %[s]\n"                                                    \
