@@ -3,8 +3,7 @@
 // diagonal blocks, compensated rows) from a device work queue, then one
 // launch adds every body's slots and integrates it. Task lists are built on
 // the host, most expensive first. With FP64 accumulation the same scheme
-// runs the FP64 symmetric plan's pieces in one-wave workgroups
-// (k_force_batch64).
+// runs the FP64 symmetric plan's pieces (k_force_batch64).
 #include "nbody_acc64.h"
 #include "nbody_device.h"
 #include "nbody_kernels.h"
@@ -89,39 +88,37 @@ __global__ __launch_bounds__(kWave * kDealWaves, 6) void k_force_batch(const For
     }
 }
 
-// The FP64-accumulation tasks: PAIR64 block pairs and DIAG64 diagonal
-// pieces are k_force_sym64's (nbody_kernels.hip, 4 bodies per lane, blocks
-// of 256), ROW64 is 64 bodies against all n in j order into slot 0. No LDS:
-// every tile's reactions go from the lanes to their slots.
-__global__ __launch_bounds__(kWave) void k_force_batch64(const ForceTask* __restrict__ tasks, int ntasks,
-                                                         unsigned* __restrict__ counter)
+// The FP64-accumulation tasks: PAIR64 block pairs and DIAG64 diagonal blocks
+// are k_force_sym64's (nbody_kernels.hip, 4 bodies per lane, blocks of 256),
+// ROW64 is 64 bodies per wave against all n in j order into slot 0.
+__global__ __launch_bounds__(kWave * kWaves64) void k_force_batch64(const ForceTask* __restrict__ tasks, int ntasks,
+                                                                    unsigned* __restrict__ counter)
 {
-    for (bool first = true;; first = false) {
-        int t = (int)blockIdx.x;
-        if (!first && threadIdx.x == 0) t = (int)atomicAdd(counter, 1u) + (int)gridDim.x;
-        t = __builtin_amdgcn_readfirstlane(t);
-        if (t >= ntasks) return;
+    __shared__ double part[kWaves64][3][kBatchBlock64];
+    __shared__ int ticket;
+    for (int t = blockIdx.x; t < ntasks;) {
+        int next = 0;
+        if (threadIdx.x == 0) next = (int)atomicAdd(counter, 1u) + (int)gridDim.x;
         const ForceTask task = tasks[t];
-        const SlotMap64 slots = SlotMap64::whole(task.part64, task.nb, task.npad);
-        if (task.kind == TASK_PAIR64) {
-            sym_pair64<kPairA64, false>(task.pm, task.n, task.eps2, slots, task.a, task.b);
-            continue;
+        if (task.kind == TASK_ROW64) {
+            const int i = task.a + (int)threadIdx.x;
+            double ax, ay, az;
+            row64<false>(task.pm, task.n, task.eps2, i, task.b, task.len, ax, ay, az);
+            if (i < task.n) {
+                const size_t plane = (size_t)task.nb * task.npad;
+                const size_t o = (size_t)task.slot * task.npad + i;
+                task.part64[o] = ax;
+                task.part64[plane + o] = ay;
+                task.part64[2 * plane + o] = az;
+            }
+        } else {
+            sym_task64<kPairA64, false>(task.pm, task.n, task.eps2,
+                                        SlotMap64::whole(task.part64, task.nb, task.npad), task.a, task.b, part);
         }
-        if (task.kind == TASK_DIAG64) {
-            sym_diag_piece64<kBatchBlock64, false>(task.pm, task.n, task.eps2, slots, task.a, task.b);
-            continue;
-        }
-        // TASK_ROW64
-        const int i = task.a + (int)threadIdx.x;
-        double ax, ay, az;
-        row64<false>(task.pm, task.n, task.eps2, i, task.b, task.len, ax, ay, az);
-        if (i < task.n) {
-            const size_t plane = (size_t)task.nb * task.npad;
-            const size_t o = (size_t)task.slot * task.npad + i;
-            task.part64[o] = ax;
-            task.part64[plane + o] = ay;
-            task.part64[2 * plane + o] = az;
-        }
+        if (threadIdx.x == 0) ticket = next;
+        __syncthreads();  // (`part` is free after it as well)
+        t = __builtin_amdgcn_readfirstlane(ticket);
+        __syncthreads();
     }
 }
 
@@ -209,8 +206,8 @@ bool is_row(const ForceTask& t) { return t.kind == TASK_ROW_COMP || t.kind == TA
 // tiles of block Q that hold bodies (padding tiles are skipped)
 // with all 8 tiles of block P, 16 per Q tile, 128 for a full pair; a
 // diagonal block of T tiles takes each pair once, T^2, 64 when full. A
-// PAIR64 task meets block P's 4 tiles, 8 per Q tile; a DIAG64 piece (one
-// tile against the block, one-sided) 2 per tile of its block.
+// PAIR64 task meets block P's 4 tiles, 8 per Q tile; a DIAG64 task (every
+// tile against the block, one-sided) 4 per tile of its block.
 constexpr int kMaxTileKey = 16 * (kBatchBlock / kWave);
 
 int tile_key(const ForceTask& t)
@@ -219,7 +216,7 @@ int tile_key(const ForceTask& t)
     switch (t.kind) {
     case TASK_PAIR: return 16 * ((std::min(kBatchBlock, t.n - t.b * kBatchBlock) + kWave - 1) / kWave);
     case TASK_PAIR64: return 8 * ((std::min(kBatchBlock64, t.n - t.b * kBatchBlock64) + kWave - 1) / kWave);
-    case TASK_DIAG64: return 2 * ceil_tiles;
+    case TASK_DIAG64: return 4 * ceil_tiles;
     default: return ceil_tiles * ceil_tiles;
     }
 }
@@ -280,7 +277,7 @@ void append_force_tasks(std::vector<ForceTask>& out, const float4* pm, void* par
         t.b = 0;
         t.len = (int)n;
         t.slot = 0;
-        for (size_t i = 0; i < n; i += acc64 ? kWave : kWave * kDealWaves) {
+        for (size_t i = 0; i < n; i += kWave * kDealWaves) {
             t.a = (int)i;
             out.push_back(t);
         }
@@ -298,15 +295,7 @@ void append_force_tasks(std::vector<ForceTask>& out, const float4* pm, void* par
         t.a = t.b = p;
         t.len = (int)std::min<size_t>(B, n - (size_t)p * B);
         t.slot = p;
-        if (!acc64) {
-            out.push_back(t);
-            continue;
-        }
-        // the pieces of 64 bodies that hold any (a ragged last block has fewer)
-        for (int k = 0; k * kWave < t.len; ++k) {
-            t.b = k;
-            out.push_back(t);
-        }
+        out.push_back(t);
     }
 }
 
@@ -391,7 +380,7 @@ int batch_force_blocks_per_cu(bool acc64)
     if (c == 0) {
         int blocks = 0;
         const hipError_t e =
-            acc64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_force_batch64, kWave, 0)
+            acc64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_force_batch64, kWave * kWaves64, 0)
                   : hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_force_batch, kWave * kDealWaves, 0);
         if (e != hipSuccess || blocks < 1) blocks = 16;
         c = blocks;
@@ -404,7 +393,7 @@ hipError_t launch_force_batch(const ForceTask* tasks, int ntasks, unsigned* coun
 {
     if (ntasks <= 0) return hipSuccess;
     blocks = blocks < ntasks ? blocks : ntasks;
-    if (acc64) k_force_batch64<<<blocks, kWave, 0, stream>>>(tasks, ntasks, counter);
+    if (acc64) k_force_batch64<<<blocks, kWave * kWaves64, 0, stream>>>(tasks, ntasks, counter);
     else k_force_batch<<<blocks, kWave * kDealWaves, 0, stream>>>(tasks, ntasks, counter);
     return hipGetLastError();
 }

@@ -126,7 +126,7 @@ namespace nbody {
 // ---- batches of independent systems (ensembles, served requests) ----------
 //
 // One persistent launch computes the forces of many systems: four-wave
-// workgroups (one-wave ones with FP64 accumulation) take ForceTasks from a device work queue (an atomic counter).
+// workgroups take ForceTasks from a device work queue (an atomic counter).
 // A system of n <= kBatchPairMaxN bodies is cut into blocks of kBatchBlock
 // and runs as the symmetric plan does (nbody_sym.h): one PAIR task per block
 // pair P < Q and one DIAG task per diagonal block, each writing its own slot
@@ -139,16 +139,16 @@ namespace nbody {
 //
 // A batch with FP64 accumulation (compensated = 2) runs the FP64 symmetric
 // plan's pieces instead (nbody_acc64.h): blocks of kBatchBlock64 (4 bodies
-// per lane, one wave), PAIR64 tasks, four DIAG64 pieces per diagonal block
-// (64 bodies one-sided against the block), FP64 slot planes summed in slot
+// per lane, four waves share block Q), PAIR64 tasks, one DIAG64 task per
+// diagonal block (its bodies one-sided against the block), FP64 slot planes summed in slot
 // order and rounded once; a system above kBatchPairMaxN64 runs as ROW64
-// tasks (64 bodies against all n, one-sided, FP64 sums) into one slot. A
+// tasks (256 bodies against all n, one-sided, FP64 sums) into one slot. A
 // system of 1024 .. kBatchPairMaxN64 bodies then gets exactly the forces of
 // the single-system FP64 symmetric plan (4 bodies per lane, blocks of 256).
 
 constexpr int kBatchBlock = 512;                     // 8 bodies per lane, four waves share block Q
 constexpr size_t kBatchPairMaxN = size_t(1) << 18;   // largest system run as block pairs
-constexpr int kBatchBlock64 = 256;                   // FP64 accumulation: 4 bodies per lane, one wave
+constexpr int kBatchBlock64 = 256;                   // FP64 accumulation: 4 bodies per lane
 constexpr size_t kBatchPairMaxN64 = size_t(1) << 17; // FP64 accumulation: largest system run as block pairs
 
 enum BatchTaskKind : int {
@@ -169,8 +169,8 @@ struct ForceTask {
     int npad;          // length of one slot row
     float eps2;
     int kind;          // BatchTaskKind
-    int a;             // PAIR, DIAG: block P; ROW_COMP, ROW64: first i body (256, or 64, of them)
-    int b;             // PAIR: block Q; DIAG: block P; DIAG64: piece (0..3); ROW_COMP, ROW64: first j body
+    int a;             // PAIR, DIAG: block P; ROW_COMP, ROW64: first i body (256 of them)
+    int b;             // PAIR: block Q; DIAG, DIAG64: block P; ROW_COMP, ROW64: first j body
     int len;           // DIAG, DIAG64: bodies in the block; ROW_COMP, ROW64: number of j bodies
     int slot;          // slot written (DIAG, DIAG64: P; ROW_COMP, ROW64: 0)
     int reserved;

@@ -548,8 +548,9 @@ __global__ __launch_bounds__(64 * 3 * kReduceGroups) void k_reduce_band(SlotMap 
     }
 }
 
-// The symmetric plan with every term added in FP64 (the accurate plan): one
-// wave per task, A bodies per lane, blocks of B = 64 A; slots are doubles.
+// The symmetric plan with every term added in FP64 (the accurate plan): four
+// waves per block pair, A bodies per lane, blocks of B = 64 A; slots are
+// doubles.
 struct SymParams64 {
     const float4* pm;
     int n;
@@ -560,17 +561,14 @@ struct SymParams64 {
 };
 
 template <int A, bool NEWTON>
-__global__ __launch_bounds__(64) void k_force_sym64(SymParams64 p)
+__global__ __launch_bounds__(64 * kWaves64) void k_force_sym64(SymParams64 p)
 {
+    __shared__ double part[kWaves64][3][64 * A];
     const int t = blockIdx.x;
-    if (t < p.npairs) {
-        int P, Q;
-        upper_pair(p.q0 * (p.q0 - 1) / 2 + t, P, Q);
-        sym_pair64<A, NEWTON>(p.pm, p.n, p.eps2, p.slots, P, Q);
-    } else {
-        const int d = t - p.npairs;
-        sym_diag_piece64<64 * A, NEWTON>(p.pm, p.n, p.eps2, p.slots, p.q0 + d / A, d % A);
-    }
+    int P, Q;
+    if (t < p.npairs) upper_pair(p.q0 * (p.q0 - 1) / 2 + t, P, Q);
+    else P = Q = p.q0 + t - p.npairs;
+    sym_task64<A, NEWTON>(p.pm, p.n, p.eps2, p.slots, P, Q, part);
 }
 
 // k_reduce_band for FP64 slots: each body's slots of the band added in slot
@@ -1166,14 +1164,14 @@ hipError_t launch_force(const ForcePlan& plan, const ForceParams& p, hipStream_t
                 sp.npairs = npairs;
                 sp.eps2 = p.eps2;
                 sp.slots = band_slots(p.hi64, q0, q1, B);
-                const int tasks = npairs + w * plan.ipl;
+                const int tasks = npairs + w;
                 if (tasks > 0) {
                     if (plan.ipl == 4) {
-                        if (plan.newton) k_force_sym64<4, true><<<tasks, 64, 0, stream>>>(sp);
-                        else k_force_sym64<4, false><<<tasks, 64, 0, stream>>>(sp);
+                        if (plan.newton) k_force_sym64<4, true><<<tasks, 64 * kWaves64, 0, stream>>>(sp);
+                        else k_force_sym64<4, false><<<tasks, 64 * kWaves64, 0, stream>>>(sp);
                     } else {
-                        if (plan.newton) k_force_sym64<8, true><<<tasks, 64, 0, stream>>>(sp);
-                        else k_force_sym64<8, false><<<tasks, 64, 0, stream>>>(sp);
+                        if (plan.newton) k_force_sym64<8, true><<<tasks, 64 * kWaves64, 0, stream>>>(sp);
+                        else k_force_sym64<8, false><<<tasks, 64 * kWaves64, 0, stream>>>(sp);
                     }
                     e = hipGetLastError();
                 }

@@ -73,3 +73,32 @@ def test_batched_blocks(oracle):
         assert mx <= TOL_MAX and rms <= TOL_RMS, (len(pm), mx, rms)
     for k in (0, 7, len(systems) - 1):
         assert np.array_equal(forces([systems[k]])[0].view(np.uint32), got[k].view(np.uint32)), sizes[k]
+
+
+def test_fp64_blocks(oracle):
+    """With FP64 accumulation (four waves share block Q's tiles, one or two to a
+    wave): a last block of every tile count, ragged or full, and every kind of
+    masses, in both shapes against the oracle; the batched form gives the bits
+    of the 4-body one."""
+    sizes = [1, 63, 64, 65] + [256 * b + 64 * t - r for b in (1, 2, 5) for t in (1, 2, 3, 4) for r in (0, 1, 63)]
+    systems = []
+    for k, n in enumerate(sizes):
+        pm, vm = ics.random_unit_bodies(n, seed=600 + k)
+        if k % 3:
+            pm[:, 3] = 0.37
+        if k % 3 == 2:
+            pm[n // 2, 3] = 0.6
+        systems.append((pm, vm))
+    with Ensemble(systems, EPS2, dt=0.002, compensated=2) as e:
+        e.run(1)
+        batched = e.split(e.read()[2])
+    for (pm, _), got in zip(systems, batched):
+        for a in (4, 8):
+            f = run_force(dev(pm), EPS2, variant=_native.SYMMETRIC, i_per_lane=a, jslice=64 * a, compensated=2)
+            if len(pm) == 1:
+                assert np.all(f[:, :3] == 0.0)
+                continue
+            mx, rms = force_errors(f, oracle.fp64_forces(pm, EPS2))
+            assert mx <= TOL_MAX and rms <= TOL_RMS, (len(pm), a, mx, rms)
+            if a == 4:
+                assert np.array_equal(f[:, :3].view(np.uint32), np.ascontiguousarray(got[:, :3]).view(np.uint32)), len(pm)
