@@ -945,20 +945,23 @@ int deal_diag_tasks(int split) { return split == 4 ? 2 : 1; }
 // Tasks per block pair of a plan's k_force_sym_deal launch, 1, 2 or 4; only in
 // a single band over every column. More tasks put more waves on a SIMD and
 // end the launch more evenly: the fullest CU gets ceil(tasks / 256) of them,
-// each 1 / split of a pair, and a pair takes 22 us of a CU whose SIMDs hold 4
-// waves or more (1.46, 1.13 and 1.08 times that with 1, 2 and 3). But each
-// further task keeps its i sides in more slot rows, which the slot sum reads
-// back (12 bytes per body and row at about 4 TB/s). Measured, whole
-// evaluations with 1, 2, 4 tasks: N = 8192 40, 27, 24 us; 12000 51, 47, 43;
-// 16384, where 2 gives every CU exactly four tasks, 70, 59, 61; 20000 94, 91,
-// 86; 32768 199, 188, 195; 49999 424, 427, 442.
+// each 1 / split of a pair, and a pair takes 18.3 us of a CU whose SIMDs hold
+// 5 waves or more (few_waves times that with fewer), a task 1.3 us besides.
+// And each further task keeps its i sides in more slot rows, which the slot
+// sum reads back (12 bytes per body and row at about 8 TB/s, some of it from
+// the caches). The figures are fitted to whole evaluations at 22 sizes; the
+// choice is within 4 % of the best at each. Some of them, with 1, 2, 4 tasks:
+// N = 10241 50, 38, 35 us; 12288 59, 42, 43; 14336 60, 53, 52; 16384, where 2
+// gives every CU exactly four tasks, 63, 55, 60; 18432 69, 74, 74; 20480 90,
+// 84, 85; 24576 119, 106, 111; 32768 177, 176, 185; 40960 265, 264, 281; 49152
+// 370, 379, 413.
 int sym_split(const ForcePlan& plan, size_t nbands)
 {
     const bool whole = plan.col0 == 0 && (plan.col1 <= 0 || plan.col1 == plan.nslices);
     if (plan.acc64 || plan.ipl != 8 || plan.jslice != 512 || !whole || nbands != 1) return 1;
     const size_t cap = plan.band_cap ? plan.band_cap : kSymBandCap;
     const double nb = plan.nslices;
-    constexpr double few_waves[] = {1.0, 1.46, 1.13, 1.08};
+    constexpr double few_waves[] = {1.0, 2.2, 1.36, 1.07, 1.14};
     int best = 1;
     double least = 0.0;
     for (int split : {1, 2, 4}) {
@@ -966,8 +969,8 @@ int sym_split(const ForcePlan& plan, size_t nbands)
         const double tasks = 0.5 * nb * (nb - 1.0) * split + nb * deal_diag_tasks(split);
         const double rows = nb + 0.5 * (nb - 1.0) * (split - 1);
         const double fullest = std::ceil(tasks / 256.0);
-        const double us = fullest * 22.0 / split * (fullest < 4.0 ? few_waves[(int)fullest] : 1.0) +
-                          rows * nb * 512.0 * 12.0 / 4.0e6;
+        const double us = fullest * (18.3 / split + 1.3) * (fullest < 5.0 ? few_waves[(int)fullest] : 1.0) +
+                          rows * nb * 512.0 * 12.0 / 8.0e6;
         if (split == 1 || us < least) {
             least = us;
             best = split;
