@@ -166,7 +166,7 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
         // launches and slice sum (one GPU's share, half of N: N = 16384 52 and, in one launch, 41 us,
         // 20000 71 and 63, 33588 153 and 188)
         const double sliced = std::max(0.26e-6 * (double)n * (double)N, 0.044 * p.jslice * p.ipl) + 16.0;
-        if (tile_allowed(N, n, opt) && tile_shape(N, n, &li, &ipl) < sliced) {
+        if (tile_allowed(N, n, opt) && tile_shape(N, n, false, &li, &ipl) < sliced) {
             p.li = li;
             p.ipl = ipl;
             p.jslice = (int)N;
@@ -195,6 +195,21 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
     }
     p.jslice = std::max(1, std::min(p.jslice, (int)N));
     p.nslices = (int)((N + p.jslice - 1) / p.jslice);
+    if (variant == VAR_LDS && p.acc64 && n > 0 && !p.newton &&
+        !(opt && (opt->i_per_lane > 0 || opt->jslice > 0 || opt->waves_per_simd > 0))) {
+        // the FP64 form of the one-launch kernel, against the sliced plan's throughput or one lane's chain
+        // through its slice, and 16 us of launches and slice sum if there are slices (8192 of 16384 bodies 74
+        // and, in one launch, 70 us; 8192 of 65536 stay sliced: 231)
+        const double sliced =
+            std::max(0.41e-6 * (double)n * (double)N, 0.0445 * p.jslice) + (p.nslices > 1 ? 16.0 : 3.0);
+        int li, ipl;
+        if (tile_shape(N, n, true, &li, &ipl) < sliced) {
+            p.li = li;
+            p.ipl = ipl;
+            p.jslice = (int)N;
+            p.nslices = 1;
+        }
+    }
     return p;
 }
 

@@ -30,6 +30,17 @@ __device__ __forceinline__ void zero(Lanes64<I>& a)
     for (int u = 0; u < I; ++u) a.x[u] = a.y[u] = a.z[u] = 0.0;
 }
 
+template <int I>
+__device__ __forceinline__ void scale(Lanes64<I>& a, double m)
+{
+#pragma unroll
+    for (int u = 0; u < I; ++u) {
+        a.x[u] *= m;
+        a.y[u] *= m;
+        a.z[u] *= m;
+    }
+}
+
 typedef SlotMapT<double> SlotMap64;
 
 // Each interaction is cut in two, the FP32 terms with their conversions at the

@@ -84,7 +84,7 @@ bool step_needs_buffer(const ForcePlan& plan);
 
 // The shape of the one-launch kernel that ends first for ni of n bodies;
 // returns its estimated microseconds.
-double tile_shape(size_t n, size_t ni, int* li, int* ipl);
+double tile_shape(size_t n, size_t ni, bool acc64, int* li, int* ipl);
 
 // Whether (i per lane, block size) is a compiled symmetric shape.
 bool symmetric_shape_ok(int ipl, int block);

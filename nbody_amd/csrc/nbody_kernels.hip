@@ -840,17 +840,20 @@ hipError_t go_family(const ForcePlan& plan, dim3 g, hipStream_t s, const ForcePa
     return hipGetLastError();
 }
 
-template <int LI, int I>
+template <int LI, int I, bool F64 = false>
 void go_tile_shape(dim3 g, hipStream_t s, const ForceParams& p, hipEvent_t done)
 {
-    const auto kernel = p.step.vm ? k_force_tile<LI, I, true> : k_force_tile<LI, I, false>;
+    const auto kernel = p.step.vm ? k_force_tile<LI, I, true, F64> : k_force_tile<LI, I, false, F64>;
     if (done) hipExtLaunchKernelGGL(kernel, g, dim3(kTileThreads), 0, s, nullptr, done, 0, p);
     else kernel<<<g, kTileThreads, 0, s>>>(p);
 }
 
 hipError_t go_tile(const ForcePlan& plan, dim3 g, hipStream_t s, const ForceParams& p, hipEvent_t done)
 {
-    switch (plan.li * 100 + plan.ipl) {
+    switch (plan.li * 100 + plan.ipl + (plan.acc64 ? 10000 : 0)) {
+    case 10401: go_tile_shape<4, 1, true>(g, s, p, done); break;
+    case 10402: go_tile_shape<4, 2, true>(g, s, p, done); break;
+    case 10802: go_tile_shape<8, 2, true>(g, s, p, done); break;
     case 401: go_tile_shape<4, 1>(g, s, p, done); break;
     case 402: go_tile_shape<4, 2>(g, s, p, done); break;
     case 403: go_tile_shape<4, 3>(g, s, p, done); break;
@@ -1017,13 +1020,14 @@ constexpr TileShape kTileShapes[] = {{4, 1, .263}, {4, 2, .200}, {4, 3, .183}, {
 
 }  // namespace
 
-double tile_shape(size_t n, size_t ni, int* li, int* ipl)
+double tile_shape(size_t n, size_t ni, bool acc64, int* li, int* ipl)
 {
     constexpr size_t cus = 256;
     double least = 0.0;
     for (const TileShape& s : kTileShapes) {
-        const size_t ti = (size_t)s.li * s.ipl, groups = (ni + ti - 1) / ti, per_cu = s.ipl <= 3 ? 2 : 1;
-        const double work = (double)ti * (double)n * s.clocks;  // of one workgroup, on a full CU
+        if (acc64 && s.ipl > 2) continue;  // (built up to 2)
+        const size_t ti = (size_t)s.li * s.ipl, groups = (ni + ti - 1) / ti, per_cu = s.ipl <= (acc64 ? 1 : 3) ? 2 : 1;
+        const double work = (double)ti * (double)n * s.clocks * (acc64 ? 1.6 : 1.0);  // of a workgroup, on a full CU
         const double fixed = 4000.0 + 900.0 * s.ipl;            // launch, first loads, last sum
         const size_t full = groups / (per_cu * cus), rest = groups % (per_cu * cus);
         double t = (double)full * ((double)per_cu * work + fixed);

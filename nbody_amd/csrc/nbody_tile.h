@@ -17,12 +17,22 @@
 // chain over all j took 11.7 and 42); above, the one-sided chain (11 VALU +
 // 1 v_rsq_f32 per interaction on one mass, 12 otherwise) at 4 or 8 waves per
 // SIMD, with a ds_read_b128 of the CU's LDS (about 12 clocks) per step of I
-// interactions: 8.1 us at N = 4096, 22.1 at 8192 (0.39 of the FP32 peak),
-// 32.6 at 10000.
+// interactions: 8.1 us at N = 4096, 21.0 at 8192 (0.41 of the FP32 peak),
+// 31 at 10000.
+//
+// With FP64 accumulation (F64) every term is added in FP64 and the groups'
+// and waves' sums stay FP64 to the end (nbody_acc64.h). There it replaces the
+// one serial chain over all j of a system below 1024 bodies or of a small i
+// range: N = 256 12.2 and 3.9 us, 1000 44.4 and 3.9, 500 of 2000 87 and 4.2,
+// 2048 of 16384 52.6 and 21.7 (two launches with slices), 1000 of 65536 70 and
+// 49.
 #pragma once
 
+#include "nbody_acc64.h"
 #include "nbody_device.h"
 #include "nbody_kernels.h"
+
+#include <type_traits>
 
 namespace nbody {
 
@@ -39,29 +49,49 @@ __device__ __forceinline__ float row_ror(float v)
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
+template <int CTRL>
+__device__ __forceinline__ double row_ror(double v)
+{
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)u, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
+}
+
 // add(partner) for each halving of a wave's groups of LI = 4 or 8 lanes; after
 // them every lane holds the sum over the groups.
 template <int LI, class Add>
 __device__ __forceinline__ void over_groups(const Add& add)
 {
     static_assert(LI == 4 || LI == 8, "groups within a row of 16 lanes");
-    if constexpr (LI == 4) add([](float v) { return row_ror<0x124>(v); });  // row_ror:4
-    add([](float v) { return row_ror<0x128>(v); });                         // row_ror:8
-    add([](float v) { return __shfl_xor(v, 16); });
-    add([](float v) { return __shfl_xor(v, 32); });
+    if constexpr (LI == 4) add([](auto v) { return row_ror<0x124>(v); });  // row_ror:4
+    add([](auto v) { return row_ror<0x128>(v); });                         // row_ror:8
+    add([](auto v) { return __shfl_xor(v, 16); });
+    add([](auto v) { return __shfl_xor(v, 32); });
 }
 
 // `steps` records t4[0], t4[stride], ... against the lane's i bodies, two
 // records at a time; the next two are read while these are in use.
-template <int I, bool EQ>
+template <int I, bool EQ, class Acc>
 __device__ __forceinline__ void tile_sweep(const vec4* t4, int stride, int steps, float eps2, const Lanes<I>& me,
-                                           Lanes<I>& acc)
+                                           Acc& acc)
 {
     auto meet = [&](const vec4& b) {
 #pragma unroll
-        for (int u = 0; u < I; ++u)
-            interact<false, false, EQ>(b.x, b.y, b.z, b.w, me.x[u], me.y[u], me.z[u], eps2, acc.x[u], acc.y[u],
-                                       acc.z[u]);
+        for (int u = 0; u < I; ++u) {
+            if constexpr (std::is_same<Acc, Lanes64<I>>::value) {
+                begin_terms();
+                const Terms64 t = terms64<false, EQ>(make_float4(b.x, b.y, b.z, b.w), me.x[u], me.y[u], me.z[u], 0.f,
+                                                     eps2);
+                begin_sums();
+                acc.x[u] = __builtin_fma(t.x, t.si, acc.x[u]);
+                acc.y[u] = __builtin_fma(t.y, t.si, acc.y[u]);
+                acc.z[u] = __builtin_fma(t.z, t.si, acc.z[u]);
+            } else {
+                interact<false, false, EQ>(b.x, b.y, b.z, b.w, me.x[u], me.y[u], me.z[u], eps2, acc.x[u], acc.y[u],
+                                           acc.z[u]);
+            }
+        }
     };
     if (steps <= 0) return;
     auto record = [&](int k) { return t4[min(k, steps - 1) * stride]; };
@@ -84,21 +114,24 @@ __device__ __forceinline__ void tile_sweep(const vec4* t4, int stride, int steps
 // Up to 3 bodies per lane the kernel fits 64 VGPRs, two workgroups (8 waves
 // per SIMD) on a CU. STEP also integrates the workgroup's bodies, into another
 // position buffer: a step of a small system is then one launch.
-template <int LI, int I, bool STEP>
-__global__ __launch_bounds__(kTileThreads, I <= 3 ? 8 : 4) void k_force_tile(ForceParams p)
+template <int LI, int I, bool STEP, bool F64>
+__global__ __launch_bounds__(kTileThreads, I <= 3 && !F64 ? 8 : 4) void k_force_tile(ForceParams p)
 {
+    typedef typename std::conditional<F64, double, float>::type Sum;
+    typedef typename std::conditional<F64, Lanes64<I>, Lanes<I>>::type Acc;
     constexpr int S = 64 / LI;             // groups per wave
     constexpr int G = kTileWaves * S;      // groups per workgroup
     constexpr int TI = LI * I;             // i bodies per workgroup
     constexpr int R = kTileChunk / kTileThreads;
-    static_assert(kTileWaves * 3 * TI * sizeof(float) <= sizeof(vec4) * 2 * kTileChunk, "last sum fits the tiles");
+    static_assert(kTileWaves * 3 * TI * sizeof(Sum) <= sizeof(vec4) * 2 * kTileChunk, "last sum fits the tiles");
     __shared__ vec4 tile[2][kTileChunk];
     __shared__ int uneven[2][kTileWaves];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int group = wave * S + lane / LI;
     const int first = blockIdx.x * TI;
 
-    Lanes<I> me, acc;
+    Lanes<I> me;
+    Acc acc;
 #pragma unroll
     for (int u = 0; u < I; ++u) {
         const float4 q = p.pm[p.i0 + min(first + u * LI + lane % LI, p.ni - 1)];
@@ -141,17 +174,17 @@ __global__ __launch_bounds__(kTileThreads, I <= 3 ? 8 : 4) void k_force_tile(For
         const vec4* t4 = tile[buf] + group;
         const int steps = len / G;
         if (massless && !eq) {
-            if (c > 0) scale<I>(acc, m0);
+            if (c > 0) scale<I>(acc, (Sum)m0);
             massless = false;
         }
-        if (massless) tile_sweep<I, true>(t4, G, steps, p.eps2, me, acc);
-        else tile_sweep<I, false>(t4, G, steps, p.eps2, me, acc);
+        if (massless) tile_sweep<I, true, Acc>(t4, G, steps, p.eps2, me, acc);
+        else tile_sweep<I, false, Acc>(t4, G, steps, p.eps2, me, acc);
         if (steps * G + group < len) {  // the chunk's ragged last step
-            if (massless) tile_sweep<I, true>(t4 + steps * G, G, 1, p.eps2, me, acc);
-            else tile_sweep<I, false>(t4 + steps * G, G, 1, p.eps2, me, acc);
+            if (massless) tile_sweep<I, true, Acc>(t4 + steps * G, G, 1, p.eps2, me, acc);
+            else tile_sweep<I, false, Acc>(t4 + steps * G, G, 1, p.eps2, me, acc);
         }
     }
-    if (massless) scale<I>(acc, m0);
+    if (massless) scale<I>(acc, (Sum)m0);
 
     // the wave's groups, then the 16 waves in order
     over_groups<LI>([&](const auto& partner) {
@@ -163,9 +196,9 @@ __global__ __launch_bounds__(kTileThreads, I <= 3 ? 8 : 4) void k_force_tile(For
         }
     });
     __syncthreads();  // the last chunk has been read by every wave
-    float* red = reinterpret_cast<float*>(&tile[0][0]);  // [wave][3][TI]
+    Sum* red = reinterpret_cast<Sum*>(&tile[0][0]);  // [wave][3][TI]
     if (lane < LI) {
-        float* o = red + wave * 3 * TI + lane;
+        Sum* o = red + wave * 3 * TI + lane;
 #pragma unroll
         for (int u = 0; u < I; ++u) {
             o[0 * TI + u * LI] = acc.x[u];
@@ -185,8 +218,8 @@ __global__ __launch_bounds__(kTileThreads, I <= 3 ? 8 : 4) void k_force_tile(For
         p.force[4 * (size_t)m + t / TI] = total;
     }
     if constexpr (STEP) {
-        float* of = red + kTileWaves * 3 * TI;  // [3][TI], behind the waves' sums
-        static_assert((kTileWaves + 1) * 3 * TI * sizeof(float) <= sizeof(vec4) * 2 * kTileChunk, "fits the tiles");
+        float* of = reinterpret_cast<float*>(red + kTileWaves * 3 * TI);  // [3][TI], behind the waves' sums
+        static_assert((kTileWaves + 1) * 3 * TI * sizeof(Sum) <= sizeof(vec4) * 2 * kTileChunk, "fits the tiles");
         if (t < 3 * TI) of[t] = total;
         __syncthreads();
         if (t < TI && m < p.ni) step_body(p.step, m, of[t], of[TI + t], of[2 * TI + t]);

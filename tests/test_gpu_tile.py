@@ -19,6 +19,7 @@ from gpu_util import dev, force_buffer, host, ptr, run_force
 from oracle_lib import force_errors
 
 from nbody_amd import _native, algorithms, ics
+from nbody_amd.engine import System
 
 pytestmark = pytest.mark.gpu
 
@@ -125,3 +126,49 @@ def test_table_entry_returns_when_the_forces_are_there(n):
         ms = algorithms.find("HIP")(f.data_ptr(), d.data_ptr(), EPS2, n)
         assert np.array_equal(f.numpy().view(np.uint32), want.view(np.uint32))
         assert 0.0 < ms < 1e3
+
+
+@pytest.mark.parametrize("n,base,count", [(1, 0, 1), (2, 0, 2), (255, 0, 255), (300, 0, 300), (1023, 0, 1023),
+                                          (2049, 0, 2049), (4097, 0, 4097), (5000, 4999, 1), (5000, 123, 1777),
+                                          (16384, 4096, 2048)])
+@pytest.mark.parametrize("masses", ["unequal", "one", "heavier late"])
+def test_fp64_accumulation(oracle, n, base, count, masses):
+    """The one-launch kernel with every term added in FP64: below 1024 bodies,
+    the LDS variant's whole systems, i ranges."""
+    pm, _ = ics.random_unit_bodies(n, seed=43)
+    if masses != "unequal":
+        pm[:, 3] = 0.37
+    if masses == "heavier late":
+        pm[n - 1, 3] = 0.6
+    opt = dict(compensated=2, variant=_native.LDS if count == n >= 1024 else _native.AUTO)
+    p = plan(n, count, **opt)
+    assert p.variant == _native.LDS and p.i_per_lane == 0 and p.jslice == 0 and p.compensated == 2
+    d = dev(pm)
+    f = run_force(d, EPS2, base, count, **opt)
+    again = run_force(d, EPS2, base, count, **dict(opt, variant=p.variant, i_per_lane=p.i_per_lane, jslice=p.jslice))
+    assert np.array_equal(f.view(np.uint32), again.view(np.uint32))
+    assert np.all(f[:, 3] == -7.0)
+    if n == 1:
+        assert np.all(f[:, :3] == 0.0)
+        return
+    mx, rms = force_errors(f, oracle.fp64_forces(pm, EPS2)[base:base + count])
+    assert mx <= TOL_MAX and rms <= TOL_RMS, (n, masses, mx, rms)
+
+
+@pytest.mark.parametrize("n", [1, 700])
+def test_fp64_accumulation_steps(n):
+    """A step in that launch against the force entry and the integrator apart."""
+    pm, vm = ics.random_unit_bodies(n, seed=44)
+    o = _native.Options.make(compensated=2)
+    L = _native.lib()
+    d_pm, d_vm, f = dev(pm), dev(vm), force_buffer(n)
+    with System(pm, vm, EPS2, dt=0.002, damping=0.97, compensated=2) as s:
+        for steps in (1, 1, 17):
+            s.run(steps)
+            for _ in range(steps):
+                _native.check(L.nbody_hip_force(ptr(f), ptr(d_pm), EPS2, n, 0, n, ctypes.byref(o), None), "force")
+                _native.check(L.nbody_hip_integrate(ptr(d_pm), ptr(d_vm), ptr(f), 0.002, 0.97, n, None), "integrate")
+            p, v, g = s.read()
+            assert np.array_equal(p.view(np.uint32), host(d_pm).view(np.uint32))
+            assert np.array_equal(v.view(np.uint32), host(d_vm).view(np.uint32))
+            assert np.array_equal(g[:, :3].copy().view(np.uint32), host(f)[:, :3].copy().view(np.uint32))
