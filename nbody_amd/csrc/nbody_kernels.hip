@@ -423,7 +423,7 @@ __global__ __launch_bounds__(64 * W) void k_force_sym(SymParams p)
 // peak), 49999 479, 429 and 379, 32768 212 and 188, 24576 141 and 115, 16384
 // 71.7, 62.2 and 54.7, 12000 53 and 43; unequal masses at 98304 1815, 1770
 // and 1541.
-template <bool NEWTON>
+template <bool NEWTON, bool LEAD>
 __global__ __launch_bounds__(64 * kDealWaves, 6) void k_force_sym_deal(SymParams p)
 {
     __shared__ float part[kDealWaves][3][512];
@@ -437,7 +437,7 @@ __global__ __launch_bounds__(64 * kDealWaves, 6) void k_force_sym_deal(SymParams
         h = t % p.split;
         upper_pair(p.q0 * (p.q0 - 1) / 2 + t / p.split, P, Q);
     }
-    sym_deal_task<NEWTON, REGS_PINNED, REGS_FREE>(p.pm, p.n, p.eps2, p.slots, P, Q, h, p.split, p.more, part);
+    sym_deal_task<NEWTON, REGS_PINNED, REGS_FREE, LEAD>(p.pm, p.n, p.eps2, p.slots, P, Q, h, p.split, p.more, part);
 }
 
 constexpr int kReduceGroups = 4;
@@ -901,8 +901,8 @@ const void* sym_kernel()
 
 const void* deal_kernel(bool newton)
 {
-    return newton ? reinterpret_cast<const void*>(&k_force_sym_deal<true>)
-                  : reinterpret_cast<const void*>(&k_force_sym_deal<false>);
+    return newton ? reinterpret_cast<const void*>(&k_force_sym_deal<true, false>)
+                  : reinterpret_cast<const void*>(&k_force_sym_deal<false, false>);
 }
 
 template <int A, int W>
@@ -921,8 +921,13 @@ hipError_t go_sym_deal(const ForcePlan& plan, const SymParams& sp, hipStream_t s
     const int tasks = sp.npairs * sp.split + sp.diag_tasks, threads = 64 * kDealWaves;
     const void* k = deal_kernel(plan.newton);
     const size_t dyn = plan.occ > 0 ? lds_for_occupancy(k, threads, plan.occ) : 0;
-    if (plan.newton) k_force_sym_deal<true><<<tasks, threads, dyn, s>>>(sp);
-    else k_force_sym_deal<false><<<tasks, threads, dyn, s>>>(sp);
+    // With at most 4 tasks to a CU every task starts at once, and the waves of a SIMD had better end together:
+    // those in the first half of their steps go first. N = 16384 54.5 and 52.6 us, unequal masses 60.1 and 57.2,
+    // 10241 35.1 and 33.8. With more tasks it keeps the next ones waiting (20480 83.7 and 90.2, 32768 172 and 181).
+    const bool lead = tasks <= 4 * 256;
+    if (plan.newton) k_force_sym_deal<true, false><<<tasks, threads, dyn, s>>>(sp);
+    else if (lead) k_force_sym_deal<false, true><<<tasks, threads, dyn, s>>>(sp);
+    else k_force_sym_deal<false, false><<<tasks, threads, dyn, s>>>(sp);
     return hipGetLastError();
 }
 
@@ -953,7 +958,8 @@ int deal_diag_tasks(int split) { return split == 4 ? 2 : 1; }
 // And each further task keeps its i sides in more slot rows, which the slot
 // sum reads back (12 bytes per body and row at about 8 TB/s, some of it from
 // the caches). The figures are fitted to whole evaluations at 22 sizes; the
-// choice is within 4 % of the best at each. Some of them, with 1, 2, 4 tasks:
+// choice is within 4 % of the best at each. Some of them, with 1, 2, 4 tasks and
+// no lead for the first halves (go_sym_deal):
 // N = 10241 50, 38, 35 us; 12288 59, 42, 43; 14336 60, 53, 52; 16384, where 2
 // gives every CU exactly four tasks, 63, 55, 60; 18432 69, 74, 74; 20480 90,
 // 84, 85; 24576 119, 106, 111; 32768 177, 176, 185; 40960 265, 264, 281; 49152

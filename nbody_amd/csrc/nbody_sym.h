@@ -118,7 +118,8 @@ __device__ __forceinline__ void upper_pair(int t, int& P, int& Q)
 // and 43.8, 61.0 and 52; 2 waves 58.7 and 53, 63.5 and 56. Of some 350
 // placements measured, one rise right before the v_rsq_f32 gives 43.8 and
 // 50.2, a fall there 52 and 58. The results are the same bits.
-#define NBODY_PRIO(p) "s_setprio " #p "\n"
+#define NBODY_PRIO(p) "s_setprio %[p" #p "]\n"
+#define NBODY_PRIO_IN(base) [p0] "n"(base), [p1] "n"((base) + 1), [p2] "n"((base) + 2)
 #define NBODY_SYM_PAIR(u)                                                                              \
     NBODY_PRIO(0)                                                                                      \
     "v_sub_f32 %[dx], %[xj], %[x" #u "]\n"                                                             \
@@ -214,7 +215,7 @@ __device__ __forceinline__ void upper_pair(int t, int& P, int& Q)
 // without). The single-system kernel keeps one running sum: it holds the
 // bound on its configured state without the extra adds.
 enum : int { REGS_FREE = 0, REGS_PINNED = 1, REGS_APART = 2 };
-template <int REGS>
+template <int REGS, int BASE>
 __device__ __forceinline__ void sym_step8(float& xj, float& yj, float& zj, float& mj, float& rx, float& ry, float& rz,
                                           Lanes<8>& acc, const Lanes<8>& me, const float (&mi)[8], float eps2)
 {
@@ -243,7 +244,7 @@ __device__ __forceinline__ void sym_step8(float& xj, float& yj, float& zj, float
                        [z0] "v"(me.z[0]), [z1] "v"(me.z[1]), [z2] "v"(me.z[2]), [z3] "v"(me.z[3]),
                        [z4] "v"(me.z[4]), [z5] "v"(me.z[5]), [z6] "v"(me.z[6]), [z7] "v"(me.z[7]),
                        [n0] "v"(mi[0]), [n1] "v"(mi[1]), [n2] "v"(mi[2]), [n3] "v"(mi[3]),
-                       [n4] "v"(mi[4]), [n5] "v"(mi[5]), [n6] "v"(mi[6]), [n7] "v"(mi[7]), [eps] "s"(eps2));
+                       [n4] "v"(mi[4]), [n5] "v"(mi[5]), [n6] "v"(mi[6]), [n7] "v"(mi[7]), [eps] "s"(eps2), NBODY_PRIO_IN(BASE));
     } else {
         asm volatile(NBODY_SYM_PAIR(0) NBODY_SYM_PAIR(1) NBODY_SYM_PAIR(2) NBODY_SYM_PAIR(3)
                      NBODY_SYM_PAIR(4) NBODY_SYM_PAIR(5) NBODY_SYM_PAIR(6) NBODY_SYM_PAIR(7)
@@ -265,7 +266,7 @@ __device__ __forceinline__ void sym_step8(float& xj, float& yj, float& zj, float
                        [z0] "v"(me.z[0]), [z1] "v"(me.z[1]), [z2] "v"(me.z[2]), [z3] "v"(me.z[3]),
                        [z4] "v"(me.z[4]), [z5] "v"(me.z[5]), [z6] "v"(me.z[6]), [z7] "v"(me.z[7]),
                        [n0] "v"(mi[0]), [n1] "v"(mi[1]), [n2] "v"(mi[2]), [n3] "v"(mi[3]),
-                       [n4] "v"(mi[4]), [n5] "v"(mi[5]), [n6] "v"(mi[6]), [n7] "v"(mi[7]), [eps] "s"(eps2));
+                       [n4] "v"(mi[4]), [n5] "v"(mi[5]), [n6] "v"(mi[6]), [n7] "v"(mi[7]), [eps] "s"(eps2), NBODY_PRIO_IN(BASE));
     }
 }
 
@@ -346,7 +347,7 @@ __device__ __forceinline__ void sym_step8(float& xj, float& yj, float& zj, float
     "v_fmac_f32 %[ay" #u "], %[dy], %[t]\n"                                                            \
     "v_fmac_f32 %[az" #u "], %[dz], %[t]\n"
 
-template <int REGS>
+template <int REGS, int BASE>
 __device__ __forceinline__ void sym_step8_eq(float& xj, float& yj, float& zj, float& rx, float& ry, float& rz,
                                              Lanes<8>& acc, const Lanes<8>& me, float eps2)
 {
@@ -373,7 +374,7 @@ __device__ __forceinline__ void sym_step8_eq(float& xj, float& yj, float& zj, fl
                        [y0] "v"(me.y[0]), [y1] "v"(me.y[1]), [y2] "v"(me.y[2]), [y3] "v"(me.y[3]),
                        [y4] "v"(me.y[4]), [y5] "v"(me.y[5]), [y6] "v"(me.y[6]), [y7] "v"(me.y[7]),
                        [z0] "v"(me.z[0]), [z1] "v"(me.z[1]), [z2] "v"(me.z[2]), [z3] "v"(me.z[3]),
-                       [z4] "v"(me.z[4]), [z5] "v"(me.z[5]), [z6] "v"(me.z[6]), [z7] "v"(me.z[7]), [eps] "s"(eps2));
+                       [z4] "v"(me.z[4]), [z5] "v"(me.z[5]), [z6] "v"(me.z[6]), [z7] "v"(me.z[7]), [eps] "s"(eps2), NBODY_PRIO_IN(BASE));
     } else if constexpr (REGS == REGS_PINNED) {
         asm volatile(NBODY_SYM_PAIR_EQ(0) NBODY_SYM_PAIR_EQ(1) NBODY_SYM_PAIR_EQ(2) NBODY_SYM_PAIR_EQ(3)
                      NBODY_SYM_PAIR_EQ(4) NBODY_SYM_PAIR_EQ(5) NBODY_SYM_PAIR_EQ(6) NBODY_SYM_PAIR_EQ(7)
@@ -393,7 +394,7 @@ __device__ __forceinline__ void sym_step8_eq(float& xj, float& yj, float& zj, fl
                        [y0] "v"(me.y[0]), [y1] "v"(me.y[1]), [y2] "v"(me.y[2]), [y3] "v"(me.y[3]),
                        [y4] "v"(me.y[4]), [y5] "v"(me.y[5]), [y6] "v"(me.y[6]), [y7] "v"(me.y[7]),
                        [z0] "v"(me.z[0]), [z1] "v"(me.z[1]), [z2] "v"(me.z[2]), [z3] "v"(me.z[3]),
-                       [z4] "v"(me.z[4]), [z5] "v"(me.z[5]), [z6] "v"(me.z[6]), [z7] "v"(me.z[7]), [eps] "s"(eps2));
+                       [z4] "v"(me.z[4]), [z5] "v"(me.z[5]), [z6] "v"(me.z[6]), [z7] "v"(me.z[7]), [eps] "s"(eps2), NBODY_PRIO_IN(BASE));
     } else {
         asm volatile(NBODY_SYM_PAIR_EQ(0) NBODY_SYM_PAIR_EQ(1) NBODY_SYM_PAIR_EQ(2) NBODY_SYM_PAIR_EQ(3)
                      NBODY_SYM_PAIR_EQ(4) NBODY_SYM_PAIR_EQ(5) NBODY_SYM_PAIR_EQ(6) NBODY_SYM_PAIR_EQ(7)
@@ -413,7 +414,7 @@ __device__ __forceinline__ void sym_step8_eq(float& xj, float& yj, float& zj, fl
                        [y0] "v"(me.y[0]), [y1] "v"(me.y[1]), [y2] "v"(me.y[2]), [y3] "v"(me.y[3]),
                        [y4] "v"(me.y[4]), [y5] "v"(me.y[5]), [y6] "v"(me.y[6]), [y7] "v"(me.y[7]),
                        [z0] "v"(me.z[0]), [z1] "v"(me.z[1]), [z2] "v"(me.z[2]), [z3] "v"(me.z[3]),
-                       [z4] "v"(me.z[4]), [z5] "v"(me.z[5]), [z6] "v"(me.z[6]), [z7] "v"(me.z[7]), [eps] "s"(eps2));
+                       [z4] "v"(me.z[4]), [z5] "v"(me.z[5]), [z6] "v"(me.z[6]), [z7] "v"(me.z[7]), [eps] "s"(eps2), NBODY_PRIO_IN(BASE));
     }
 }
 
@@ -434,7 +435,7 @@ __device__ __forceinline__ void sym_step2(float& xj, float& yj, float& zj, float
                    [ay1] "+v"(acc.y[1]), [az0] "+v"(acc.z[0]), [az1] "+v"(acc.z[1]), [dx] "=&v"(dx),
                    [dy] "=&v"(dy), [dz] "=&v"(dz), [s] "=&v"(s), [t] "=&v"(t)
                  : [x0] "v"(me.x[0]), [x1] "v"(me.x[1]), [y0] "v"(me.y[0]), [y1] "v"(me.y[1]), [z0] "v"(me.z[0]),
-                   [z1] "v"(me.z[1]), [n0] "v"(mi[0]), [n1] "v"(mi[1]), [eps] "s"(eps2));
+                   [z1] "v"(me.z[1]), [n0] "v"(mi[0]), [n1] "v"(mi[1]), [eps] "s"(eps2), NBODY_PRIO_IN(0));
 }
 
 __device__ __forceinline__ void sym_step2_eq(float& xj, float& yj, float& zj, float& rx, float& ry, float& rz,
@@ -449,7 +450,7 @@ __device__ __forceinline__ void sym_step2_eq(float& xj, float& yj, float& zj, fl
                    [az0] "+v"(acc.z[0]), [az1] "+v"(acc.z[1]), [dx] "=&v"(dx), [dy] "=&v"(dy), [dz] "=&v"(dz),
                    [s] "=&v"(s), [t] "=&v"(t)
                  : [x0] "v"(me.x[0]), [x1] "v"(me.x[1]), [y0] "v"(me.y[0]), [y1] "v"(me.y[1]), [z0] "v"(me.z[0]),
-                   [z1] "v"(me.z[1]), [eps] "s"(eps2));
+                   [z1] "v"(me.z[1]), [eps] "s"(eps2), NBODY_PRIO_IN(0));
 }
 
 // One rotation step of diagonal tile T (see sym_diag_phases) in assembly, in
@@ -475,7 +476,7 @@ __device__ __forceinline__ void sym_step2_eq(float& xj, float& yj, float& zj, fl
       [y7] "v"(me.y[7]), [z0] "v"(me.z[0]), [z1] "v"(me.z[1]), [z2] "v"(me.z[2]), [z3] "v"(me.z[3]), \
       [z4] "v"(me.z[4]), [z5] "v"(me.z[5]), [z6] "v"(me.z[6]), [z7] "v"(me.z[7]), [n0] "v"(mi[0]), \
       [n1] "v"(mi[1]), [n2] "v"(mi[2]), [n3] "v"(mi[3]), [n4] "v"(mi[4]), [n5] "v"(mi[5]), [n6] "v"(mi[6]), \
-      [n7] "v"(mi[7]), [eps] "s"(eps2), [mask] "s"(mask)
+      [n7] "v"(mi[7]), [eps] "s"(eps2), NBODY_PRIO_IN(0), [mask] "s"(mask)
 
 // NBODY_LT<k>(P) expands to P(0) ... P(k-1): the pairs with the sub-blocks below tile k.
 #define NBODY_LT0(P)
@@ -611,6 +612,7 @@ __device__ __forceinline__ void sym_diag_step8(float& xj, float& yj, float& zj, 
 #undef NBODY_ROR_GEN
 #undef NBODY_ROR_EQ
 #undef NBODY_PRIO
+#undef NBODY_PRIO_IN
 #undef NBODY_SYM_PAIR_M
 #undef NBODY_SYM_PAIR_EQ_M
 #undef NBODY_SYM_PAIR_EQ_FIRST
@@ -623,13 +625,13 @@ __device__ __forceinline__ void sym_diag_step8(float& xj, float& yj, float& zj, 
 
 // One rotation step with A i bodies per lane: the assembly chain for 8 and 2,
 // else (and with a Newton step) the generic loop, which it equals bit for bit.
-template <int A, bool NEWTON, bool EQ, int REGS>
+template <int A, bool NEWTON, bool EQ, int REGS, int BASE = 0>
 __device__ __forceinline__ void sym_step(float& xj, float& yj, float& zj, float& mj, float& rx, float& ry, float& rz,
                                          Lanes<A>& acc, const Lanes<A>& me, const float (&mi)[A], float eps2)
 {
     if constexpr (A == 8 && !NEWTON) {
-        if constexpr (EQ) sym_step8_eq<REGS>(xj, yj, zj, rx, ry, rz, acc, me, eps2);
-        else sym_step8<REGS>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+        if constexpr (EQ) sym_step8_eq<REGS, BASE>(xj, yj, zj, rx, ry, rz, acc, me, eps2);
+        else sym_step8<REGS, BASE>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
     } else if constexpr (A == 2 && !NEWTON) {
         if constexpr (EQ) sym_step2_eq(xj, yj, zj, rx, ry, rz, acc, me, eps2);
         else sym_step2(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
@@ -811,8 +813,9 @@ constexpr int kDealWaves = 4;
 // wave alone meets the tile with these i bodies). With halves = 2 (one tile)
 // this wave takes steps 0..31 (half 0) or 32..63 (half 1), where it starts
 // half a turn on, and leaves the scaled reactions in r: half 0's in the lane
-// half a turn from the body's, half 1's in the body's own lane.
-template <bool NEWTON, bool EQ, int REGS>
+// half a turn from the body's, half 1's in the body's own lane. With LEAD the
+// first half of the wave's steps runs one priority higher.
+template <bool NEWTON, bool EQ, int REGS, bool LEAD>
 __device__ __forceinline__ void sym_deal_tiles(const float4* __restrict__ pm, int n, float eps2, int j0, int t0,
                                                int t1, int step, int half, int halves, const Lanes<8>& me,
                                                const float (&mi)[8], Lanes<8>& acc, float* jdst, size_t plane,
@@ -828,7 +831,13 @@ __device__ __forceinline__ void sym_deal_tiles(const float4* __restrict__ pm, in
         float xj = b.x, yj = b.y, zj = b.z, mj = b.w;
         rx = ry = rz = 0.f;
         const int steps = halves == 2 ? 32 : 64;
-        for (int k = 0; k < steps; ++k)
+        int k = 0;
+        if constexpr (LEAD) {
+            const int early = t1 - t0 > 1 ? (tile + step < t1 ? 64 : 0) : steps / 2;
+            for (; k < early; ++k)
+                sym_step<8, NEWTON, EQ, REGS, 1>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+        }
+        for (; k < steps; ++k)
             sym_step<8, NEWTON, EQ, REGS>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
         rx *= scale;
         ry *= scale;
@@ -896,7 +905,7 @@ __device__ __forceinline__ void sym_deal_diag(const float4* __restrict__ pm, int
 // the diagonal block, or with split 4 half h of it. Task h's i sides go `more`
 // elements past task h - 1's. `part` is the workgroup's LDS. EQ_REGS, GEN_REGS:
 // the steps' registers on one mass and otherwise.
-template <bool NEWTON, int EQ_REGS, int GEN_REGS>
+template <bool NEWTON, int EQ_REGS, int GEN_REGS, bool LEAD = false>
 __device__ __forceinline__ void sym_deal_task(const float4* __restrict__ pm, int n, float eps2, const SlotMap& slots,
                                               int P, int Q, int h, int split, size_t more, float (*part)[3][512])
 {
@@ -940,10 +949,10 @@ __device__ __forceinline__ void sym_deal_task(const float4* __restrict__ pm, int
         const int out = t0 * 64;
         float r[3];
         if (eq)
-            sym_deal_tiles<NEWTON, true, EQ_REGS>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst,
+            sym_deal_tiles<NEWTON, true, EQ_REGS, LEAD>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst,
                                                   plane, m0, r);
         else
-            sym_deal_tiles<NEWTON, false, GEN_REGS>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst,
+            sym_deal_tiles<NEWTON, false, GEN_REGS, LEAD>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst,
                                                     plane, 1.0f, r);
         if (halves == 2) {
             // the first half's reactions are half a turn from home; the second wave adds both in order
