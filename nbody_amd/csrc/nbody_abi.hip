@@ -77,8 +77,8 @@ constexpr size_t kSmallSymN = 5120;
 
 // Bodies up to which NBODY_HIP_AUTO evaluates a whole system in one launch
 // over the whole j range (nbody_tile.h) instead of by the symmetric plan. The
-// two: N = 4096 8.1 and 16.2 us, 8192 22 and 24, 10000 33 and 35, 12288 45
-// and 43.
+// two: N = 6144 14.8 and 24.9 us, 8192 20.9 and 26.3, 9216 29.3 and 29.0, 10240
+// 31.9 and 34.4, 11264 38.9 and 36.1.
 constexpr size_t kTileMaxN = 10240;
 
 // Whether the options leave an i range free to run so: plain sums, no Newton
@@ -95,7 +95,8 @@ bool tile_allowed(size_t N, size_t n, const nbody_hip_options* opt)
 // also the workgroups, so only past kLdsWideWork interactions; slices as
 // short as give each CU about 20 workgroups (the launch ends unevenly with
 // fewer), 256 bodies at least, and longer than 1024 only where even those give
-// it 80 (the slice sum reads 16 or 32 bytes per body and slice). Microseconds
+// it 80 (the slice sum reads 16 or 32 bytes per body and slice). Microseconds,
+// before the chains' wave priorities took 4 % off each,
 // for one GPU's eighth of N = 98304 with slices of 256, 512, 1024, 2048, two
 // bodies per lane: 308, 299, 305, 350, and with one: 332, 324, 326, 344; its
 // quarter of 150751: 1536, 1492, 1472, 1528; half of 33588 153, 164, 188, 240.

@@ -205,8 +205,9 @@ __device__ __forceinline__ void upper_pair(int t, int& P, int& Q)
 // 1.18 to 1.29 VALU instructions per clock per CU, and those five at the top
 // of that range. In the batched kernel the compiler picks a slow set, and
 // pinning raises its rate by about 7 %; in k_force_sym_deal, whose equal-mass
-// steps are REGS_PINNED, by 11 % (N = 98304: 1.74 and 1.57 ms). The general
-// step's own allocation there is as fast as the pinned one.
+// steps are REGS_PINNED, by 11 % (N = 98304: 1.74 and 1.57 ms; both before the
+// wave priorities, with which the compiler's set still loses 1 %). The
+// general step's own allocation there is as fast as the pinned one.
 // The batched kernel's steps (REGS_APART) also sum each step's 8 reaction terms
 // apart and add that partial to the running reaction (3 more VALU per 8
 // pairs, 1.2 % of its rate): the running j-side sums then take 64 roundings
