@@ -164,9 +164,10 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
         lds_shape(N, n, cus, &p.ipl, &p.jslice);
         int li, ipl;
         // the sliced plan's time: a wave's chain through its slice at the least, and about 16 us of
-        // launches and slice sum (one GPU's share, half of N: N = 16384 52 and, in one launch, 41 us,
-        // 20000 71 and 63, 33588 153 and 188)
-        const double sliced = std::max(0.26e-6 * (double)n * (double)N, 0.044 * p.jslice * p.ipl) + 16.0;
+        // launches and slice sum (sliced and in one launch: 1000 of 4096 bodies 19.5 and 4.6 us, 8192 of
+        // 16384 45 and 41, 10000 of 20000 67 and 59, 8000 of 33588 85 and 80, 6144 of 49152 88 and 90, 8192 of
+        // 65536 141 and 152, 32768 of 65536 505 and 580)
+        const double sliced = std::max(0.225e-6 * (double)n * (double)N, 0.044 * p.jslice * p.ipl) + 15.5;
         if (tile_allowed(N, n, opt) && tile_shape(N, n, false, &li, &ipl) < sliced) {
             p.li = li;
             p.ipl = ipl;

@@ -1016,13 +1016,18 @@ int natural_occupancy(bool newton)
 namespace {
 
 // The compiled shapes of k_force_tile and the clocks of a CU one interaction
-// takes in them when the workgroups fill it (measured at N = 8192 to 16384).
+// takes in them when the workgroups fill it, fitted with tile_shape's other
+// figures to every shape at ten sizes from N = 1000 to 10240. The choice is the
+// fastest shape at nine of them and within 5 % at N = 1000. Some of them, in
+// the order below: N = 2048 4.4, 4.3, 5.0, 5.2, 6.5, 7.7, 9.0, 10.3 us; 4096
+// 10.5, 8.6, 10.4, 7.8, 10.1, 12.3, 14.8, 17.0; 8192 32.0, 25.2, 25.4, 21.3,
+// 28.3, 21.7, 25.9, 30.2; 10240 47.5, 37.1, 39.5, 37.3, 35.0, 50.4, 31.7, 36.9.
 struct TileShape {
     int li, ipl;
     double clocks;
 };
-constexpr TileShape kTileShapes[] = {{4, 1, .263}, {4, 2, .200}, {4, 3, .183}, {8, 2, .175},
-                                     {8, 3, .172}, {8, 4, .180}, {8, 5, .178}, {8, 6, .175}};
+constexpr TileShape kTileShapes[] = {{4, 1, .242}, {4, 2, .191}, {4, 3, .175}, {8, 2, .161},
+                                     {8, 3, .157}, {8, 4, .166}, {8, 5, .164}, {8, 6, .163}};
 
 }  // namespace
 
@@ -1033,19 +1038,19 @@ double tile_shape(size_t n, size_t ni, bool acc64, int* li, int* ipl)
     for (const TileShape& s : kTileShapes) {
         if (acc64 && s.ipl > 2) continue;  // (built up to 2)
         const size_t ti = (size_t)s.li * s.ipl, groups = (ni + ti - 1) / ti, per_cu = s.ipl <= (acc64 ? 1 : 3) ? 2 : 1;
-        const double work = (double)ti * (double)n * s.clocks * (acc64 ? 1.6 : 1.0);  // of a workgroup, on a full CU
-        const double fixed = 4000.0 + 900.0 * s.ipl;            // launch, first loads, last sum
+        const double work = (double)ti * (double)n * s.clocks * (acc64 ? 1.85 : 1.0);  // of a workgroup, on a full CU
+        const double fixed = 1860.0 + 367.0 * s.ipl;            // first loads, last sum
         const size_t full = groups / (per_cu * cus), rest = groups % (per_cu * cus);
         double t = (double)full * ((double)per_cu * work + fixed);
         // a last round of one workgroup per CU has half the waves where two fit
-        if (rest) t += fixed + (rest > cus ? 2.0 * work : per_cu == 2 ? 1.15 * work : work);
+        if (rest) t += fixed + (rest > cus ? 2.0 * work : per_cu == 2 ? 1.04 * work : work);
         if (least == 0.0 || t < least) {
             least = t;
             *li = s.li;
             *ipl = s.ipl;
         }
     }
-    return least / 2400.0;
+    return least / 2400.0 + 2.1;
 }
 
 bool fuses_step(const ForcePlan& plan) { return plan.li > 0 || (plan.variant == VAR_SYMMETRIC && !plan.acc64); }
