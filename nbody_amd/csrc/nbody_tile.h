@@ -17,7 +17,7 @@
 // chain over all j took 11.7 and 42); above, the one-sided chain (11 VALU +
 // 1 v_rsq_f32 per interaction on one mass, 12 otherwise) at 4 or 8 waves per
 // SIMD, with a ds_read_b128 of the CU's LDS (about 12 clocks) per step of I
-// interactions: 8.1 us at N = 4096, 21.0 at 8192 (0.41 of the FP32 peak),
+// interactions: 7.8 us at N = 4096, 21.0 at 8192 (0.41 of the FP32 peak),
 // 31 at 10000.
 //
 // With FP64 accumulation (F64) every term is added in FP64 and the groups'
