@@ -454,14 +454,13 @@ __device__ __forceinline__ void sym_step2_eq(float& xj, float& yj, float& zj, fl
                    [z1] "v"(me.z[1]), [eps] "s"(eps2), NBODY_PRIO_IN(0));
 }
 
-// One rotation step of diagonal tile T (see sym_diag_phases) in assembly, in
+// One rotation step of diagonal tile T (see sym_diag_tile) in assembly, in
 // the chain order of sym_step8: the pairs with the i sub-blocks u < T, then
 // (MODE 1) the tile's own sub-block, or (MODE 2) the same with the weights of
 // the lanes outside `mask` cleared; then the rotation. Every operand of
 // sym_step8 is bound (they are live through the task anyway), so the
-// registers stay those of the block-pair step; the temporaries are pinned as
-// in sym_step8<true> (the batched kernel is the only user). With EQ the mass
-// neither enters nor rotates.
+// registers stay those of the block-pair step; the temporaries are REGS_PINNED.
+// With EQ the mass neither enters nor rotates.
 #define NBODY_DIAG_OPS \
     : [xj] "+v"(xj), [yj] "+v"(yj), [zj] "+v"(zj), [mj] "+v"(mj), [rx] "+v"(rx), [ry] "+v"(ry), [rz] "+v"(rz), \
       [ax0] "+v"(acc.x[0]), [ax1] "+v"(acc.x[1]), [ax2] "+v"(acc.x[2]), [ax3] "+v"(acc.x[3]), \
@@ -669,7 +668,7 @@ __device__ __forceinline__ void sym_step(float& xj, float& yj, float& zj, float&
 // The phases of block pair (P, Q): every wave streams the T tiles of block Q
 // past its A i bodies per lane, adding the i side into acc and each tile's
 // reaction into jacc. With EQ the pair weights leave out the (common) mass.
-template <int A, int W, bool NEWTON, bool EQ, int REGS>
+template <int A, int W, bool NEWTON, bool EQ>
 __device__ __forceinline__ void sym_phases(const float4* __restrict__ pm, int n, float eps2, int Q,
                                            const Lanes<A>& me, const float (&mi)[A], Lanes<A>& acc,
                                            float (*jacc)[64 * A * W])
@@ -690,7 +689,7 @@ __device__ __forceinline__ void sym_phases(const float4* __restrict__ pm, int n,
             const float4 b = lane < n - jbase ? pm[jbase + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
             float xj = b.x, yj = b.y, zj = b.z, mj = b.w;
             float rx = 0.f, ry = 0.f, rz = 0.f;
-            for (int k = 0; k < 64; ++k) sym_step<A, NEWTON, EQ, REGS>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+            for (int k = 0; k < 64; ++k) sym_step<A, NEWTON, EQ, REGS_FREE>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
             const int slot = tile * 64 + lane;
             jacc[0][slot] += rx;
             jacc[1][slot] += ry;
@@ -715,7 +714,7 @@ __device__ __forceinline__ bool workgroup_all(bool ok)
 // weights leave the mass out and the partials are multiplied by it once, at
 // the store; with m = 1 (or any power of two) the result is bit-identical to
 // the general weights.
-template <int A, int W, bool NEWTON, int REGS = REGS_FREE>
+template <int A, int W, bool NEWTON>
 __device__ __forceinline__ void sym_pair(const float4* __restrict__ pm, int n, float eps2, const SlotMap& slots, int P,
                                          int Q, float (*jacc)[64 * A * W])
 {
@@ -745,8 +744,8 @@ __device__ __forceinline__ void sym_pair(const float4* __restrict__ pm, int n, f
     for (int k = threadIdx.x; k < B; k += 64 * W) jacc[0][k] = jacc[1][k] = jacc[2][k] = 0.f;
     __syncthreads();
     const bool eq = workgroup_all<W>(same);
-    if (eq) sym_phases<A, W, NEWTON, true, REGS>(pm, n, eps2, Q, me, mi, acc, jacc);
-    else sym_phases<A, W, NEWTON, false, REGS>(pm, n, eps2, Q, me, mi, acc, jacc);
+    if (eq) sym_phases<A, W, NEWTON, true>(pm, n, eps2, Q, me, mi, acc, jacc);
+    else sym_phases<A, W, NEWTON, false>(pm, n, eps2, Q, me, mi, acc, jacc);
     const float scale = eq ? m0 : 1.0f;
     float* __restrict__ jdst = slots.j_side(P, Q, B);
     for (int k = threadIdx.x; k < B; k += 64 * W) {
