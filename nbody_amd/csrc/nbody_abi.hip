@@ -106,7 +106,8 @@ void lds_shape(size_t N, size_t n, int cus, int* ipl, int* jslice)
 {
     *ipl = (double)n * (double)N >= kLdsWideWork ? 2 : 1;
     const double per_cu = std::ceil((double)n / (256.0 * *ipl)) * (double)N / std::max(cus, 1);
-    const double len = per_cu / 20.0 <= 1024.0 ? per_cu / 20.0 : std::max(1024.0, per_cu / 80.0);
+    double len = per_cu / 20.0 <= 1024.0 ? per_cu / 20.0 : std::max(1024.0, per_cu / 80.0);
+    len = std::min(len, (double)N);  // (past 1.5e8 bodies the quotient no longer fits an int; N does)
     *jslice = std::max(1, (int)(len / 256.0 + 0.5)) * 256;
 }
 

@@ -1,0 +1,43 @@
+"""The library's choice of plans, asked through its internal host functions
+(tests/native/plan_probe.cpp, linked against the built library): no GPU call
+is made."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import ROOT, TESTS
+
+from nbody_amd import _native
+
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+@pytest.fixture(scope="session")
+def probe(tmp_path_factory):
+    """probe(line, ...) -> one list of ints per line."""
+    exe = str(tmp_path_factory.mktemp("plan") / "plan_probe")
+    libdir = os.path.dirname(_native.LIB_PATH)
+    subprocess.run([shutil.which("g++") or "g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__",
+                    "-I", os.path.join(ROCM, "include"), "-I", os.path.join(ROOT, "nbody_amd", "csrc"),
+                    "-I", os.path.join(ROOT, "include"), os.path.join(TESTS, "native", "plan_probe.cpp"), "-o", exe,
+                    "-L", libdir, "-lnbody_hip", "-L", os.path.join(ROCM, "lib"), "-lamdhip64",
+                    f"-Wl,-rpath,{libdir}", f"-Wl,-rpath,{os.path.join(ROCM, 'lib')}"], check=True)
+
+    def ask(*lines):
+        out = subprocess.run([exe], input="\n".join(lines) + "\n", stdout=subprocess.PIPE, check=True, text=True)
+        return [[int(v) for v in row.split()] for row in out.stdout.splitlines()]
+
+    return ask
+
+
+@pytest.mark.parametrize("n_all", [160_000_000, 215_000_000, 1 << 28])
+def test_lds_slices_of_the_largest_systems(probe, n_all):
+    """The slice length stays within the system and the slices within a launch's
+    second dimension, for whole systems, halves and single bodies."""
+    counts = [n_all, n_all // 2, n_all // 3, 1000, 1]
+    for n, (_, ipl, jslice, nslices, li) in zip(counts, probe(*[f"default {_native.LDS} {n_all} {n} 256"
+                                                               for n in counts])):
+        assert 1 <= jslice <= n_all and ipl in (1, 2) and (li == 0 or nslices == 1), (n, jslice)
+        assert nslices == -(-n_all // jslice) and nslices <= 65535, (n, jslice, nslices)
