@@ -422,9 +422,10 @@ __global__ __launch_bounds__(64 * W) void k_force_sym(SymParams p)
 // wave priorities too: N = 98304 1619, 1560 and 1358 us (0.905 of the FP32
 // peak), 49999 479, 429 and 379, 32768 212 and 188, 24576 141 and 115, 16384
 // 71.7, 62.2 and 54.7, 12000 53 and 43; unequal masses at 98304 1815, 1770
-// and 1541.
-template <bool NEWTON, bool LEAD>
-__global__ __launch_bounds__(64 * kDealWaves, 6) void k_force_sym_deal(SymParams p)
+// and 1541. FOLD: kFoldMaxBlocks below. LEAD (go_sym_deal) runs at most 4
+// workgroups to a CU and holds more registers.
+template <bool NEWTON, bool FOLD, bool LEAD>
+__global__ __launch_bounds__(64 * kDealWaves, LEAD ? 4 : 6) void k_force_sym_deal(SymParams p)
 {
     __shared__ float part[kDealWaves][3][512];
     const int halves = p.split == 4 ? 2 : 1;
@@ -437,7 +438,7 @@ __global__ __launch_bounds__(64 * kDealWaves, 6) void k_force_sym_deal(SymParams
         h = t % p.split;
         upper_pair(p.q0 * (p.q0 - 1) / 2 + t / p.split, P, Q);
     }
-    sym_deal_task<NEWTON, REGS_PINNED, REGS_FREE, LEAD>(p.pm, p.n, p.eps2, p.slots, P, Q, h, p.split, p.more, part);
+    sym_deal_task<NEWTON, REGS_PINNED, REGS_FREE, FOLD, LEAD>(p.pm, p.n, p.eps2, p.slots, P, Q, h, p.split, p.more, part);
 }
 
 constexpr int kReduceGroups = 4;
@@ -901,8 +902,8 @@ const void* sym_kernel()
 
 const void* deal_kernel(bool newton)
 {
-    return newton ? reinterpret_cast<const void*>(&k_force_sym_deal<true, false>)
-                  : reinterpret_cast<const void*>(&k_force_sym_deal<false, false>);
+    return newton ? reinterpret_cast<const void*>(&k_force_sym_deal<true, true, false>)
+                  : reinterpret_cast<const void*>(&k_force_sym_deal<false, true, false>);
 }
 
 template <int A, int W>
@@ -916,6 +917,16 @@ hipError_t go_sym(const ForcePlan& plan, const SymParams& sp, int band_blocks, h
     return hipGetLastError();
 }
 
+// Up to this many blocks the tiles' reactions are folded (nbody_sym.h), and
+// always with a Newton step. A body's force is the exact sum of its block
+// slots, so the fewer there are the more each slot's rounding counts. RMS error
+// on a uniform ball with blocks of 128 (N < 16384) or 256, with blocks of 512
+// unfolded, and folded: N = 13312 4.3e-8, 6.3e-8, 4.0e-8; 16384 5.5e-8, 6.3e-8,
+// 4.3e-8; 32767 4.5e-8, 4.9e-8, 3.8e-8. Folding takes 0 to 2 % of the time up to
+// there (42.4 and 42.5 us, 53.6 and 54.4, 178 and 178) and 1 to 2.5 % of N = 98304,
+// where the error is below that of one wave per block pair without it.
+constexpr int kFoldMaxBlocks = 64;
+
 hipError_t go_sym_deal(const ForcePlan& plan, const SymParams& sp, hipStream_t s)
 {
     const int tasks = sp.npairs * sp.split + sp.diag_tasks, threads = 64 * kDealWaves;
@@ -925,9 +936,10 @@ hipError_t go_sym_deal(const ForcePlan& plan, const SymParams& sp, hipStream_t s
     // those in the first half of their steps go first. N = 16384 54.5 and 52.6 us, unequal masses 60.1 and 57.2,
     // 10241 35.1 and 33.8. With more tasks it keeps the next ones waiting (20480 83.7 and 90.2, 32768 172 and 181).
     const bool lead = tasks <= 4 * 256;
-    if (plan.newton) k_force_sym_deal<true, false><<<tasks, threads, dyn, s>>>(sp);
-    else if (lead) k_force_sym_deal<false, true><<<tasks, threads, dyn, s>>>(sp);
-    else k_force_sym_deal<false, false><<<tasks, threads, dyn, s>>>(sp);
+    if (plan.newton) k_force_sym_deal<true, true, false><<<tasks, threads, dyn, s>>>(sp);
+    else if (lead) k_force_sym_deal<false, true, true><<<tasks, threads, dyn, s>>>(sp);
+    else if (plan.nslices <= kFoldMaxBlocks) k_force_sym_deal<false, true, false><<<tasks, threads, dyn, s>>>(sp);
+    else k_force_sym_deal<false, false, false><<<tasks, threads, dyn, s>>>(sp);
     return hipGetLastError();
 }
 

@@ -764,6 +764,40 @@ __device__ __forceinline__ void sym_pair(const float4* __restrict__ pm, int n, f
     }
 }
 
+// Steps of a rotation after which a tile's running reactions are put away.
+constexpr int kFoldSteps = 8;
+
+// A tile's reactions summed in parts: a running sum over some of the steps is
+// put away in LDS under the lane in which the body began (the rotation goes up
+// by a lane per step), and the next one starts from zero. One wave's own; its
+// LDS operations run in order.
+struct TileSums {
+    float (*total)[512];  // [3][...], 64 of each in use
+
+    __device__ __forceinline__ void set(int began, float& rx, float& ry, float& rz) const
+    {
+        total[0][began] = rx;
+        total[1][began] = ry;
+        total[2][began] = rz;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        rx = ry = rz = 0.f;
+    }
+    // The end of every kFoldSteps steps, after `steps` of them.
+    __device__ __forceinline__ void fold(int steps, float& rx, float& ry, float& rz) const
+    {
+        const int began = (threadIdx.x - steps) & 63;
+        if (steps != kFoldSteps) add_to(began, rx, ry, rz);
+        set(began, rx, ry, rz);
+    }
+    __device__ __forceinline__ void add_to(int began, float& rx, float& ry, float& rz) const
+    {
+        rx = total[0][began] + rx;
+        ry = total[1][began] + ry;
+        rz = total[2][began] + rz;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+};
+
 // Tile t of block P against the block, on one wave with 8 bodies per lane
 // (blocks of 512); the block's 8 tiles together take each of its pairs once.
 // The tile rotates past the lanes as in a block pair and meets the i
@@ -775,8 +809,9 @@ __device__ __forceinline__ void sym_pair(const float4* __restrict__ pm, int n, f
 // same bodies' i sums, and are added there: no LDS, no cross-lane traffic.
 // `which` 0 or 1 takes steps 0..31 or 32..63 alone, -1 all of them. The second
 // half starts half a turn on; the first one's reactions end half a turn from
-// home and are brought there across the wave.
-template <int T, bool EQ>
+// home and are brought there across the wave. With HALVES all of them are two
+// sums, one per half.
+template <int T, bool EQ, bool HALVES>
 __device__ __forceinline__ void sym_diag_tile(const float4* __restrict__ pm, int n, float eps2, int P, int which,
                                               const Lanes<8>& me, const float (&mi)[8], Lanes<8>& acc)
 {
@@ -792,13 +827,20 @@ __device__ __forceinline__ void sym_diag_tile(const float4* __restrict__ pm, int
         sym_diag_step8<T, 0, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
         for (int k = 1; k < 32; ++k) sym_diag_step8<T, 1, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
     }
-    if (which != 0) {
-        sym_diag_step8<T, 2, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
-        for (int k = 33; k < 64; ++k) sym_diag_step8<T, 0, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
-    } else {
+    if (which == 0 || (HALVES && which < 0)) {
         rx = __shfl_xor(rx, 32);
         ry = __shfl_xor(ry, 32);
         rz = __shfl_xor(rz, 32);
+    }
+    if (HALVES && which < 0) {
+        acc.x[T] += rx;
+        acc.y[T] += ry;
+        acc.z[T] += rz;
+        rx = ry = rz = 0.f;
+    }
+    if (which != 0) {
+        sym_diag_step8<T, 2, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
+        for (int k = 33; k < 64; ++k) sym_diag_step8<T, 0, EQ>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2, upper);
     }
     acc.x[T] += rx;
     acc.y[T] += ry;
@@ -814,13 +856,16 @@ constexpr int kDealWaves = 4;
 // this wave takes steps 0..31 (half 0) or 32..63 (half 1), where it starts
 // half a turn on, and leaves the scaled reactions in r: half 0's in the lane
 // half a turn from the body's, half 1's in the body's own lane. With LEAD the
-// first half of the wave's steps runs one priority higher.
-template <bool NEWTON, bool EQ, int REGS, bool LEAD>
+// first half of the wave's steps runs one priority higher. With FOLD a tile's
+// reactions are summed in parts of kFoldSteps steps, 64 roundings each: one
+// running sum over a whole tile takes 512.
+template <bool NEWTON, bool EQ, int REGS, bool LEAD, bool FOLD>
 __device__ __forceinline__ void sym_deal_tiles(const float4* __restrict__ pm, int n, float eps2, int j0, int t0,
                                                int t1, int step, int half, int halves, const Lanes<8>& me,
                                                const float (&mi)[8], Lanes<8>& acc, float* jdst, size_t plane,
-                                               float scale, float (&r)[3])
+                                               float scale, float (&r)[3], const TileSums& sums)
 {
+    static_assert(FOLD || !LEAD, "the leading steps end at a fold");
     const int lane = threadIdx.x & 63;
     float rx = 0.f, ry = 0.f, rz = 0.f;
     for (int tile = t0; tile < t1; tile += step) {
@@ -830,15 +875,24 @@ __device__ __forceinline__ void sym_deal_tiles(const float4* __restrict__ pm, in
         const float4 b = from < n - jbase ? pm[jbase + from] : make_float4(0.f, 0.f, 0.f, 0.f);
         float xj = b.x, yj = b.y, zj = b.z, mj = b.w;
         rx = ry = rz = 0.f;
-        const int steps = halves == 2 ? 32 : 64;
+        const int steps = halves == 2 ? 32 : 64, run = FOLD ? kFoldSteps : steps;
         int k = 0;
         if constexpr (LEAD) {
             const int early = t1 - t0 > 1 ? (tile + step < t1 ? 64 : 0) : steps / 2;
-            for (; k < early; ++k)
-                sym_step<8, NEWTON, EQ, REGS, 1>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+            while (k < early) {
+                for (int m = 0; m < run; ++m)
+                    sym_step<8, NEWTON, EQ, REGS, 1>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+                k += run;
+                if constexpr (FOLD) sums.fold(k, rx, ry, rz);
+            }
         }
-        for (; k < steps; ++k)
-            sym_step<8, NEWTON, EQ, REGS>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+        while (k < steps) {
+            for (int m = 0; m < run; ++m)
+                sym_step<8, NEWTON, EQ, REGS>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+            k += run;
+            if constexpr (FOLD) sums.fold(k, rx, ry, rz);
+        }
+        if constexpr (FOLD) sums.add_to((lane - steps) & 63, rx, ry, rz);  // (to zero)
         rx *= scale;
         ry *= scale;
         rz *= scale;
@@ -859,12 +913,13 @@ __device__ __forceinline__ void sym_deal_tiles(const float4* __restrict__ pm, in
 // and two halves on every wave, all 64 steps or those of one half (halves = 2).
 // With a Newton step (whose pair chains are not in assembly): sub-blocks w and
 // w + 4 one-sided, against the block or one half of it.
-template <bool NEWTON>
+template <bool NEWTON, bool FOLD>
 __device__ __forceinline__ void sym_deal_diag(const float4* __restrict__ pm, int n, float eps2, int P, int wave,
                                               int half, int halves, bool eq, const Lanes<8>& me, const float (&mi)[8],
                                               Lanes<8>& acc)
 {
     if constexpr (NEWTON) {
+        // (in runs of 64 bodies, as many terms as the tiles' folds)
         const int j0 = P * 512 + half * 256, len = min(n - j0, halves == 2 ? 256 : 512);
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
@@ -873,21 +928,23 @@ __device__ __forceinline__ void sym_deal_diag(const float4* __restrict__ pm, int
             one.x[0] = me.x[u];
             one.y[0] = me.y[u];
             one.z[0] = me.z[u];
-            zero<1>(sum);
-            sweep_sgpr<1, true>(pm + j0, len, eps2, one, sum);
-            acc.x[u] = sum.x[0];
-            acc.y[u] = sum.y[0];
-            acc.z[u] = sum.z[0];
+            for (int c = 0; c < len; c += 64) {
+                zero<1>(sum);
+                sweep_sgpr<1, true>(pm + j0 + c, min(len - c, 64), eps2, one, sum);
+                acc.x[u] += sum.x[0];
+                acc.y[u] += sum.y[0];
+                acc.z[u] += sum.z[0];
+            }
         }
     } else {
         const int which = halves == 2 ? half : -1;
         auto tiles = [&](auto lo, auto hi) {
             if (eq) {
-                sym_diag_tile<lo, true>(pm, n, eps2, P, which, me, mi, acc);
-                sym_diag_tile<hi, true>(pm, n, eps2, P, which, me, mi, acc);
+                sym_diag_tile<lo, true, FOLD>(pm, n, eps2, P, which, me, mi, acc);
+                sym_diag_tile<hi, true, FOLD>(pm, n, eps2, P, which, me, mi, acc);
             } else {
-                sym_diag_tile<lo, false>(pm, n, eps2, P, which, me, mi, acc);
-                sym_diag_tile<hi, false>(pm, n, eps2, P, which, me, mi, acc);
+                sym_diag_tile<lo, false, FOLD>(pm, n, eps2, P, which, me, mi, acc);
+                sym_diag_tile<hi, false, FOLD>(pm, n, eps2, P, which, me, mi, acc);
             }
         };
         switch (wave) {
@@ -905,7 +962,7 @@ __device__ __forceinline__ void sym_deal_diag(const float4* __restrict__ pm, int
 // the diagonal block, or with split 4 half h of it. Task h's i sides go `more`
 // elements past task h - 1's. `part` is the workgroup's LDS. EQ_REGS, GEN_REGS:
 // the steps' registers on one mass and otherwise.
-template <bool NEWTON, int EQ_REGS, int GEN_REGS, bool LEAD = false>
+template <bool NEWTON, int EQ_REGS, int GEN_REGS, bool FOLD = false, bool LEAD = false>
 __device__ __forceinline__ void sym_deal_task(const float4* __restrict__ pm, int n, float eps2, const SlotMap& slots,
                                               int P, int Q, int h, int split, size_t more, float (*part)[3][512])
 {
@@ -929,10 +986,11 @@ __device__ __forceinline__ void sym_deal_task(const float4* __restrict__ pm, int
         same &= (i < n) & (q.w == m0);
     }
     zero<8>(acc);
+    const TileSums sums{part[wave]};
     float scale = 1.0f;
     if (diag) {
         const bool eq = !NEWTON && __builtin_amdgcn_ballot_w64(!same) == 0;
-        sym_deal_diag<NEWTON>(pm, n, eps2, P, wave, h, halves, eq, me, mi, acc);
+        sym_deal_diag<NEWTON, FOLD>(pm, n, eps2, P, wave, h, halves, eq, me, mi, acc);
         if (eq) scale = m0;
     } else {
         // tiles t0, t0 + W, ... < t1 of block Q
@@ -949,11 +1007,11 @@ __device__ __forceinline__ void sym_deal_task(const float4* __restrict__ pm, int
         const int out = t0 * 64;
         float r[3];
         if (eq)
-            sym_deal_tiles<NEWTON, true, EQ_REGS, LEAD>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst,
-                                                  plane, m0, r);
+            sym_deal_tiles<NEWTON, true, EQ_REGS, LEAD, FOLD>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi, acc,
+                                                        jdst, plane, m0, r, sums);
         else
-            sym_deal_tiles<NEWTON, false, GEN_REGS, LEAD>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi, acc, jdst,
-                                                    plane, 1.0f, r);
+            sym_deal_tiles<NEWTON, false, GEN_REGS, LEAD, FOLD>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi,
+                                                          acc, jdst, plane, 1.0f, r, sums);
         if (halves == 2) {
             // the first half's reactions are half a turn from home; the second wave adds both in order
             if (half == 0) {
