@@ -74,6 +74,26 @@ constexpr int kSymSlotsTarget = 512;
 // blocks of 512, whose 36 block pairs leave most CUs idle; at N = 6000 26.1
 // against 22.5.
 constexpr size_t kSmallSymN = 5120;
+// A share of the block pairs with less work than this per share takes blocks
+// of 128 bodies below N = 16384 and of 256 below 32768 all the same: a share's
+// pairs are one task each, and a block pair of 512 that has its CU to itself takes
+// 48 us. The busiest share's microseconds with the fine blocks and with 512:
+// N = 6000 of 2 23.5 and 51.5, 8192 of 2 29 and 50, of 8 22 and 50, 12000 of 2 42
+// and 52, 16384 of 8 47 and 51, of 4 48 and 51, 24576 of 8 49 and 52; and past
+// it 16384 of 2 73 and 58, 24576 of 4 71 and 60, 32767 of 8 72 and 61.
+// The fine blocks' slots have to fit a budget the caller gave: in several
+// column bands they lose (16384 of 4 within 1 MiB 174 and 98).
+constexpr double kFineShareWork = 1.0e8;
+
+bool fine_share(size_t N, int shares, size_t slot_bytes, int* ipl)
+{
+    if (shares <= 1 || N >= 32768 || (double)N * (double)N >= kFineShareWork * shares) return false;
+    const int fine = N < 16384 ? 2 : 4;
+    const size_t nb = (N + 64 * fine - 1) / (64 * fine);
+    if (slot_bytes > 0 && 12 * nb * nb * 64 * fine > slot_bytes) return false;
+    *ipl = fine;
+    return true;
+}
 
 // Bodies up to which NBODY_HIP_AUTO evaluates a whole system in one launch
 // over the whole j range (nbody_tile.h) instead of by the symmetric plan. The
@@ -114,7 +134,7 @@ void lds_shape(size_t N, size_t n, int cus, int* ipl, int* jslice)
 // Default decomposition: enough blocks for ~48 waves per SIMD (the dispatcher
 // balances them across the 256 CUs), j slices of at least 1024 bodies in
 // multiples of 256.
-ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip_options* opt)
+ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip_options* opt, int shares)
 {
     ForcePlan p;
     p.variant = variant;
@@ -140,6 +160,8 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
         if (!shape_given && N < kSmallSymN) {
             p.ipl = 2;
             p.jslice = 128;
+        } else if (!shape_given && fine_share(N, shares, opt ? opt->slot_bytes : 0, &p.ipl)) {
+            p.jslice = 64 * p.ipl;
         } else if (opt && opt->jslice > 0) {
             p.jslice = opt->jslice;
         } else if (p.ipl == 2) {
@@ -276,7 +298,7 @@ int validate_plan(const ForcePlan& p, size_t N)
     return OK;
 }
 
-int make_plan(DeviceState& d, size_t N, size_t n, const nbody_hip_options* opt, ForcePlan* plan)
+int make_plan(DeviceState& d, size_t N, size_t n, const nbody_hip_options* opt, ForcePlan* plan, int shares)
 {
     const int requested = opt ? opt->variant : NBODY_HIP_AUTO;
     const int variant = requested == NBODY_HIP_AUTO ? auto_variant(N, n, opt) : requested;
@@ -284,7 +306,7 @@ int make_plan(DeviceState& d, size_t N, size_t n, const nbody_hip_options* opt, 
         set_error("unknown variant %d", requested);
         return E_ARG;
     }
-    ForcePlan p = default_plan(variant, N, n, d.cus, opt);
+    ForcePlan p = default_plan(variant, N, n, d.cus, opt, shares);
     const bool explicit_shape = opt && (opt->i_per_lane > 0 || opt->jslice > 0 || opt->waves_per_simd > 0);
     if (!explicit_shape) {
         auto it = d.tuned.find(tune_key(opt, N, n));
@@ -637,7 +659,7 @@ int nbody_hip_force_pair_share(double* force64, const float* posMass, float soft
     else o.compensated = -1;
     o.variant = NBODY_HIP_SYMMETRIC;
     ForcePlan plan;
-    if (int r = make_plan(*d, N, N, &o, &plan)) return r;
+    if (int r = make_plan(*d, N, N, &o, &plan, shares)) return r;
     symmetric_share_columns(plan.nslices, share, shares, &plan.col0, &plan.col1);
     return run_force(*d, plan, nullptr, posMass, softeningSquared, N, 0, N, static_cast<hipStream_t>(stream), nullptr,
                      true, force64);

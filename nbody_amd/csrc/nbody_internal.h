@@ -128,8 +128,9 @@ extern std::mutex g_mutex;
 void set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 int device_state(DeviceState** out);
 int round_up(int v, int m);
-ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip_options* opt);
-int make_plan(DeviceState& d, size_t N, size_t n, const nbody_hip_options* opt, ForcePlan* plan);
+// (`shares`: of how many shares of the block pairs the plan is to run one)
+ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip_options* opt, int shares = 1);
+int make_plan(DeviceState& d, size_t N, size_t n, const nbody_hip_options* opt, ForcePlan* plan, int shares = 1);
 // The plan as options (nbody_hip_plan, nbody_hip_system_plan).
 void describe_plan(const ForcePlan& p, nbody_hip_options* out);
 int check_args(const void* force, const void* pm, size_t N, size_t base, size_t n);
