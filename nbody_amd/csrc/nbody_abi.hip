@@ -54,8 +54,6 @@ int device_state(DeviceState** out)
         snprintf(d.arch, sizeof d.arch, "%s", prop.gcnArchName);
         HIP_TRY(hipEventCreate(&d.ev0));
         HIP_TRY(hipEventCreate(&d.ev1));
-        HIP_TRY(hipEventCreateWithFlags(&d.one0, hipEventDisableSystemFence));
-        HIP_TRY(hipEventCreateWithFlags(&d.one1, hipEventReleaseToSystem));
         HIP_TRY(hipEventCreateWithFlags(&d.partial_done, hipEventDisableTiming));
         d.init = true;
     }
@@ -350,8 +348,7 @@ int check_args(const void* force, const void* pm, size_t N, size_t base, size_t 
 
 // Queue one force evaluation on `stream` (caller holds g_mutex).
 int run_force(DeviceState& d, const ForcePlan& plan, float* force, const float* pm, float eps2, size_t N, size_t base,
-              size_t n, hipStream_t stream, Buffer* own, bool timed, double* force64, const StepParams* step,
-              hipEvent_t done)
+              size_t n, hipStream_t stream, Buffer* own, bool timed, double* force64, const StepParams* step)
 {
     Buffer& buf = own ? *own : d.partial;
     if (plan.variant == VAR_SYMMETRIC && (base != 0 || n != N)) {
@@ -403,7 +400,7 @@ int run_force(DeviceState& d, const ForcePlan& plan, float* force, const float* 
         after = d.timer_events[d.timer_used].second;
         d.timer_used++;
     }
-    HIP_TRY(launch_force(plan, p, stream, before, after, done));
+    HIP_TRY(launch_force(plan, p, stream, before, after));
     if (shared) {
         HIP_TRY(hipEventRecord(d.partial_done, stream));
         d.partial_stream = stream;
@@ -514,22 +511,20 @@ float timed_force(const nbody_hip_options* opt, float* force, const float* pm, f
         set_error("cannot allocate %zu bytes of slice scratch", bytes);
         return 0.0f;
     }
-    // A small system's call is mostly the two markers around its kernel: one
-    // launch that completes its own end event behind a plain start marker
-    // takes 10.7 us instead of 15.5 (empty kernel). With two launches the
-    // gain is under 2 us of 70 and more, and the ordinary pair stays.
-    const bool one = plan.li > 0;
-    const hipEvent_t start = one ? d->one0 : d->ev0, end = one ? d->one1 : d->ev1;
-    if (hipError_t e = hipEventRecord(start, nullptr); e != hipSuccess) {
+    // A small system's call is mostly the two markers around its kernel. An end
+    // event attached to the launch itself takes 2.5 to 3 us off the call (N =
+    // 1000 16.0 and 13.1 us), but leaves the stream unfinished as the runtime sees
+    // it: the caller's next synchronisation or copy then takes 8 us longer (3.3
+    // and 11.4 us). So the ordinary pair.
+    if (hipError_t e = hipEventRecord(d->ev0, nullptr); e != hipSuccess) {
         set_error("timing failed: %s", hipGetErrorString(e));
         return 0.0f;
     }
-    if (run_force(*d, plan, force, pm, eps2, N, 0, N, nullptr, nullptr, true, nullptr, nullptr, one ? end : nullptr))
-        return 0.0f;
+    if (run_force(*d, plan, force, pm, eps2, N, 0, N, nullptr)) return 0.0f;
     float ms = 0.0f;
-    hipError_t e = one ? hipSuccess : hipEventRecord(end, nullptr);
-    if (e == hipSuccess) e = hipEventSynchronize(end);
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms, start, end);
+    hipError_t e = hipEventRecord(d->ev1, nullptr);
+    if (e == hipSuccess) e = hipEventSynchronize(d->ev1);
+    if (e == hipSuccess) e = hipEventElapsedTime(&ms, d->ev0, d->ev1);
     if (e != hipSuccess) {
         set_error("timing failed: %s", hipGetErrorString(e));
         return 0.0f;

@@ -90,10 +90,6 @@ struct DeviceState {
     int clock_khz = 0;
     char arch[64] = {0};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    // The same pair around a single launch: a start marker that leaves the
-    // caches alone, and an end that the launch itself completes, with a
-    // system-scope release (`force` may be host memory).
-    hipEvent_t one0 = nullptr, one1 = nullptr;
     Buffer partial;   // FP32 slice partials, shared by the calls that bring no scratch of their own
     // The last queued use of `partial`: its stream and an event recorded
     // after its kernels. A call on another stream waits for that event
@@ -145,7 +141,7 @@ int check_args(const void* force, const void* pm, size_t N, size_t base, size_t 
 // step (a plan that fuses_step) the last launch also integrates the bodies.
 int run_force(DeviceState& d, const ForcePlan& plan, float* force, const float* pm, float eps2, size_t N, size_t base,
               size_t n, hipStream_t stream, Buffer* own = nullptr, bool timed = true, double* force64 = nullptr,
-              const StepParams* step = nullptr, hipEvent_t done = nullptr);
+              const StepParams* step = nullptr);
 
 }  // namespace detail
 }  // namespace nbody

@@ -98,11 +98,9 @@ size_t plan_scratch_bytes(const ForcePlan& plan, int ni);
 
 // Queue the force kernel and, for sliced plans, the slice reduction on
 // `stream`. When before/after are given they are recorded on the stream
-// around the force kernel alone. With a one-launch plan (plan.li > 0) the
-// launch itself completes `done`, with no marker behind it; other plans leave
-// it alone.
+// around the force kernel alone.
 hipError_t launch_force(const ForcePlan& plan, const ForceParams& p, hipStream_t stream,
-                        hipEvent_t before = nullptr, hipEvent_t after = nullptr, hipEvent_t done = nullptr);
+                        hipEvent_t before = nullptr, hipEvent_t after = nullptr);
 
 // integrateGravitation (src/nbody.cu:158-236) on float4 records.
 hipError_t launch_integrate(float4* posMass, float4* velInvMass, const float4* force, float dt,

@@ -19,8 +19,6 @@
 #include "nbody_sym.h"
 #include "nbody_tile.h"
 
-#include <hip/hip_ext.h>
-
 #include <algorithm>
 #include <cmath>
 #include <map>
@@ -842,27 +840,26 @@ hipError_t go_family(const ForcePlan& plan, dim3 g, hipStream_t s, const ForcePa
 }
 
 template <int LI, int I, bool F64 = false>
-void go_tile_shape(dim3 g, hipStream_t s, const ForceParams& p, hipEvent_t done)
+void go_tile_shape(dim3 g, hipStream_t s, const ForceParams& p)
 {
     const auto kernel = p.step.vm ? k_force_tile<LI, I, true, F64> : k_force_tile<LI, I, false, F64>;
-    if (done) hipExtLaunchKernelGGL(kernel, g, dim3(kTileThreads), 0, s, nullptr, done, 0, p);
-    else kernel<<<g, kTileThreads, 0, s>>>(p);
+    kernel<<<g, kTileThreads, 0, s>>>(p);
 }
 
-hipError_t go_tile(const ForcePlan& plan, dim3 g, hipStream_t s, const ForceParams& p, hipEvent_t done)
+hipError_t go_tile(const ForcePlan& plan, dim3 g, hipStream_t s, const ForceParams& p)
 {
     switch (plan.li * 100 + plan.ipl + (plan.acc64 ? 10000 : 0)) {
-    case 10401: go_tile_shape<4, 1, true>(g, s, p, done); break;
-    case 10402: go_tile_shape<4, 2, true>(g, s, p, done); break;
-    case 10802: go_tile_shape<8, 2, true>(g, s, p, done); break;
-    case 401: go_tile_shape<4, 1>(g, s, p, done); break;
-    case 402: go_tile_shape<4, 2>(g, s, p, done); break;
-    case 403: go_tile_shape<4, 3>(g, s, p, done); break;
-    case 802: go_tile_shape<8, 2>(g, s, p, done); break;
-    case 803: go_tile_shape<8, 3>(g, s, p, done); break;
-    case 804: go_tile_shape<8, 4>(g, s, p, done); break;
-    case 805: go_tile_shape<8, 5>(g, s, p, done); break;
-    case 806: go_tile_shape<8, 6>(g, s, p, done); break;
+    case 10401: go_tile_shape<4, 1, true>(g, s, p); break;
+    case 10402: go_tile_shape<4, 2, true>(g, s, p); break;
+    case 10802: go_tile_shape<8, 2, true>(g, s, p); break;
+    case 401: go_tile_shape<4, 1>(g, s, p); break;
+    case 402: go_tile_shape<4, 2>(g, s, p); break;
+    case 403: go_tile_shape<4, 3>(g, s, p); break;
+    case 802: go_tile_shape<8, 2>(g, s, p); break;
+    case 803: go_tile_shape<8, 3>(g, s, p); break;
+    case 804: go_tile_shape<8, 4>(g, s, p); break;
+    case 805: go_tile_shape<8, 5>(g, s, p); break;
+    case 806: go_tile_shape<8, 6>(g, s, p); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1141,7 +1138,7 @@ size_t plan_scratch_bytes(const ForcePlan& plan, int ni)
 }
 
 hipError_t launch_force(const ForcePlan& plan, const ForceParams& p, hipStream_t stream, hipEvent_t before,
-                        hipEvent_t after, hipEvent_t done)
+                        hipEvent_t after)
 {
     if (p.ni <= 0 || p.n <= 0) return hipSuccess;
     if (before) {
@@ -1161,7 +1158,7 @@ hipError_t launch_force(const ForcePlan& plan, const ForceParams& p, hipStream_t
     }
     if (plan.li > 0) {
         const dim3 g((p.ni + plan.li * plan.ipl - 1) / (plan.li * plan.ipl));
-        e = go_tile(plan, g, stream, p, done);
+        e = go_tile(plan, g, stream, p);
         if (e == hipSuccess && after) e = hipEventRecord(after, stream);
         return e;
     }
