@@ -136,10 +136,12 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
 {
     ForcePlan p;
     p.variant = variant;
+    p.cus = cus;
     p.newton = opt && opt->newton > 0;
     const int comp_opt = opt ? opt->compensated : -1;
     p.comp = comp_opt < 0 ? (N > 65536) : comp_opt > 0;
     p.acc64 = comp_opt == 2;
+    const double chips = std::max(cus, 1) / 256.0;  // of the chip that the times below were measured on
     if (variant == VAR_SYMMETRIC && p.acc64) {
         // one wave per block pair, 4 (or 8) bodies per lane, blocks of 64 per lane
         p.ipl = (opt && opt->i_per_lane > 0) ? opt->i_per_lane : 4;
@@ -188,8 +190,8 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
         // launches and slice sum (sliced and in one launch: 1000 of 4096 bodies 19.5 and 4.6 us, 8192 of
         // 16384 45 and 41, 10000 of 20000 67 and 59, 8000 of 33588 85 and 80, 6144 of 49152 88 and 90, 8192 of
         // 65536 141 and 152, 32768 of 65536 505 and 580)
-        const double sliced = std::max(0.225e-6 * (double)n * (double)N, 0.044 * p.jslice * p.ipl) + 15.5;
-        if (tile_allowed(N, n, opt) && tile_shape(N, n, false, &li, &ipl) < sliced) {
+        const double sliced = std::max(0.225e-6 * (double)n * (double)N / chips, 0.044 * p.jslice * p.ipl) + 15.5;
+        if (tile_allowed(N, n, opt) && tile_shape(N, n, false, cus, &li, &ipl) < sliced) {
             p.li = li;
             p.ipl = ipl;
             p.jslice = (int)N;
@@ -224,9 +226,9 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
         // through its slice, and 16 us of launches and slice sum if there are slices (8192 of 16384 bodies 74
         // and, in one launch, 70 us; 8192 of 65536 stay sliced: 231)
         const double sliced =
-            std::max(0.41e-6 * (double)n * (double)N, 0.0445 * p.jslice) + (p.nslices > 1 ? 16.0 : 3.0);
+            std::max(0.41e-6 * (double)n * (double)N / chips, 0.0445 * p.jslice) + (p.nslices > 1 ? 16.0 : 3.0);
         int li, ipl;
-        if (tile_shape(N, n, true, &li, &ipl) < sliced) {
+        if (tile_shape(N, n, true, cus, &li, &ipl) < sliced) {
             p.li = li;
             p.ipl = ipl;
             p.jslice = (int)N;

@@ -32,6 +32,7 @@ struct ForcePlan {
     bool acc64 = false; // every term added in FP64, partial sums kept in FP64 (LDS and symmetric)
     bool newton = false;
     int occ = 0;        // symmetric: waves per SIMD cap (0 = register-limited occupancy)
+    int cus = 256;      // compute units of the device it is for
     size_t band_cap = 0;  // symmetric: bytes of slot partials one band may keep (0 = kSymBandCap)
     int col0 = 0, col1 = 0;  // symmetric: the column blocks [col0, col1) of the block triangle (0, 0 = all)
 };
@@ -82,9 +83,14 @@ struct ForceParams {
 bool fuses_step(const ForcePlan& plan);
 bool step_needs_buffer(const ForcePlan& plan);
 
-// The shape of the one-launch kernel that ends first for ni of n bodies;
-// returns its estimated microseconds.
-double tile_shape(size_t n, size_t ni, bool acc64, int* li, int* ipl);
+// The shape of the one-launch kernel that ends first for ni of n bodies on
+// `cus` compute units; returns its estimated microseconds.
+double tile_shape(size_t n, size_t ni, bool acc64, int cus, int* li, int* ipl);
+
+// Whether a symmetric launch of `tasks` four-wave workgroups (blocks of 512)
+// has them all resident at once, so that the first halves of their steps go
+// first (k_force_sym_deal's LEAD).
+bool deal_leads(const ForcePlan& plan, int tasks);
 
 // Whether (i per lane, block size) is a compiled symmetric shape.
 bool symmetric_shape_ok(int ipl, int block);

@@ -897,10 +897,12 @@ const void* sym_kernel()
     return reinterpret_cast<const void*>(&k_force_sym<A, W, NEWTON>);
 }
 
-const void* deal_kernel(bool newton)
+const void* deal_kernel(bool newton, bool fold, bool lead)
 {
     return newton ? reinterpret_cast<const void*>(&k_force_sym_deal<true, true, false>)
-                  : reinterpret_cast<const void*>(&k_force_sym_deal<false, true, false>);
+           : lead ? reinterpret_cast<const void*>(&k_force_sym_deal<false, true, true>)
+           : fold ? reinterpret_cast<const void*>(&k_force_sym_deal<false, true, false>)
+                  : reinterpret_cast<const void*>(&k_force_sym_deal<false, false, false>);
 }
 
 template <int A, int W>
@@ -927,15 +929,12 @@ constexpr int kFoldMaxBlocks = 64;
 hipError_t go_sym_deal(const ForcePlan& plan, const SymParams& sp, hipStream_t s)
 {
     const int tasks = sp.npairs * sp.split + sp.diag_tasks, threads = 64 * kDealWaves;
-    const void* k = deal_kernel(plan.newton);
-    const size_t dyn = plan.occ > 0 ? lds_for_occupancy(k, threads, plan.occ) : 0;
-    // With at most 4 tasks to a CU every task starts at once, and the waves of a SIMD had better end together:
-    // those in the first half of their steps go first. N = 16384 54.5 and 52.6 us, unequal masses 60.1 and 57.2,
-    // 10241 35.1 and 33.8. With more tasks it keeps the next ones waiting (20480 83.7 and 90.2, 32768 172 and 181).
-    const bool lead = tasks <= 4 * 256;
+    const bool lead = deal_leads(plan, tasks), fold = plan.nslices <= kFoldMaxBlocks;
+    const size_t dyn =
+        plan.occ > 0 ? lds_for_occupancy(deal_kernel(plan.newton, fold, false), threads, plan.occ) : 0;
     if (plan.newton) k_force_sym_deal<true, true, false><<<tasks, threads, dyn, s>>>(sp);
     else if (lead) k_force_sym_deal<false, true, true><<<tasks, threads, dyn, s>>>(sp);
-    else if (plan.nslices <= kFoldMaxBlocks) k_force_sym_deal<false, true, false><<<tasks, threads, dyn, s>>>(sp);
+    else if (fold) k_force_sym_deal<false, true, false><<<tasks, threads, dyn, s>>>(sp);
     else k_force_sym_deal<false, false, false><<<tasks, threads, dyn, s>>>(sp);
     return hipGetLastError();
 }
@@ -961,7 +960,7 @@ int deal_diag_tasks(int split) { return split == 4 ? 2 : 1; }
 
 // Tasks per block pair of a plan's k_force_sym_deal launch, 1, 2 or 4; only in
 // a single band over every column. More tasks put more waves on a SIMD and
-// end the launch more evenly: the fullest CU gets ceil(tasks / 256) of them,
+// end the launch more evenly: the fullest CU gets ceil(tasks / CUs) of them,
 // each 1 / split of a pair, and a pair takes 18.3 us of a CU whose SIMDs hold
 // 5 waves or more (few_waves times that with fewer), a task 1.3 us besides.
 // And each further task keeps its i sides in more slot rows, which the slot
@@ -986,7 +985,7 @@ int sym_split(const ForcePlan& plan, size_t nbands)
         if (split > 1 && split * band_floats(0, plan.nslices, 512) * sizeof(float) > cap) break;
         const double tasks = 0.5 * nb * (nb - 1.0) * split + nb * deal_diag_tasks(split);
         const double rows = nb + 0.5 * (nb - 1.0) * (split - 1);
-        const double fullest = std::ceil(tasks / 256.0);
+        const double fullest = std::ceil(tasks / std::max(plan.cus, 1));
         const double us = fullest * (18.3 / split + 1.3) * (fullest < 5.0 ? few_waves[(int)fullest] : 1.0) +
                           rows * nb * 512.0 * 12.0 / 8.0e6;
         if (split == 1 || us < least) {
@@ -1040,9 +1039,9 @@ constexpr TileShape kTileShapes[] = {{4, 1, .242}, {4, 2, .191}, {4, 3, .175}, {
 
 }  // namespace
 
-double tile_shape(size_t n, size_t ni, bool acc64, int* li, int* ipl)
+double tile_shape(size_t n, size_t ni, bool acc64, int cu_count, int* li, int* ipl)
 {
-    constexpr size_t cus = 256;
+    const size_t cus = (size_t)std::max(cu_count, 1);
     double least = 0.0;
     for (const TileShape& s : kTileShapes) {
         if (acc64 && s.ipl > 2) continue;  // (built up to 2)
@@ -1060,6 +1059,15 @@ double tile_shape(size_t n, size_t ni, bool acc64, int* li, int* ipl)
         }
     }
     return least / 2400.0 + 2.1;
+}
+
+// With at most 4 tasks to a CU every task starts at once, and the waves of a SIMD had better end together: those in the
+// first half of their steps go first. N = 16384 54.5 and 52.6 us, unequal masses
+// 60.1 and 57.2, 10241 35.1 and 33.8. With more tasks it keeps the next ones
+// waiting (20480 83.7 and 90.2, 32768 172 and 181).
+bool deal_leads(const ForcePlan& plan, int tasks)
+{
+    return !plan.newton && tasks <= 4 * std::max(plan.cus, 1);
 }
 
 bool fuses_step(const ForcePlan& plan) { return plan.li > 0 || (plan.variant == VAR_SYMMETRIC && !plan.acc64); }
@@ -1082,7 +1090,7 @@ int symmetric_natural_occupancy(const ForcePlan& plan)
     if (plan.ipl == 4)
         return w == 1 ? natural_occupancy<4, 1>(plan.newton) : w == 2 ? natural_occupancy<4, 2>(plan.newton)
                                                                       : natural_occupancy<4, 4>(plan.newton);
-    if (w == 1) return blocks_per_cu(deal_kernel(plan.newton), 64 * kDealWaves, 0) * kDealWaves / 4;
+    if (w == 1) return blocks_per_cu(deal_kernel(plan.newton, false, false), 64 * kDealWaves, 0) * kDealWaves / 4;
     return w == 2 ? natural_occupancy<8, 2>(plan.newton) : natural_occupancy<8, 4>(plan.newton);
 }
 

@@ -41,3 +41,27 @@ def test_lds_slices_of_the_largest_systems(probe, n_all):
                                                                for n in counts])):
         assert 1 <= jslice <= n_all and ipl in (1, 2) and (li == 0 or nslices == 1), (n, jslice)
         assert nslices == -(-n_all // jslice) and nslices <= 65535, (n, jslice, nslices)
+
+
+@pytest.mark.parametrize("acc64", [0, 1])
+def test_one_launch_shape_follows_the_cu_count(probe, acc64):
+    """A quarter of the compute units with a quarter of the i bodies has the same
+    number of workgroups per unit, so the same shape (480 bodies are whole
+    workgroups of every shape)."""
+    cases = [(n, 480 * k) for n in (1000, 4096, 8192, 30000) for k in range(1, 9)]
+    whole = probe(*[f"tile {n} {4 * ni} {acc64} 256" for n, ni in cases])
+    quarter = probe(*[f"tile {n} {ni} {acc64} 64" for n, ni in cases])
+    assert whole == quarter
+    assert len({tuple(s) for s in whole}) > 1
+
+
+def test_tasks_per_block_pair_follow_the_cu_count(probe):
+    """Block pairs are split to fill the chip: not where a small one is full anyway."""
+    small, large, small_chip = [r[0] for r in probe("tasks 12288 256", "tasks 98304 256", "tasks 12288 16")]
+    assert small > 1 and large == 1 and small_chip == 1
+
+
+def test_lead_needs_every_task_resident(probe):
+    """Four workgroups to a compute unit."""
+    lines = {"1024 256 0": 1, "1025 256 0": 0, "128 32 0": 1, "129 32 0": 0}
+    assert [r[0] for r in probe(*[f"lead {k}" for k in lines])] == list(lines.values())
