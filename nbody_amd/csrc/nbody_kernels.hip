@@ -931,7 +931,7 @@ hipError_t go_sym_deal(const ForcePlan& plan, const SymParams& sp, hipStream_t s
     const int tasks = sp.npairs * sp.split + sp.diag_tasks, threads = 64 * kDealWaves;
     const bool lead = deal_leads(plan, tasks), fold = plan.nslices <= kFoldMaxBlocks;
     const size_t dyn =
-        plan.occ > 0 ? lds_for_occupancy(deal_kernel(plan.newton, fold, false), threads, plan.occ) : 0;
+        plan.occ > 0 ? lds_for_occupancy(deal_kernel(plan.newton, fold, lead), threads, plan.occ) : 0;
     if (plan.newton) k_force_sym_deal<true, true, false><<<tasks, threads, dyn, s>>>(sp);
     else if (lead) k_force_sym_deal<false, true, true><<<tasks, threads, dyn, s>>>(sp);
     else if (fold) k_force_sym_deal<false, true, false><<<tasks, threads, dyn, s>>>(sp);
@@ -1061,13 +1061,15 @@ double tile_shape(size_t n, size_t ni, bool acc64, int cu_count, int* li, int* i
     return least / 2400.0 + 2.1;
 }
 
-// With at most 4 tasks to a CU every task starts at once, and the waves of a SIMD had better end together: those in the
+// With at most 4 tasks to a CU (fewer if the plan caps its waves) every task
+// starts at once, and the waves of a SIMD had better end together: those in the
 // first half of their steps go first. N = 16384 54.5 and 52.6 us, unequal masses
 // 60.1 and 57.2, 10241 35.1 and 33.8. With more tasks it keeps the next ones
 // waiting (20480 83.7 and 90.2, 32768 172 and 181).
 bool deal_leads(const ForcePlan& plan, int tasks)
 {
-    return !plan.newton && tasks <= 4 * std::max(plan.cus, 1);
+    const int per_cu = plan.occ > 0 ? std::min(4, plan.occ) : 4;
+    return !plan.newton && tasks <= per_cu * std::max(plan.cus, 1);
 }
 
 bool fuses_step(const ForcePlan& plan) { return plan.li > 0 || (plan.variant == VAR_SYMMETRIC && !plan.acc64); }

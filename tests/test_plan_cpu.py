@@ -62,6 +62,7 @@ def test_tasks_per_block_pair_follow_the_cu_count(probe):
 
 
 def test_lead_needs_every_task_resident(probe):
-    """Four workgroups to a compute unit."""
-    lines = {"1024 256 0": 1, "1025 256 0": 0, "128 32 0": 1, "129 32 0": 0}
+    """Four workgroups to a compute unit, or as many as the plan's cap leaves."""
+    lines = {"1024 256 0": 1, "1025 256 0": 0, "512 256 2": 1, "513 256 2": 0, "768 256 3": 1, "769 256 3": 0,
+             "1024 256 6": 1, "1025 256 6": 0, "128 32 0": 1, "129 32 0": 0}
     assert [r[0] for r in probe(*[f"lead {k}" for k in lines])] == list(lines.values())
