@@ -72,18 +72,19 @@ __device__ __forceinline__ void body_body(float xj, float yj, float zj, float mj
 // this one. JC is the register class of the j body: "v" (from LDS or a DPP
 // tile) or "s" (from scalar loads).
 #define NBODY_BODY_CHAIN(NAME, JC)                                                                     \
+    template <bool PRIO>                                                                               \
     __device__ __forceinline__ void NAME(float xj, float yj, float zj, float mj, float xi, float yi,   \
                                          float zi, float eps2, float& ax, float& ay, float& az)        \
     {                                                                                                  \
         float dx, dy, dz, s, t;                                                                        \
-        asm volatile("s_setprio 0\n"                                                                   \
+        asm volatile(".if %[prio]\n s_setprio 0\n .endif\n"                                            \
                      "v_sub_f32 %[dx], %[xj], %[xi]\n"                                                 \
                      "v_sub_f32 %[dy], %[yj], %[yi]\n"                                                 \
                      "v_sub_f32 %[dz], %[zj], %[zi]\n"                                                 \
                      "v_fma_f32 %[s], %[dx], %[dx], %[eps]\n"                                          \
                      "v_fmac_f32 %[s], %[dy], %[dy]\n"                                                 \
                      "v_fmac_f32 %[s], %[dz], %[dz]\n"                                                 \
-                     "s_setprio 1\n"                                                                   \
+                     ".if %[prio]\n s_setprio 1\n .endif\n"                                            \
                      "v_rsq_f32 %[s], %[s]\n"                                                          \
                      "s_nop 0\n"                                                                       \
                      "v_mul_f32 %[t], %[mj], %[s]\n"                                                   \
@@ -95,7 +96,7 @@ __device__ __forceinline__ void body_body(float xj, float yj, float zj, float mj
                      : [ax] "+v"(ax), [ay] "+v"(ay), [az] "+v"(az), [dx] "=&v"(dx), [dy] "=&v"(dy),     \
                        [dz] "=&v"(dz), [s] "=&v"(s), [t] "=&v"(t)                                      \
                      : [xj] JC(xj), [yj] JC(yj), [zj] JC(zj), [mj] JC(mj), [xi] "v"(xi), [yi] "v"(yi),  \
-                       [zi] "v"(zi), [eps] "s"(eps2));                                                 \
+                       [zi] "v"(zi), [eps] "s"(eps2), [prio] "n"(PRIO ? 1 : 0));                       \
     }
 NBODY_BODY_CHAIN(body_body_chain_v, "v")
 NBODY_BODY_CHAIN(body_body_chain_s, "s")
@@ -109,18 +110,19 @@ NBODY_BODY_CHAIN(body_body_chain_s, "s")
 // 16-byte load (gfx950 has no 12-byte scalar load, and the scalar-broadcast
 // kernel would otherwise get vector loads for x, y, z).
 #define NBODY_BODY_CHAIN_EQ(NAME, JC)                                                                  \
+    template <bool PRIO>                                                                               \
     __device__ __forceinline__ void NAME(float xj, float yj, float zj, float mj, float xi, float yi,   \
                                          float zi, float eps2, float& ax, float& ay, float& az)        \
     {                                                                                                  \
         float dx, dy, dz, s, t;                                                                        \
-        asm volatile("s_setprio 0\n"                                                                   \
+        asm volatile(".if %[prio]\n s_setprio 0\n .endif\n"                                            \
                      "v_sub_f32 %[dx], %[xj], %[xi]\n"                                                 \
                      "v_sub_f32 %[dy], %[yj], %[yi]\n"                                                 \
                      "v_sub_f32 %[dz], %[zj], %[zi]\n"                                                 \
                      "v_fma_f32 %[s], %[dx], %[dx], %[eps]\n"                                          \
                      "v_fmac_f32 %[s], %[dy], %[dy]\n"                                                 \
                      "v_fmac_f32 %[s], %[dz], %[dz]\n"                                                 \
-                     "s_setprio 1\n"                                                                   \
+                     ".if %[prio]\n s_setprio 1\n .endif\n"                                            \
                      "v_rsq_f32 %[s], %[s]\n"                                                          \
                      "s_nop 0\n"                                                                       \
                      "v_mul_f32 %[t], %[s], %[s]\n"                                                    \
@@ -131,7 +133,7 @@ NBODY_BODY_CHAIN(body_body_chain_s, "s")
                      : [ax] "+v"(ax), [ay] "+v"(ay), [az] "+v"(az), [dx] "=&v"(dx), [dy] "=&v"(dy),     \
                        [dz] "=&v"(dz), [s] "=&v"(s), [t] "=&v"(t)                                      \
                      : [xj] JC(xj), [yj] JC(yj), [zj] JC(zj), [mj] JC(mj), [xi] "v"(xi), [yi] "v"(yi),  \
-                       [zi] "v"(zi), [eps] "s"(eps2));                                                 \
+                       [zi] "v"(zi), [eps] "s"(eps2), [prio] "n"(PRIO ? 1 : 0));                       \
     }
 NBODY_BODY_CHAIN_EQ(body_body_chain_eq_v, "v")
 NBODY_BODY_CHAIN_EQ(body_body_chain_eq_s, "s")
@@ -139,16 +141,17 @@ NBODY_BODY_CHAIN_EQ(body_body_chain_eq_s, "s")
 
 // body_body for the kernels: the assembly chain when no Newton step is asked
 // for, with the j body in VGPRs (SGPR_J false) or SGPRs (SGPR_J true). EQ
-// leaves the mass out (the mass-free chain; with a Newton step, m = 1).
-template <bool NEWTON, bool SGPR_J, bool EQ = false>
+// leaves the mass out (the mass-free chain; with a Newton step, m = 1). PRIO:
+// the chain's wave priorities.
+template <bool NEWTON, bool SGPR_J, bool EQ = false, bool PRIO = true>
 __device__ __forceinline__ void interact(float xj, float yj, float zj, float mj, float xi, float yi, float zi,
                                          float eps2, float& ax, float& ay, float& az)
 {
     if constexpr (NEWTON) body_body<true>(xj, yj, zj, EQ ? 1.0f : mj, xi, yi, zi, eps2, ax, ay, az);
-    else if constexpr (EQ && SGPR_J) body_body_chain_eq_s(xj, yj, zj, mj, xi, yi, zi, eps2, ax, ay, az);
-    else if constexpr (EQ) body_body_chain_eq_v(xj, yj, zj, mj, xi, yi, zi, eps2, ax, ay, az);
-    else if constexpr (SGPR_J) body_body_chain_s(xj, yj, zj, mj, xi, yi, zi, eps2, ax, ay, az);
-    else body_body_chain_v(xj, yj, zj, mj, xi, yi, zi, eps2, ax, ay, az);
+    else if constexpr (EQ && SGPR_J) body_body_chain_eq_s<PRIO>(xj, yj, zj, mj, xi, yi, zi, eps2, ax, ay, az);
+    else if constexpr (EQ) body_body_chain_eq_v<PRIO>(xj, yj, zj, mj, xi, yi, zi, eps2, ax, ay, az);
+    else if constexpr (SGPR_J) body_body_chain_s<PRIO>(xj, yj, zj, mj, xi, yi, zi, eps2, ax, ay, az);
+    else body_body_chain_v<PRIO>(xj, yj, zj, mj, xi, yi, zi, eps2, ax, ay, az);
 }
 
 // src/nbody.cu:158-182 integrateOne, in the operation order the reference's
@@ -218,7 +221,7 @@ __device__ __forceinline__ void fold(Lanes<I>& hi, Lanes<I>& lo, const Lanes<I>&
 // One sweep over j bodies in groups of G: the G loads are issued before the
 // G x I interaction chains that consume them (the chains are assembly the
 // compiler neither reorders nor unrolls around), then the remainder.
-template <int I, bool NEWTON, bool SGPR_J, int G, bool EQ = false, class Load>
+template <int I, bool NEWTON, bool SGPR_J, int G, bool EQ = false, bool PRIO = true, class Load>
 __device__ __forceinline__ void sweep_grouped(const Load& load, int len, float eps2, const Lanes<I>& me,
                                               Lanes<I>& acc)
 {
@@ -231,26 +234,26 @@ __device__ __forceinline__ void sweep_grouped(const Load& load, int len, float e
         for (int q = 0; q < G; ++q)
 #pragma unroll
             for (int u = 0; u < I; ++u)
-                interact<NEWTON, SGPR_J, EQ>(b[q].x, b[q].y, b[q].z, b[q].w, me.x[u], me.y[u], me.z[u], eps2,
+                interact<NEWTON, SGPR_J, EQ, PRIO>(b[q].x, b[q].y, b[q].z, b[q].w, me.x[u], me.y[u], me.z[u], eps2,
                                              acc.x[u], acc.y[u], acc.z[u]);
     }
     for (; j < len; ++j) {
         const float4 b = load(j);
 #pragma unroll
         for (int u = 0; u < I; ++u)
-            interact<NEWTON, SGPR_J, EQ>(b.x, b.y, b.z, b.w, me.x[u], me.y[u], me.z[u], eps2, acc.x[u], acc.y[u],
-                                         acc.z[u]);
+            interact<NEWTON, SGPR_J, EQ, PRIO>(b.x, b.y, b.z, b.w, me.x[u], me.y[u], me.z[u], eps2, acc.x[u],
+                                               acc.y[u], acc.z[u]);
     }
 }
 
 // j bodies read with wave-uniform addresses: the compiler emits s_load_dwordx16
 // (four bodies per load) and the VALU ops take x_j, y_j, z_j, m_j as SGPR
 // operands, so no instruction is spent on the broadcast.
-template <int I, bool NEWTON, bool EQ = false>
+template <int I, bool NEWTON, bool EQ = false, bool PRIO = true>
 __device__ __forceinline__ void sweep_sgpr(const float4* __restrict__ src, int len, float eps2,
                                            const Lanes<I>& me, Lanes<I>& acc)
 {
-    sweep_grouped<I, NEWTON, true, 8, EQ>([src](int k) { return src[k]; }, len, eps2, me, acc);
+    sweep_grouped<I, NEWTON, true, 8, EQ, PRIO>([src](int k) { return src[k]; }, len, eps2, me, acc);
 }
 
 // Read-only view of body records for kernels whose body pointers are not
@@ -259,12 +262,12 @@ __device__ __forceinline__ void sweep_sgpr(const float4* __restrict__ src, int l
 // wave-uniform reads stay scalar loads (s_load) into SGPR operands.
 typedef const __attribute__((address_space(4))) float const_body_float;
 
-template <int I, bool NEWTON, bool EQ = false>
+template <int I, bool NEWTON, bool EQ = false, bool PRIO = true>
 __device__ __forceinline__ void sweep_const(const float4* src4, int len, float eps2, const Lanes<I>& me,
                                             Lanes<I>& acc)
 {
     const const_body_float* src = (const const_body_float*)(const void*)src4;
-    sweep_grouped<I, NEWTON, true, 8, EQ>(
+    sweep_grouped<I, NEWTON, true, 8, EQ, PRIO>(
         [src](int k) { return make_float4(src[4 * k + 0], src[4 * k + 1], src[4 * k + 2], src[4 * k + 3]); }, len,
         eps2, me, acc);
 }

@@ -126,7 +126,7 @@ __device__ __forceinline__ void slice_sums_mass(const float4* __restrict__ src, 
     }
 }
 
-template <int I, bool COMP, bool NEWTON>
+template <int I, bool COMP, bool NEWTON, bool PRIO>
 __global__ __launch_bounds__(kBlock) void k_force_sgpr(ForceParams p)
 {
     Lanes<I> me, hi, lo;
@@ -141,8 +141,8 @@ __global__ __launch_bounds__(kBlock) void k_force_sgpr(ForceParams p)
     // vector loads of the slice in the kernel, the compiler keeps only one of
     // the two sweeps' wave-uniform loads scalar otherwise
     slice_sums_mass<I, COMP>(
-        src, len, [&](int c, int l, Lanes<I>& a) { sweep_const<I, NEWTON, true>(src + c, l, eps2, me, a); },
-        [&](int c, int l, Lanes<I>& a) { sweep_const<I, NEWTON>(src + c, l, eps2, me, a); }, hi, lo);
+        src, len, [&](int c, int l, Lanes<I>& a) { sweep_const<I, NEWTON, true, PRIO>(src + c, l, eps2, me, a); },
+        [&](int c, int l, Lanes<I>& a) { sweep_const<I, NEWTON, false, PRIO>(src + c, l, eps2, me, a); }, hi, lo);
     store<I>(p, hi, COMP ? &lo : nullptr);
 }
 
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kBlock) void k_force_aos(ForceParams p)
 // j tiles of 256 bodies staged in LDS by the whole block (one coalesced float4
 // per lane), double-buffered so one barrier per tile suffices; each wave then
 // reads body k with a uniform address (a broadcast ds_read_b128).
-template <int I, bool COMP, bool NEWTON>
+template <int I, bool COMP, bool NEWTON, bool PRIO>
 __global__ __launch_bounds__(kBlock) void k_force_lds(ForceParams p)
 {
     __shared__ float4 tile[2][kBlock];
@@ -188,8 +188,8 @@ __global__ __launch_bounds__(kBlock) void k_force_lds(ForceParams p)
         zero<I>(part);
         Lanes<I>& acc = COMP ? part : hi;
         const float4* t4 = tile[buf];
-        if (eq) sweep_grouped<I, NEWTON, false, 4, true>([t4](int q) { return t4[q]; }, cnt, p.eps2, me, acc);
-        else sweep_grouped<I, NEWTON, false, 4>([t4](int q) { return t4[q]; }, cnt, p.eps2, me, acc);
+        if (eq) sweep_grouped<I, NEWTON, false, 4, true, PRIO>([t4](int q) { return t4[q]; }, cnt, p.eps2, me, acc);
+        else sweep_grouped<I, NEWTON, false, 4, false, PRIO>([t4](int q) { return t4[q]; }, cnt, p.eps2, me, acc);
         if constexpr (COMP) fold<I>(hi, lo, part);
     }
     if (eq) {
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(kBlock) void k_force_lds64(ForceParams p)
 // (base, n) gives each body the bits of the whole-system one. Compensated
 // plans fold the terms per 128 as the other variants do. Bodies past the
 // last full tile go through the scalar-load sweep.
-template <int I, bool NEWTON, bool EQ>
+template <int I, bool NEWTON, bool EQ, bool PRIO>
 __device__ __forceinline__ void sweep_dpp(const float4* __restrict__ src, int len, int shift, float eps2,
                                           const Lanes<I>& me, Lanes<I>& acc)
 {
@@ -285,8 +285,8 @@ __device__ __forceinline__ void sweep_dpp(const float4* __restrict__ src, int le
         for (int k = 0; k < 64; ++k) {
 #pragma unroll
             for (int u = 0; u < I; ++u)
-                interact<NEWTON, false, EQ>(xj, yj, zj, mj, me.x[u], me.y[u], me.z[u], eps2, acc.x[u], acc.y[u],
-                                            acc.z[u]);
+                interact<NEWTON, false, EQ, PRIO>(xj, yj, zj, mj, me.x[u], me.y[u], me.z[u], eps2, acc.x[u], acc.y[u],
+                                                  acc.z[u]);
             xj = wave_ror1(xj);
             yj = wave_ror1(yj);
             zj = wave_ror1(zj);
@@ -295,14 +295,14 @@ __device__ __forceinline__ void sweep_dpp(const float4* __restrict__ src, int le
     }
     // (through the constant address space: scalar loads, and no vector
     // registers for the group of j bodies in flight)
-    if (g < len) sweep_const<I, NEWTON, EQ>(src + g, len - g, eps2, me, acc);
+    if (g < len) sweep_const<I, NEWTON, EQ, PRIO>(src + g, len - g, eps2, me, acc);
 }
 
 // Compensated plans keep the TwoSum residues of the DPP kernel in LDS, one
 // column per thread (no thread reads another's, so no barrier), written once
 // per kChunk terms: with 8 bodies per lane the residues in VGPRs took the
 // kernel to 144 VGPRs, 3 waves per SIMD. Same arithmetic, same bits.
-template <int I, bool COMP, bool NEWTON>
+template <int I, bool COMP, bool NEWTON, bool PRIO>
 __global__ __launch_bounds__(kBlock) void k_force_dpp(ForceParams p)
 {
     Lanes<I> me, hi;
@@ -313,8 +313,12 @@ __global__ __launch_bounds__(kBlock) void k_force_dpp(ForceParams p)
     const float4* __restrict__ src = p.pm + j0;
     const float eps2 = p.eps2;
     const int shift = p.i0 & 63;
-    auto eq_sweep = [&](int c, int l, Lanes<I>& a) { sweep_dpp<I, NEWTON, true>(src + c, l, shift, eps2, me, a); };
-    auto gen_sweep = [&](int c, int l, Lanes<I>& a) { sweep_dpp<I, NEWTON, false>(src + c, l, shift, eps2, me, a); };
+    auto eq_sweep = [&](int c, int l, Lanes<I>& a) {
+        sweep_dpp<I, NEWTON, true, PRIO>(src + c, l, shift, eps2, me, a);
+    };
+    auto gen_sweep = [&](int c, int l, Lanes<I>& a) {
+        sweep_dpp<I, NEWTON, false, PRIO>(src + c, l, shift, eps2, me, a);
+    };
     if constexpr (!COMP) {
         Lanes<I> lo;
         zero<I>(lo);
@@ -382,7 +386,7 @@ struct SymParams {
     size_t more;     // floats from the slot rows of a pair's task h to those of task h + 1
 };
 
-template <int A, int W, bool NEWTON>
+template <int A, int W, bool NEWTON, bool PRIO>
 __global__ __launch_bounds__(64 * W) void k_force_sym(SymParams p)
 {
     constexpr int B = 64 * A * W;
@@ -391,10 +395,10 @@ __global__ __launch_bounds__(64 * W) void k_force_sym(SymParams p)
     if (t < p.npairs) {
         int P, Q;
         upper_pair(p.q0 * (p.q0 - 1) / 2 + t, P, Q);
-        sym_pair<A, W, NEWTON>(p.pm, p.n, p.eps2, p.slots, P, Q, jacc);
+        sym_pair<A, W, NEWTON, PRIO ? 0 : NO_PRIO>(p.pm, p.n, p.eps2, p.slots, P, Q, jacc);
     } else {
         const int d = t - p.npairs;
-        sym_diag_piece<B, NEWTON, false>(p.pm, p.n, p.eps2, p.slots, p.q0 + d / A, d % A, 64 * W);
+        sym_diag_piece<B, NEWTON, PRIO, false>(p.pm, p.n, p.eps2, p.slots, p.q0 + d / A, d % A, 64 * W);
     }
 }
 
@@ -798,10 +802,10 @@ __global__ void k_energy_fp64_final(const double* __restrict__ partial, int bloc
 #define NBODY_KERNEL_FAMILY(NAME, KERNEL, MAX_I)                                                 \
     struct NAME {                                                                                \
         static constexpr int kMaxI = MAX_I;                                                      \
-        template <int I, bool C, bool N>                                                         \
+        template <int I, bool C, bool N, bool P>                                                 \
         static void go(dim3 g, hipStream_t s, const ForceParams& p)                              \
         {                                                                                        \
-            KERNEL<I, C, N><<<g, kBlock, 0, s>>>(p);                                             \
+            KERNEL<I, C, N, P><<<g, kBlock, 0, s>>>(p);                                          \
         }                                                                                        \
     };
 NBODY_KERNEL_FAMILY(FamSgpr, k_force_sgpr, 4)
@@ -809,15 +813,27 @@ NBODY_KERNEL_FAMILY(FamLds, k_force_lds, 4)
 NBODY_KERNEL_FAMILY(FamDpp, k_force_dpp, 8)
 #undef NBODY_KERNEL_FAMILY
 
+// Whether a launch of so many waves leaves every SIMD with one at most. Its
+// chains then run without wave priorities, which take an issue slot each (a
+// Newton step's have none). With and without them: the DPP variant 43.7 and 40.4
+// us at N = 1000, 51.1 and 47.7 at 8192; scalar loads 54.8 and 51.8 at 8192; the
+// symmetric plan in blocks of 128 21.8 and 20.4 at 3000, in blocks of 1024 337 and
+// 295 at 16384. With four waves to a SIMD the priorities win (16384, scalar
+// loads: 98.6 and 86.0).
+bool lone_waves(const ForcePlan& plan, size_t waves) { return waves <= 4 * (size_t)std::max(plan.cus, 1); }
+
 template <class Fam, int I>
 void go_i(const ForcePlan& plan, dim3 g, hipStream_t s, const ForceParams& p)
 {
+    const bool lone = lone_waves(plan, (size_t)g.x * g.y * (kBlock / 64));
     if (plan.comp) {
-        if (plan.newton) Fam::template go<I, true, true>(g, s, p);
-        else Fam::template go<I, true, false>(g, s, p);
+        if (plan.newton) Fam::template go<I, true, true, true>(g, s, p);
+        else if (lone) Fam::template go<I, true, false, false>(g, s, p);
+        else Fam::template go<I, true, false, true>(g, s, p);
     } else {
-        if (plan.newton) Fam::template go<I, false, true>(g, s, p);
-        else Fam::template go<I, false, false>(g, s, p);
+        if (plan.newton) Fam::template go<I, false, true, true>(g, s, p);
+        else if (lone) Fam::template go<I, false, false, false>(g, s, p);
+        else Fam::template go<I, false, false, true>(g, s, p);
     }
 }
 
@@ -891,10 +907,12 @@ size_t lds_for_occupancy(const void* kernel, int threads, int waves)
     return dyn;
 }
 
-template <int A, int W, bool NEWTON>
-const void* sym_kernel()
+template <int A, int W>
+const void* sym_kernel(bool newton, bool lone)
 {
-    return reinterpret_cast<const void*>(&k_force_sym<A, W, NEWTON>);
+    return newton ? reinterpret_cast<const void*>(&k_force_sym<A, W, true, true>)
+           : lone ? reinterpret_cast<const void*>(&k_force_sym<A, W, false, false>)
+                  : reinterpret_cast<const void*>(&k_force_sym<A, W, false, true>);
 }
 
 const void* deal_kernel(bool newton, bool fold, bool lead)
@@ -909,10 +927,11 @@ template <int A, int W>
 hipError_t go_sym(const ForcePlan& plan, const SymParams& sp, int band_blocks, hipStream_t s)
 {
     const int tasks = sp.npairs + band_blocks * A;
-    const void* k = plan.newton ? sym_kernel<A, W, true>() : sym_kernel<A, W, false>();
-    const size_t dyn = plan.occ > 0 ? lds_for_occupancy(k, 64 * W, plan.occ) : 0;
-    if (plan.newton) k_force_sym<A, W, true><<<tasks, 64 * W, dyn, s>>>(sp);
-    else k_force_sym<A, W, false><<<tasks, 64 * W, dyn, s>>>(sp);
+    const bool lone = plan.occ == 1 || lone_waves(plan, (size_t)tasks * W);
+    const size_t dyn = plan.occ > 0 ? lds_for_occupancy(sym_kernel<A, W>(plan.newton, lone), 64 * W, plan.occ) : 0;
+    if (plan.newton) k_force_sym<A, W, true, true><<<tasks, 64 * W, dyn, s>>>(sp);
+    else if (lone) k_force_sym<A, W, false, false><<<tasks, 64 * W, dyn, s>>>(sp);
+    else k_force_sym<A, W, false, true><<<tasks, 64 * W, dyn, s>>>(sp);
     return hipGetLastError();
 }
 
@@ -1016,7 +1035,7 @@ SlotMapT<T> band_slots(T* base, int q0, int q1, int B, int split = 1)
 template <int A, int W>
 int natural_occupancy(bool newton)
 {
-    return blocks_per_cu(newton ? sym_kernel<A, W, true>() : sym_kernel<A, W, false>(), 64 * W, 0) * W / 4;
+    return blocks_per_cu(sym_kernel<A, W>(newton, false), 64 * W, 0) * W / 4;
 }
 
 }  // namespace

@@ -118,8 +118,14 @@ __device__ __forceinline__ void upper_pair(int t, int& P, int& Q)
 // and 43.8, 61.0 and 52; 2 waves 58.7 and 53, 63.5 and 56. Of some 350
 // placements measured, one rise right before the v_rsq_f32 gives 43.8 and
 // 50.2, a fall there 52 and 58. The results are the same bits.
-#define NBODY_PRIO(p) "s_setprio %[p" #p "]\n"
-#define NBODY_PRIO_IN(base) [p0] "n"(base), [p1] "n"((base) + 1), [p2] "n"((base) + 2)
+//
+// With one wave to a SIMD there is nobody to pair with, and the priorities only
+// take issue slots: such launches run the chain without them (BASE NO_PRIO;
+// lone_waves in nbody_kernels.hip).
+enum : int { NO_PRIO = -1 };
+#define NBODY_PRIO(p) ".if %[prio]\n s_setprio %[p" #p "]\n .endif\n"
+#define NBODY_PRIO_IN(base) \
+    [prio] "n"((base) >= 0 ? 1 : 0), [p0] "n"(base), [p1] "n"((base) + 1), [p2] "n"((base) + 2)
 #define NBODY_SYM_PAIR(u)                                                                              \
     NBODY_PRIO(0)                                                                                      \
     "v_sub_f32 %[dx], %[xj], %[x" #u "]\n"                                                             \
@@ -424,6 +430,7 @@ __device__ __forceinline__ void sym_step8_eq(float& xj, float& yj, float& zj, fl
 // faster than this chain order (blocks of 256 at N = 24576..65536: 0.54-0.71
 // of the FP32 peak against 0.53-0.68; the same at N = 16384), so that shape
 // runs the generic loop; with 2 and 8 the chain order is faster.
+template <int BASE>
 __device__ __forceinline__ void sym_step2(float& xj, float& yj, float& zj, float& mj, float& rx, float& ry, float& rz,
                                           Lanes<2>& acc, const Lanes<2>& me, const float (&mi)[2], float eps2)
 {
@@ -436,9 +443,10 @@ __device__ __forceinline__ void sym_step2(float& xj, float& yj, float& zj, float
                    [ay1] "+v"(acc.y[1]), [az0] "+v"(acc.z[0]), [az1] "+v"(acc.z[1]), [dx] "=&v"(dx),
                    [dy] "=&v"(dy), [dz] "=&v"(dz), [s] "=&v"(s), [t] "=&v"(t)
                  : [x0] "v"(me.x[0]), [x1] "v"(me.x[1]), [y0] "v"(me.y[0]), [y1] "v"(me.y[1]), [z0] "v"(me.z[0]),
-                   [z1] "v"(me.z[1]), [n0] "v"(mi[0]), [n1] "v"(mi[1]), [eps] "s"(eps2), NBODY_PRIO_IN(0));
+                   [z1] "v"(me.z[1]), [n0] "v"(mi[0]), [n1] "v"(mi[1]), [eps] "s"(eps2), NBODY_PRIO_IN(BASE));
 }
 
+template <int BASE>
 __device__ __forceinline__ void sym_step2_eq(float& xj, float& yj, float& zj, float& rx, float& ry, float& rz,
                                           Lanes<2>& acc, const Lanes<2>& me, float eps2)
 {
@@ -451,7 +459,7 @@ __device__ __forceinline__ void sym_step2_eq(float& xj, float& yj, float& zj, fl
                    [az0] "+v"(acc.z[0]), [az1] "+v"(acc.z[1]), [dx] "=&v"(dx), [dy] "=&v"(dy), [dz] "=&v"(dz),
                    [s] "=&v"(s), [t] "=&v"(t)
                  : [x0] "v"(me.x[0]), [x1] "v"(me.x[1]), [y0] "v"(me.y[0]), [y1] "v"(me.y[1]), [z0] "v"(me.z[0]),
-                   [z1] "v"(me.z[1]), [eps] "s"(eps2), NBODY_PRIO_IN(0));
+                   [z1] "v"(me.z[1]), [eps] "s"(eps2), NBODY_PRIO_IN(BASE));
 }
 
 // One rotation step of diagonal tile T (see sym_diag_tile) in assembly, in
@@ -633,8 +641,8 @@ __device__ __forceinline__ void sym_step(float& xj, float& yj, float& zj, float&
         if constexpr (EQ) sym_step8_eq<REGS, BASE>(xj, yj, zj, rx, ry, rz, acc, me, eps2);
         else sym_step8<REGS, BASE>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
     } else if constexpr (A == 2 && !NEWTON) {
-        if constexpr (EQ) sym_step2_eq(xj, yj, zj, rx, ry, rz, acc, me, eps2);
-        else sym_step2(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+        if constexpr (EQ) sym_step2_eq<BASE>(xj, yj, zj, rx, ry, rz, acc, me, eps2);
+        else sym_step2<BASE>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
     } else {
 #pragma unroll
         for (int u = 0; u < A; ++u) {
@@ -668,7 +676,7 @@ __device__ __forceinline__ void sym_step(float& xj, float& yj, float& zj, float&
 // The phases of block pair (P, Q): every wave streams the T tiles of block Q
 // past its A i bodies per lane, adding the i side into acc and each tile's
 // reaction into jacc. With EQ the pair weights leave out the (common) mass.
-template <int A, int W, bool NEWTON, bool EQ>
+template <int A, int W, bool NEWTON, bool EQ, int BASE>
 __device__ __forceinline__ void sym_phases(const float4* __restrict__ pm, int n, float eps2, int Q,
                                            const Lanes<A>& me, const float (&mi)[A], Lanes<A>& acc,
                                            float (*jacc)[64 * A * W])
@@ -689,7 +697,8 @@ __device__ __forceinline__ void sym_phases(const float4* __restrict__ pm, int n,
             const float4 b = lane < n - jbase ? pm[jbase + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
             float xj = b.x, yj = b.y, zj = b.z, mj = b.w;
             float rx = 0.f, ry = 0.f, rz = 0.f;
-            for (int k = 0; k < 64; ++k) sym_step<A, NEWTON, EQ, REGS_FREE>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
+            for (int k = 0; k < 64; ++k)
+                sym_step<A, NEWTON, EQ, REGS_FREE, BASE>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
             const int slot = tile * 64 + lane;
             jacc[0][slot] += rx;
             jacc[1][slot] += ry;
@@ -714,7 +723,7 @@ __device__ __forceinline__ bool workgroup_all(bool ok)
 // weights leave the mass out and the partials are multiplied by it once, at
 // the store; with m = 1 (or any power of two) the result is bit-identical to
 // the general weights.
-template <int A, int W, bool NEWTON>
+template <int A, int W, bool NEWTON, int BASE>
 __device__ __forceinline__ void sym_pair(const float4* __restrict__ pm, int n, float eps2, const SlotMap& slots, int P,
                                          int Q, float (*jacc)[64 * A * W])
 {
@@ -744,8 +753,8 @@ __device__ __forceinline__ void sym_pair(const float4* __restrict__ pm, int n, f
     for (int k = threadIdx.x; k < B; k += 64 * W) jacc[0][k] = jacc[1][k] = jacc[2][k] = 0.f;
     __syncthreads();
     const bool eq = workgroup_all<W>(same);
-    if (eq) sym_phases<A, W, NEWTON, true>(pm, n, eps2, Q, me, mi, acc, jacc);
-    else sym_phases<A, W, NEWTON, false>(pm, n, eps2, Q, me, mi, acc, jacc);
+    if (eq) sym_phases<A, W, NEWTON, true, BASE>(pm, n, eps2, Q, me, mi, acc, jacc);
+    else sym_phases<A, W, NEWTON, false, BASE>(pm, n, eps2, Q, me, mi, acc, jacc);
     const float scale = eq ? m0 : 1.0f;
     float* __restrict__ jdst = slots.j_side(P, Q, B);
     for (int k = threadIdx.x; k < B; k += 64 * W) {
@@ -1052,7 +1061,7 @@ __device__ __forceinline__ void sym_deal_task(const float4* __restrict__ pm, int
 // into slot P. Lanes past n compute on a zero body and store into padding
 // that no reduction reads. CONST_VIEW reads the j bodies through the constant
 // address space (pointers that come from memory rather than kernel arguments).
-template <int B, bool NEWTON, bool CONST_VIEW>
+template <int B, bool NEWTON, bool PRIO, bool CONST_VIEW>
 __device__ __forceinline__ void sym_diag_piece(const float4* __restrict__ pm, int n, float eps2, const SlotMap& slots,
                                                int P, int k, int threads)
 {
@@ -1065,8 +1074,8 @@ __device__ __forceinline__ void sym_diag_piece(const float4* __restrict__ pm, in
     me.z[0] = q.z;
     zero<1>(acc);
     const int j0 = P * B;
-    if constexpr (CONST_VIEW) sweep_const<1, NEWTON>(pm + j0, min(n - j0, B), eps2, me, acc);
-    else sweep_sgpr<1, NEWTON>(pm + j0, min(n - j0, B), eps2, me, acc);
+    if constexpr (CONST_VIEW) sweep_const<1, NEWTON, false, PRIO>(pm + j0, min(n - j0, B), eps2, me, acc);
+    else sweep_sgpr<1, NEWTON, false, PRIO>(pm + j0, min(n - j0, B), eps2, me, acc);
     // slot P of block P's bodies: a band block, region B
     float* __restrict__ dst = slots.j_side(P, P, B) + k * threads + threadIdx.x;
     dst[0] = acc.x[0];
