@@ -68,10 +68,13 @@ int round_up(int v, int m) { return (v + m - 1) / m * m; }
 // time).
 constexpr int kSymSlotsTarget = 512;
 // Below this N the default symmetric plan takes blocks of 128 bodies, one wave
-// each with 2 bodies per lane: at N = 4096 it takes 16.2 us against 18.0 with
-// blocks of 512, whose 36 block pairs leave most CUs idle; at N = 6000 26.1
-// against 22.5.
-constexpr size_t kSmallSymN = 5120;
+// each with 2 bodies per lane, whose launch leaves a SIMD one wave at most: at
+// N = 4096 it took 16.2 us against 18.0 with blocks of 512, whose 36 block pairs
+// leave most CUs idle, at 5200 and 5504 it takes 21.1 and 21.7 against 23.5, at 6000
+// 24.4 to 26.1 against 25.0. With a Newton step, whose chains take 1.6 times as
+// long: 5200 22.7 and 31.9, 7000 34.1 and 35.6, 8192 33.4 and 36.5, 9000 44.3 and
+// 44.5, 10240 54.9 and 52.1.
+constexpr size_t kSmallSymN = 5633, kSmallSymNewtonN = 9217;
 // A share of the block pairs with less work than this per share takes blocks
 // of 128 bodies below N = 16384 and of 256 below 32768 all the same: a share's
 // pairs are one task each, and a block pair of 512 that has its CU to itself takes
@@ -157,7 +160,7 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
         // TwoSum
         p.ipl = (opt && opt->i_per_lane > 0) ? opt->i_per_lane : 8;
         const bool shape_given = opt && (opt->i_per_lane > 0 || opt->jslice > 0);
-        if (!shape_given && N < kSmallSymN) {
+        if (!shape_given && N < (p.newton ? kSmallSymNewtonN : kSmallSymN)) {
             p.ipl = 2;
             p.jslice = 128;
         } else if (!shape_given && fine_share(N, shares, opt ? opt->slot_bytes : 0, &p.ipl)) {

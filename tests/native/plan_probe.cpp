@@ -1,5 +1,6 @@
 // Prints the library's plans without a GPU: one line of input, one of output.
 //   default VARIANT N n CUS -> variant i_per_lane jslice nslices li
+//   newton VARIANT N n CUS  -> the same with a Newton step
 //   tile n ni ACC64 CUS     -> li i_per_lane
 //   tasks N CUS             -> tasks per block pair of the symmetric plan's blocks of 512
 //   lead TASKS CUS OCC      -> whether that launch's first halves go first
@@ -15,11 +16,12 @@ int main()
 {
     std::string what;
     while (std::cin >> what) {
-        if (what == "default") {
+        if (what == "default" || what == "newton") {
             int variant, cus;
             size_t N, n;
             std::cin >> variant >> N >> n >> cus;
-            const ForcePlan p = detail::default_plan(variant, N, n, cus, nullptr);
+            const nbody_hip_options o{variant, 0, 0, -1, what == "newton" ? 1 : 0, 0, 0};
+            const ForcePlan p = detail::default_plan(variant, N, n, cus, &o);
             std::printf("%d %d %d %d %d\n", p.variant, p.ipl, p.jslice, p.nslices, p.li);
         } else if (what == "tile") {
             size_t n, ni;

@@ -66,3 +66,13 @@ def test_lead_needs_every_task_resident(probe):
     lines = {"1024 256 0": 1, "1025 256 0": 0, "512 256 2": 1, "513 256 2": 0, "768 256 3": 1, "769 256 3": 0,
              "1024 256 6": 1, "1025 256 6": 0, "128 32 0": 1, "129 32 0": 0}
     assert [r[0] for r in probe(*[f"lead {k}" for k in lines])] == list(lines.values())
+
+
+def test_small_symmetric_blocks(probe):
+    """Blocks of 128 up to 44 of them, with a Newton step up to 72; 512 past that."""
+    sym = _native.SYMMETRIC
+    shapes = {f"default {sym} {n} {n} 256": (2, 128) for n in (1024, 5121, 5632)}
+    shapes |= {f"default {sym} {n} {n} 256": (8, 512) for n in (5633, 9216)}
+    shapes |= {f"newton {sym} {n} {n} 256": (2, 128) for n in (1024, 5633, 9216)}
+    shapes |= {f"newton {sym} {n} {n} 256": (8, 512) for n in (9217, 30000)}
+    assert [(r[1], r[2]) for r in probe(*shapes)] == list(shapes.values())
