@@ -121,15 +121,19 @@ bool tile_allowed(size_t N, size_t n, const nbody_hip_options* opt)
 // for one GPU's eighth of N = 98304 with slices of 256, 512, 1024, 2048, two
 // bodies per lane: 308, 299, 305, 350, and with one: 332, 324, 326, 344; its
 // quarter of 150751: 1536, 1492, 1472, 1528; half of 33588 153, 164, 188, 240.
+// With a Newton step and plain sums one body per lane stays ahead, over the
+// same slices (N = 24000 214 and 239, 32768 377 and 415, 65536 1450 and 1595; with
+// compensated sums two: an eighth of 98304 441 and 424).
 constexpr double kLdsWideWork = 5.0e8;
 
-void lds_shape(size_t N, size_t n, int cus, int* ipl, int* jslice)
+void lds_shape(size_t N, size_t n, int cus, bool newton_plain, int* ipl, int* jslice)
 {
     *ipl = (double)n * (double)N >= kLdsWideWork ? 2 : 1;
     const double per_cu = std::ceil((double)n / (256.0 * *ipl)) * (double)N / std::max(cus, 1);
     double len = per_cu / 20.0 <= 1024.0 ? per_cu / 20.0 : std::max(1024.0, per_cu / 80.0);
     len = std::min(len, (double)N);  // (past 1.5e8 bodies the quotient no longer fits an int; N does)
     *jslice = std::max(1, (int)(len / 256.0 + 0.5)) * 256;
+    if (newton_plain) *ipl = 1;
 }
 
 // Default decomposition: enough blocks for ~48 waves per SIMD (the dispatcher
@@ -187,7 +191,7 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
         return p;
     }
     if (variant == VAR_LDS && !p.acc64 && !(opt && (opt->i_per_lane > 0 || opt->jslice > 0))) {
-        lds_shape(N, n, cus, &p.ipl, &p.jslice);
+        lds_shape(N, n, cus, p.newton && !p.comp, &p.ipl, &p.jslice);
         int li, ipl;
         // the sliced plan's time: a wave's chain through its slice at the least, and about 16 us of
         // launches and slice sum (sliced and in one launch: 1000 of 4096 bodies 19.5 and 4.6 us, 8192 of

@@ -76,3 +76,11 @@ def test_small_symmetric_blocks(probe):
     shapes |= {f"newton {sym} {n} {n} 256": (2, 128) for n in (1024, 5633, 9216)}
     shapes |= {f"newton {sym} {n} {n} 256": (8, 512) for n in (9217, 30000)}
     assert [(r[1], r[2]) for r in probe(*shapes)] == list(shapes.values())
+
+
+def test_bodies_per_lane_of_large_lds_evaluations(probe):
+    """Two past 5e8 pairs, but one with a Newton step and plain sums (the default up to N = 65536)."""
+    lds = _native.LDS
+    want = {f"default {lds} 30000 30000 256": 2, f"newton {lds} 30000 30000 256": 1,
+            f"newton {lds} 65536 65536 256": 1, f"newton {lds} 98304 12288 256": 2, f"default {lds} 98304 12288 256": 2}
+    assert [r[1] for r in probe(*want)] == list(want.values())
