@@ -325,6 +325,58 @@ int make_plan(DeviceState& d, size_t N, size_t n, const nbody_hip_options* opt, 
     return OK;
 }
 
+std::vector<ForcePlan> tune_candidates(int fam, size_t N, int cus)
+{
+    std::vector<ForcePlan> cands;
+    nbody_hip_options o{fam, 0, 0, -1, 0};
+    if (fam == VAR_AOS) {
+        cands.push_back(default_plan(fam, N, N, cus, &o));
+    } else if (fam == VAR_SYMMETRIC) {
+        const int shapes[][2] = {{2, 128}, {2, 512}, {4, 256}, {4, 512}, {4, 1024}, {8, 512}, {8, 1024}, {8, 2048}};
+        for (const auto& sh : shapes) {
+            o.i_per_lane = sh[0];
+            o.jslice = sh[1];
+            ForcePlan c = default_plan(fam, N, N, cus, &o);
+            if (c.nslices > kMaxSymBlocks) continue;
+            cands.push_back(c);
+            // the same shape with one and two fewer resident waves per
+            // SIMD, and with two: a launch of a few tasks per SIMD ends
+            // unevenly when they all start at once, while at two resident
+            // waves (about the issue rate of six) the later tasks start
+            // as slots free
+            const int natural = symmetric_natural_occupancy(c);
+            int last = natural;
+            for (int waves : {natural - 1, natural - 2, 2}) {
+                if (waves < 2 || waves >= last) continue;
+                last = waves;
+                c.occ = waves;
+                cands.push_back(c);
+            }
+        }
+    } else {
+        // the default itself: the LDS variant's is no shape of those below (two
+        // bodies per lane over slices of its own length, or one launch)
+        cands.push_back(default_plan(fam, N, N, cus, &o));
+        for (int ipl : {1, 2, 4, 8}) {
+            if (ipl == 8 && fam != VAR_DPP) continue;
+            o.i_per_lane = ipl;
+            o.jslice = 0;
+            const ForcePlan q = default_plan(fam, N, N, cus, &o);
+            for (int mul : {1, 2, 4}) {
+                for (int div : {1, 2, 4}) {
+                    if (mul > 1 && div > 1) continue;
+                    ForcePlan c = q;
+                    c.jslice = std::min((int)N, round_up(std::max(256, q.jslice * mul / div), 256));
+                    c.nslices = (int)((N + c.jslice - 1) / c.jslice);
+                    if (c.ipl != cands.front().ipl || c.jslice != cands.front().jslice || cands.front().li > 0)
+                        cands.push_back(c);
+                }
+            }
+        }
+    }
+    return cands;
+}
+
 void describe_plan(const ForcePlan& p, nbody_hip_options* out)
 {
     // the one-launch kernel has no slices and its shape is no option: zeros
@@ -816,50 +868,8 @@ float nbody_hip_autotune(float* force, const float* posMass, float softeningSqua
     }
     std::vector<ForcePlan> cands;
     for (int fam : families) {
-        nbody_hip_options o = base;
-        o.variant = fam;
-        if (fam == VAR_AOS) {
-            cands.push_back(default_plan(fam, N, N, d->cus, &o));
-        } else if (fam == VAR_SYMMETRIC) {
-            const int shapes[][2] = {{2, 128}, {2, 512}, {4, 256}, {4, 512}, {4, 1024}, {8, 512}, {8, 1024}, {8, 2048}};
-            for (const auto& sh : shapes) {
-                o.i_per_lane = sh[0];
-                o.jslice = sh[1];
-                ForcePlan c = default_plan(fam, N, N, d->cus, &o);
-                if (c.nslices > kMaxSymBlocks) continue;
-                cands.push_back(c);
-                // the same shape with one and two fewer resident waves per
-                // SIMD, and with two: a launch of a few tasks per SIMD ends
-                // unevenly when they all start at once, while at two resident
-                // waves (about the issue rate of six) the later tasks start
-                // as slots free
-                const int natural = symmetric_natural_occupancy(c);
-                int last = natural;
-                for (int waves : {natural - 1, natural - 2, 2}) {
-                    if (waves < 2 || waves >= last) continue;
-                    last = waves;
-                    c.occ = waves;
-                    cands.push_back(c);
-                }
-            }
-        } else {
-            if (ForcePlan c = default_plan(fam, N, N, d->cus, &o); c.li > 0) cands.push_back(c);
-            for (int ipl : {1, 2, 4, 8}) {
-                if (ipl == 8 && fam != VAR_DPP) continue;
-                o.i_per_lane = ipl;
-                o.jslice = 0;
-                ForcePlan q = default_plan(fam, N, N, d->cus, &o);
-                for (int mul : {1, 2, 4}) {
-                    for (int div : {1, 2, 4}) {
-                        if (mul > 1 && div > 1) continue;
-                        ForcePlan c = q;
-                        c.jslice = std::min((int)N, round_up(std::max(256, q.jslice * mul / div), 256));
-                        c.nslices = (int)((N + c.jslice - 1) / c.jslice);
-                        cands.push_back(c);
-                    }
-                }
-            }
-        }
+        const std::vector<ForcePlan> more = tune_candidates(fam, N, d->cus);
+        cands.insert(cands.end(), more.begin(), more.end());
     }
     if (cands.empty()) {
         set_error("no plan of variant %d fits N = %zu", variant, N);

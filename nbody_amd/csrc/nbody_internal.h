@@ -127,6 +127,9 @@ int round_up(int v, int m);
 // (`shares`: of how many shares of the block pairs the plan is to run one)
 ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip_options* opt, int shares = 1);
 int make_plan(DeviceState& d, size_t N, size_t n, const nbody_hip_options* opt, ForcePlan* plan, int shares = 1);
+// The plans of one variant that nbody_hip_autotune times for N bodies, its
+// default among them.
+std::vector<ForcePlan> tune_candidates(int fam, size_t N, int cus);
 // The plan as options (nbody_hip_plan, nbody_hip_system_plan).
 void describe_plan(const ForcePlan& p, nbody_hip_options* out);
 int check_args(const void* force, const void* pm, size_t N, size_t base, size_t n);

@@ -4,6 +4,7 @@
 //   tile n ni ACC64 CUS     -> li i_per_lane
 //   tasks N CUS             -> tasks per block pair of the symmetric plan's blocks of 512
 //   lead TASKS CUS OCC      -> whether that launch's first halves go first
+//   tuned VARIANT N CUS     -> how many plans autotune times, and how many of them are the default
 #include "nbody_internal.h"
 
 #include <cstdio>
@@ -37,6 +38,16 @@ int main()
             const ForcePlan p = detail::default_plan(VAR_SYMMETRIC, N, N, cus, &o);
             const size_t one = (size_t)12 * 512 * p.nslices * p.nslices;
             std::printf("%zu\n", plan_scratch_bytes(p, (int)N) / one);
+        } else if (what == "tuned") {
+            int variant, cus, same = 0;
+            size_t N;
+            std::cin >> variant >> N >> cus;
+            const ForcePlan p = detail::default_plan(variant, N, N, cus, nullptr);
+            const auto all = detail::tune_candidates(variant, N, cus);
+            for (const ForcePlan& c : all)
+                same += c.li == p.li && c.ipl == p.ipl && c.jslice == p.jslice && c.nslices == p.nslices &&
+                        c.comp == p.comp;
+            std::printf("%zu %d\n", all.size(), same);
         } else if (what == "lead") {
             ForcePlan p;
             int tasks;

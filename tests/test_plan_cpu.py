@@ -84,3 +84,13 @@ def test_bodies_per_lane_of_large_lds_evaluations(probe):
     want = {f"default {lds} 30000 30000 256": 2, f"newton {lds} 30000 30000 256": 1,
             f"newton {lds} 65536 65536 256": 1, f"newton {lds} 98304 12288 256": 2, f"default {lds} 98304 12288 256": 2}
     assert [r[1] for r in probe(*want)] == list(want.values())
+
+
+def test_autotune_times_the_default(probe):
+    """The plan a call uses untuned is one of those the tuner compares, once."""
+    cases = [(v, n) for v in (_native.AOS, _native.LDS, _native.DPP, _native.SGPR)
+             for n in (1, 300, 1000, 8192, 16384, 30000, 65537, 98304, 1 << 20)]
+    for (v, n), (count, same) in zip(cases, probe(*[f"tuned {v} {n} 256" for v, n in cases])):
+        assert same >= 1 and count >= 1, (v, n)
+        if n >= 8192 and v != _native.AOS:
+            assert same == 1 and count >= 8, (v, n)
