@@ -277,7 +277,8 @@ void append_force_tasks(std::vector<ForceTask>& out, const float4* pm, void* par
         t.b = 0;
         t.len = (int)n;
         t.slot = 0;
-        for (size_t i = 0; i < n; i += kWave * kDealWaves) {
+        const size_t rows = kWave * (acc64 ? kWaves64 : kDealWaves);  // a workgroup's, of either kernel
+        for (size_t i = 0; i < n; i += rows) {
             t.a = (int)i;
             out.push_back(t);
         }
