@@ -398,7 +398,7 @@ __global__ __launch_bounds__(64 * W) void k_force_sym(SymParams p)
         sym_pair<A, W, NEWTON, PRIO ? 0 : NO_PRIO>(p.pm, p.n, p.eps2, p.slots, P, Q, jacc);
     } else {
         const int d = t - p.npairs;
-        sym_diag_piece<B, NEWTON, PRIO, false>(p.pm, p.n, p.eps2, p.slots, p.q0 + d / A, d % A, 64 * W);
+        sym_diag_piece<B, NEWTON, PRIO>(p.pm, p.n, p.eps2, p.slots, p.q0 + d / A, d % A, 64 * W);
     }
 }
 
@@ -873,9 +873,7 @@ hipError_t go_tile(const ForcePlan& plan, dim3 g, hipStream_t s, const ForcePara
     case 403: go_tile_shape<4, 3>(g, s, p); break;
     case 802: go_tile_shape<8, 2>(g, s, p); break;
     case 803: go_tile_shape<8, 3>(g, s, p); break;
-    case 804: go_tile_shape<8, 4>(g, s, p); break;
     case 805: go_tile_shape<8, 5>(g, s, p); break;
-    case 806: go_tile_shape<8, 6>(g, s, p); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1046,15 +1044,16 @@ namespace {
 // takes in them when the workgroups fill it, fitted with tile_shape's other
 // figures to every shape at ten sizes from N = 1000 to 10240. The choice is the
 // fastest shape at nine of them and within 5 % at N = 1000. Some of them, in
-// the order below: N = 2048 4.4, 4.3, 5.0, 5.2, 6.5, 7.7, 9.0, 10.3 us; 4096
-// 10.5, 8.6, 10.4, 7.8, 10.1, 12.3, 14.8, 17.0; 8192 32.0, 25.2, 25.4, 21.3,
-// 28.3, 21.7, 25.9, 30.2; 10240 47.5, 37.1, 39.5, 37.3, 35.0, 50.4, 31.7, 36.9.
+// the order below: N = 2048 4.4, 4.3, 5.0, 5.2, 6.5, 9.0 us; 4096 10.5, 8.6, 10.4,
+// 7.8, 10.1, 14.8; 8192 32.0, 25.2, 25.4, 21.3, 28.3, 25.9; 10240 47.5, 37.1, 39.5,
+// 37.3, 35.0, 31.7. (8 lanes times 4 or 6 bodies, one workgroup to a CU, never beat
+// two workgroups of 8 times 2 or 3.)
 struct TileShape {
     int li, ipl;
     double clocks;
 };
 constexpr TileShape kTileShapes[] = {{4, 1, .242}, {4, 2, .191}, {4, 3, .175}, {8, 2, .161},
-                                     {8, 3, .157}, {8, 4, .166}, {8, 5, .164}, {8, 6, .163}};
+                                     {8, 3, .157}, {8, 5, .164}};
 
 }  // namespace
 

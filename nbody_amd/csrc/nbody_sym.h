@@ -1059,9 +1059,8 @@ __device__ __forceinline__ void sym_deal_task(const float4* __restrict__ pm, int
 // Piece k (of A) of block P's diagonal: its 64*W threads take bodies
 // P*B + k*64*W + threadIdx.x against block P's bodies, a plain sum in j order,
 // into slot P. Lanes past n compute on a zero body and store into padding
-// that no reduction reads. CONST_VIEW reads the j bodies through the constant
-// address space (pointers that come from memory rather than kernel arguments).
-template <int B, bool NEWTON, bool PRIO, bool CONST_VIEW>
+// that no reduction reads.
+template <int B, bool NEWTON, bool PRIO>
 __device__ __forceinline__ void sym_diag_piece(const float4* __restrict__ pm, int n, float eps2, const SlotMap& slots,
                                                int P, int k, int threads)
 {
@@ -1074,8 +1073,7 @@ __device__ __forceinline__ void sym_diag_piece(const float4* __restrict__ pm, in
     me.z[0] = q.z;
     zero<1>(acc);
     const int j0 = P * B;
-    if constexpr (CONST_VIEW) sweep_const<1, NEWTON, false, PRIO>(pm + j0, min(n - j0, B), eps2, me, acc);
-    else sweep_sgpr<1, NEWTON, false, PRIO>(pm + j0, min(n - j0, B), eps2, me, acc);
+    sweep_sgpr<1, NEWTON, false, PRIO>(pm + j0, min(n - j0, B), eps2, me, acc);
     // slot P of block P's bodies: a band block, region B
     float* __restrict__ dst = slots.j_side(P, P, B) + k * threads + threadIdx.x;
     dst[0] = acc.x[0];
