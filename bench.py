@@ -948,7 +948,7 @@ def single_system(args, L, _native, ics, np, torch):
             "frac": round(achieved / PEAK_FP32_TFLOPS, 4),
             "traffic": traffic_from_profiles(workload),
             "kernel_ms": round(kernel_ms, 4),
-            "kernel": KERNEL_NAMES[plan.variant],
+            "kernel": "k_force_tile" if plan.variant == _native.LDS and plan.jslice == 0 else KERNEL_NAMES[plan.variant],
             "flops_per_launch": 20 * int(inter),
             "pair_evaluations_per_launch": pair_evaluations(plan, n),
         },

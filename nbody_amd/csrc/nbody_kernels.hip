@@ -938,8 +938,8 @@ hipError_t go_sym(const ForcePlan& plan, const SymParams& sp, int band_blocks, h
 // slots, so the fewer there are the more each slot's rounding counts. RMS error
 // on a uniform ball with blocks of 128 (N < 16384) or 256, with blocks of 512
 // unfolded, and folded: N = 13312 4.3e-8, 6.3e-8, 4.0e-8; 16384 5.5e-8, 6.3e-8,
-// 4.3e-8; 32767 4.5e-8, 4.9e-8, 3.8e-8. Folding takes 0 to 2 % of the time up to
-// there (42.4 and 42.5 us, 53.6 and 54.4, 178 and 178) and 1 to 2.5 % of N = 98304,
+// 4.4e-8; 32767 4.5e-8, 4.9e-8, 3.9e-8. Folding takes 0 to 2.5 % of the time up to
+// there (42.2 and 43.2 us, 53.0 and 53.5, 174 and 176) and 1 to 2.5 % of N = 98304,
 // where the error is below that of one wave per block pair without it.
 constexpr int kFoldMaxBlocks = 64;
 

@@ -219,8 +219,9 @@ enum : int { NO_PRIO = -1 };
 // pairs, 1.2 % of its rate): the running j-side sums then take 64 roundings
 // per tile instead of 512, which keeps every system of the 512-system
 // ensemble within 1e-5 of the FP64 sum on its evolved states (1.8e-5
-// without). The single-system kernel keeps one running sum: it holds the
-// bound on its configured state without the extra adds.
+// without). The single-system kernel sums a tile's reactions in parts up to 64
+// blocks (TileSums below, at a fraction of the cost) and keeps one running sum
+// past that: it holds the bound on its configured state without the extra adds.
 enum : int { REGS_FREE = 0, REGS_PINNED = 1, REGS_APART = 2 };
 template <int REGS, int BASE>
 __device__ __forceinline__ void sym_step8(float& xj, float& yj, float& zj, float& mj, float& rx, float& ry, float& rz,
@@ -773,8 +774,12 @@ __device__ __forceinline__ void sym_pair(const float4* __restrict__ pm, int n, f
     }
 }
 
-// Steps of a rotation after which a tile's running reactions are put away.
-constexpr int kFoldSteps = 8;
+// Steps of a rotation after which a tile's running reactions are put away: 8,
+// and 16 (0.5 % faster) from 32 blocks on where block pairs are several tasks,
+// with i sides of 64 roundings a wave. RMS error relative to the finer blocks':
+// with 8 0.80 to 0.99, with 16 at N = 16384 0.75 to 0.83, 32767 0.78 to
+// 0.89, but at N = 13312 0.97 to 1.07.
+__device__ __forceinline__ int fold_steps(int n, int split) { return split > 1 && n > 31 * 512 ? 16 : 8; }
 
 // A tile's reactions summed in parts: a running sum over some of the steps is
 // put away in LDS under the lane in which the body began (the rotation goes up
@@ -791,11 +796,11 @@ struct TileSums {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         rx = ry = rz = 0.f;
     }
-    // The end of every kFoldSteps steps, after `steps` of them.
-    __device__ __forceinline__ void fold(int steps, float& rx, float& ry, float& rz) const
+    // The end of a part, after `steps` steps of the tile.
+    __device__ __forceinline__ void fold(int steps, bool first, float& rx, float& ry, float& rz) const
     {
         const int began = (threadIdx.x - steps) & 63;
-        if (steps != kFoldSteps) add_to(began, rx, ry, rz);
+        if (!first) add_to(began, rx, ry, rz);
         set(began, rx, ry, rz);
     }
     __device__ __forceinline__ void add_to(int began, float& rx, float& ry, float& rz) const
@@ -866,11 +871,11 @@ constexpr int kDealWaves = 4;
 // half a turn on, and leaves the scaled reactions in r: half 0's in the lane
 // half a turn from the body's, half 1's in the body's own lane. With LEAD the
 // first half of the wave's steps runs one priority higher. With FOLD a tile's
-// reactions are summed in parts of kFoldSteps steps, 64 roundings each: one
+// reactions are summed in parts of `run` steps, 64 or 128 roundings each: one
 // running sum over a whole tile takes 512.
 template <bool NEWTON, bool EQ, int REGS, bool LEAD, bool FOLD>
 __device__ __forceinline__ void sym_deal_tiles(const float4* __restrict__ pm, int n, float eps2, int j0, int t0,
-                                               int t1, int step, int half, int halves, const Lanes<8>& me,
+                                               int t1, int step, int half, int halves, int run, const Lanes<8>& me,
                                                const float (&mi)[8], Lanes<8>& acc, float* jdst, size_t plane,
                                                float scale, float (&r)[3], const TileSums& sums)
 {
@@ -884,7 +889,8 @@ __device__ __forceinline__ void sym_deal_tiles(const float4* __restrict__ pm, in
         const float4 b = from < n - jbase ? pm[jbase + from] : make_float4(0.f, 0.f, 0.f, 0.f);
         float xj = b.x, yj = b.y, zj = b.z, mj = b.w;
         rx = ry = rz = 0.f;
-        const int steps = halves == 2 ? 32 : 64, run = FOLD ? kFoldSteps : steps;
+        const int steps = halves == 2 ? 32 : 64;
+        if constexpr (!FOLD) run = steps;
         int k = 0;
         if constexpr (LEAD) {
             const int early = t1 - t0 > 1 ? (tile + step < t1 ? 64 : 0) : steps / 2;
@@ -892,14 +898,14 @@ __device__ __forceinline__ void sym_deal_tiles(const float4* __restrict__ pm, in
                 for (int m = 0; m < run; ++m)
                     sym_step<8, NEWTON, EQ, REGS, 1>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
                 k += run;
-                if constexpr (FOLD) sums.fold(k, rx, ry, rz);
+                if constexpr (FOLD) sums.fold(k, k == run, rx, ry, rz);
             }
         }
         while (k < steps) {
             for (int m = 0; m < run; ++m)
                 sym_step<8, NEWTON, EQ, REGS>(xj, yj, zj, mj, rx, ry, rz, acc, me, mi, eps2);
             k += run;
-            if constexpr (FOLD) sums.fold(k, rx, ry, rz);
+            if constexpr (FOLD) sums.fold(k, k == run, rx, ry, rz);
         }
         if constexpr (FOLD) sums.add_to((lane - steps) & 63, rx, ry, rz);  // (to zero)
         rx *= scale;
@@ -1013,14 +1019,14 @@ __device__ __forceinline__ void sym_deal_task(const float4* __restrict__ pm, int
         if (eq) scale = m0;
         float* jdst = slots.j_side(P, Q, B);
         const size_t plane = slots.bplane;
-        const int out = t0 * 64;
+        const int out = t0 * 64, run = fold_steps(n, split);
         float r[3];
         if (eq)
-            sym_deal_tiles<NEWTON, true, EQ_REGS, LEAD, FOLD>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi, acc,
-                                                        jdst, plane, m0, r, sums);
+            sym_deal_tiles<NEWTON, true, EQ_REGS, LEAD, FOLD>(pm, n, eps2, Q * B, t0, t1, W, half, halves, run, me, mi,
+                                                              acc, jdst, plane, m0, r, sums);
         else
-            sym_deal_tiles<NEWTON, false, GEN_REGS, LEAD, FOLD>(pm, n, eps2, Q * B, t0, t1, W, half, halves, me, mi,
-                                                          acc, jdst, plane, 1.0f, r, sums);
+            sym_deal_tiles<NEWTON, false, GEN_REGS, LEAD, FOLD>(pm, n, eps2, Q * B, t0, t1, W, half, halves, run, me,
+                                                                mi, acc, jdst, plane, 1.0f, r, sums);
         if (halves == 2) {
             // the first half's reactions are half a turn from home; the second wave adds both in order
             if (half == 0) {
