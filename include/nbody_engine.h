@@ -41,7 +41,8 @@ nbody_hip_system *nbody_hip_system_create(const float *posMass, const float *vel
 int nbody_hip_system_run(nbody_hip_system *s, int steps, int use_graph, float *ms);
 /* Copies the current state (and the last force) to the host; NULL skips one. */
 int nbody_hip_system_read(const nbody_hip_system *s, float *posMass, float *velInvMass, float *force);
-/* The plan in use. */
+/* The plan in use, described as by nbody_hip_plan (i_per_lane and jslice are 0
+ * for the one-launch plan of small systems). */
 int nbody_hip_system_plan(const nbody_hip_system *s, nbody_hip_options *plan);
 void nbody_hip_system_destroy(nbody_hip_system *s);
 
@@ -51,7 +52,8 @@ typedef struct nbody_hip_ensemble nbody_hip_ensemble;
 
 enum {
     NBODY_HIP_BATCHED_GRAPH = 0, /* per step, for each of two groups of systems on its own stream: one
-                                    persistent force launch + one slot-sum-and-integrate launch; from a graph */
+                                    persistent force launch + one slot-sum-and-integrate launch; 16 steps at a
+                                    time from a graph, the steps past the last whole 16 without */
     NBODY_HIP_BATCHED = 1,       /* the same launches per step, without a graph */
     NBODY_HIP_PER_SYSTEM = 2     /* every system on its own: its best single-system plan, one after another */
 };
@@ -59,10 +61,10 @@ enum {
 /* count systems of N[s] bodies, stored back to back in posMass/velInvMass
  * (system s starts at body sum_{r<s} N[r]); softeningSquared[s] per system;
  * dt and damping shared. The batched modes evaluate a system of N <= 2^18
- * bodies pairwise-symmetrically in blocks of 512, each pair once (block
- * pairs exactly as nbody_hip_force's symmetric plan with 8 bodies per lane
- * and blocks of 512; each diagonal block as one task, where that plan sums
- * it one-sidedly, so the two agree to rounding), keeping 12 * ceil(N/512)^2 * 512 bytes of
+ * bodies pairwise-symmetrically in blocks of 512, each pair once (as
+ * nbody_hip_force's symmetric plan with 8 bodies per lane and blocks of 512,
+ * with one task per block pair and the reactions summed per step, so the two
+ * agree to rounding), keeping 12 * ceil(N/512)^2 * 512 bytes of
  * block partials in HBM; a larger one one-sidedly with compensated sums
  * (12 N bytes of partials). */
 nbody_hip_ensemble *nbody_hip_ensemble_create(size_t count, const size_t *N, const float *posMass,

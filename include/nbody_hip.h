@@ -47,7 +47,8 @@ enum {
     NBODY_HIP_DPP = 2,       /* j tile passed around the wave64 by DPP (src/nbody_GPU_Shuffle.cu:44-107) */
     NBODY_HIP_SGPR = 3,      /* scalar-memory broadcast (src/nbody_GPU_AOS_const.cu:45-121) */
     NBODY_HIP_SYMMETRIC = 4, /* each pair once, no global atomics (src/nbody_GPU_AOS_tiled.cu:44-220) */
-    NBODY_HIP_AUTO = -1      /* the autotuned plan, else SYMMETRIC for whole systems of N > 10240, else LDS */
+    NBODY_HIP_AUTO = -1      /* the autotuned plan, else SYMMETRIC for whole systems of N > 10240 (of N >= 1024
+                                with compensated, newton, slot_bytes or a shape given), else LDS */
 };
 
 /* Options of the general entry; zero / -1 fields mean "choose".

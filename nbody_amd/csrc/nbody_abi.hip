@@ -136,9 +136,10 @@ void lds_shape(size_t N, size_t n, int cus, bool newton_plain, int* ipl, int* js
     if (newton_plain) *ipl = 1;
 }
 
-// Default decomposition: enough blocks for ~48 waves per SIMD (the dispatcher
-// balances them across the 256 CUs), j slices of at least 1024 bodies in
-// multiples of 256.
+// Default decomposition. Scalar loads and DPP: enough blocks for ~48 waves per
+// SIMD (the dispatcher balances them across the CUs), j slices of at least 1024
+// bodies in multiples of 256; the LDS variant as lds_shape has it, or in one
+// launch; the symmetric plans' blocks below.
 ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip_options* opt, int shares)
 {
     ForcePlan p;
@@ -150,7 +151,7 @@ ForcePlan default_plan(int variant, size_t N, size_t n, int cus, const nbody_hip
     p.acc64 = comp_opt == 2;
     const double chips = std::max(cus, 1) / 256.0;  // of the chip that the times below were measured on
     if (variant == VAR_SYMMETRIC && p.acc64) {
-        // one wave per block pair, 4 (or 8) bodies per lane, blocks of 64 per lane
+        // four waves per block pair, 4 (or 8) bodies per lane, blocks of 64 per body of a lane
         p.ipl = (opt && opt->i_per_lane > 0) ? opt->i_per_lane : 4;
         p.jslice = (opt && opt->jslice > 0) ? opt->jslice : 64 * p.ipl;
         p.nslices = (int)((N + p.jslice - 1) / p.jslice);

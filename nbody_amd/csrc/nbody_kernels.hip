@@ -9,7 +9,7 @@
 //     wave-uniform body at a time (scalar loads into SGPRs, an LDS
 //     broadcast), or a 64-body tile that DPP moves one lane per step;
 //   * slice partials (float4, plus a float4 of TwoSum residues when
-//     compensated) are summed by k_reduce in slice order, so a result depends
+//     compensated) are summed by k_reduce in a fixed order, so a result depends
 //     on the plan only, never on scheduling.
 // With one slice the kernel writes force directly. Force records are written
 // x, y, z only; w is left alone (the contract of src/nbody.cu:351-371).
@@ -423,7 +423,7 @@ __global__ __launch_bounds__(64 * W) void k_force_sym(SymParams p)
 // in one-sided pieces at the end, with this split, and with the pair chain's
 // wave priorities too: N = 98304 1619, 1560 and 1358 us (0.905 of the FP32
 // peak), 49999 479, 429 and 379, 32768 212 and 188, 24576 141 and 115, 16384
-// 71.7, 62.2 and 54.7, 12000 53 and 43; unequal masses at 98304 1815, 1770
+// 71.7, 62.2 and 53.5, 12000 53 and 43; unequal masses at 98304 1815, 1770
 // and 1541. FOLD: kFoldMaxBlocks below. LEAD (go_sym_deal) runs at most 4
 // workgroups to a CU and holds more registers.
 template <bool NEWTON, bool FOLD, bool LEAD>
@@ -633,7 +633,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce64(const double* __restrict__ 
     f[2] = (float)z;
 }
 
-// Slice partials summed in slice order; compensated plans merge the TwoSum
+// Slice partials summed in a fixed order; compensated plans merge the TwoSum
 // residues and round once at the end. A workgroup takes 64 bodies, each of its
 // waves a quarter of the slices (four in flight), and wave 0 then adds the
 // quarters in order: one lane per body over all slices was bound by its chain
@@ -1081,9 +1081,9 @@ double tile_shape(size_t n, size_t ni, bool acc64, int cu_count, int* li, int* i
 
 // With at most 4 tasks to a CU (fewer if the plan caps its waves) every task
 // starts at once, and the waves of a SIMD had better end together: those in the
-// first half of their steps go first. N = 16384 54.5 and 52.6 us, unequal masses
-// 60.1 and 57.2, 10241 35.1 and 33.8. With more tasks it keeps the next ones
-// waiting (20480 83.7 and 90.2, 32768 172 and 181).
+// first half of their steps go first. Before the folds N = 16384 54.5 and 52.6 us,
+// unequal masses 60.1 and 57.2, 10241 35.1 and 33.8. With more tasks it keeps the
+// next ones waiting (20480 83.7 and 90.2, 32768 172 and 181).
 bool deal_leads(const ForcePlan& plan, int tasks)
 {
     const int per_cu = plan.occ > 0 ? std::min(4, plan.occ) : 4;

@@ -30,8 +30,8 @@ class System:
             raise _native.NativeError(_native.last_error())
 
     def run(self, steps, graph=True):
-        """Runs `steps` steps (graph: one captured graph replay per step) and
-        returns their milliseconds."""
+        """Runs `steps` steps (graph: 16 at a time from a captured graph, the
+        rest launched directly) and returns their milliseconds."""
         ms = ctypes.c_float()
         _native.check(_native.lib().nbody_hip_system_run(self.h, steps, 1 if graph else 0, ctypes.byref(ms)), "run")
         return ms.value
@@ -46,6 +46,8 @@ class System:
         return pm, vm, f
 
     def plan(self):
+        """The plan in use (i_per_lane and jslice 0: the one-launch plan of
+        small systems, which has neither)."""
         out = _native.Options()
         _native.check(_native.lib().nbody_hip_system_plan(self.h, ctypes.byref(out)), "plan")
         return out
